@@ -23,12 +23,24 @@
 //  - per z the lane does one FMA for vIndex, v_cvt_flr/v_fract, one address op, the LDS
 //    read and 4 FMAs, with the reads software-pipelined in small groups; the
 //    per-column geometry (one reciprocal) is amortised over the run;
+//  - a step runs in one of three forms: unmasked where the tile's run lies inside the
+//    detector window (8 VALU instructions per update and 22 per column), masked by groups
+//    of four slices where part of it does not, and voxel by voxel from global memory where
+//    the box does not fit the LDS;
 //  - boxes are computed by wave 0 for 64 projections at a time (one lane per projection);
 //    a projection whose box exceeds the tile capacity reads entries from global memory
 //    instead, so any geometry stays correct;
 //  - workgroups are numbered so that each XCD (dispatch is round-robin over 8 XCDs)
 //    receives a contiguous range of tiles, in 4x4 blocks of tiles, and shares detector
 //    footprints in its own L2.
+//
+// What bounds it (1024^3 x 720 x 1024^2, MI355X): with FP32 entries the traffic of boxes that
+// miss L2 (747 GB per launch, 4.6 TB/s; 137 ms instead of 162 when every staged line hits),
+// then the LDS (a ds_read_b128 takes 4.8 cycles per wave and CU, a staging DMA instruction
+// 17 whatever its lane mask); with 8-byte entries VALU issue (116 of 133 ms remain without
+// any staging).  Accumulators updated in place, three forms per step and tests left out where
+// a box lies inside the window took FP32 from 177 to 163 ms, FP16 from 147 to 133 ms, and a
+// 256^3 x 360 scan from 2.67 to 2.2 ms.
 #include "ctg_internal.h"
 
 #include <hip/hip_fp16.h>
@@ -63,7 +75,7 @@ struct BpArgs {
 struct EF32 {
     using T = float4;
     static constexpr int kBytes = 16;
-    static constexpr int kMinWaves = 1;  // LDS limits FP32 tiles to 3 workgroups per CU anyway
+    static constexpr int kMinWaves = 4;  // 127 VGPRs; the LDS may allow only 3
     static constexpr int kGrp = 4;       // LDS reads per software-pipeline group
     __device__ static float eval(const T& e, float fu, float fv) {
         return fmaf(fv, fmaf(fu, e.w, e.z), fmaf(fu, e.y, e.x));
@@ -72,8 +84,8 @@ struct EF32 {
 struct EF16 {
     using T = uint2;
     static constexpr int kBytes = 8;
-    static constexpr int kMinWaves = 4;  // VALU-bound: keep 4 waves per SIMD (at most 128 VGPRs)
-    static constexpr int kGrp = 2;       // (groups of 4 need spills at 128 VGPRs: measured slower)
+    static constexpr int kMinWaves = 5;  // VALU-bound: 5 waves per SIMD (at most 96 VGPRs)
+    static constexpr int kGrp = 2;       // (groups of 4 need more registers: measured slower)
     __device__ static float lo(uint32_t e) { return __half2float(__ushort_as_half((unsigned short)(e & 0xffffu))); }
     __device__ static float hi(uint32_t e) { return __half2float(__ushort_as_half((unsigned short)(e >> 16))); }
     __device__ static float eval(const T& e, float fu, float fv) {
@@ -83,7 +95,7 @@ struct EF16 {
 struct EBF16 {
     using T = uint2;
     static constexpr int kBytes = 8;
-    static constexpr int kMinWaves = 4;
+    static constexpr int kMinWaves = 5;
     static constexpr int kGrp = 2;
     __device__ static float lo(uint32_t e) { return __uint_as_float(e << 16); }
     __device__ static float hi(uint32_t e) { return __uint_as_float(e & 0xffff0000u); }
@@ -117,6 +129,28 @@ template <int B>
 __device__ inline void lds_dma(dma_rsrc, unsigned, int, void*) {}
 #endif
 
+// acc += w * q, in place.  Written as the two-address instruction because the accumulators
+// meet again after paths that differ per step: with fmaf() the compiler gives the fast
+// path's sums registers of their own and copies all ZPL of them back on every step (one
+// more VALU instruction per update, and 162 VGPRs instead of 127 for FP32 entries, 128
+// instead of 95 for 8-byte entries).
+__device__ inline void fmac(float& acc, float w, float q) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_fmac_f32 %0, %1, %2" : "+v"(acc) : "v"(w), "v"(q));
+#else
+    acc = fmaf(w, q, acc);
+#endif
+}
+
+// A wave-uniform value that the optimiser knows nothing about.
+__device__ inline int opaque_uniform(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    v = __builtin_amdgcn_readfirstlane(v);
+    asm volatile("" : "+s"(v));
+#endif
+    return v;
+}
+
 __device__ inline int cvt_flr(float x) {
     int r;
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
@@ -125,10 +159,12 @@ __device__ inline int cvt_flr(float x) {
 
 // box: x = first entry column, y = first row, w = rows, z = ncols | flags.
 // bits 28-29: 0 the block cannot hit the detector, 1 staged in LDS, 2 global reads;
-// bit 27: the fast (unmasked) path may be used.
+// bit 27: the unmasked path may be used; bit 26: it may be used without any test, because
+// the whole tile and run lie inside the detector window.
 __device__ inline int box_kind(int4 b) { return ((unsigned)b.z >> 28) & 3; }
 __device__ inline bool box_fast(int4 b) { return (b.z >> 27) & 1; }
-__device__ inline int box_nc(int4 b) { return b.z & 0x07ffffff; }
+__device__ inline bool box_inside(int4 b) { return (b.z >> 26) & 1; }
+__device__ inline int box_nc(int4 b) { return b.z & 0x03ffffff; }
 __device__ inline int box_nr(int4 b) { return b.w & 0xffff; }
 __device__ inline int box_pitch(int4 b) { return (unsigned)b.w >> 16; }
 
@@ -181,7 +217,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     const int zfirst = a.zshift - zb;
     const int zlast = a.nzs + a.zshift - zb;
     const bool colvol = xi < a.nx && yi < a.ny;
-    const float x = (float)xi - a.xpre, y = (float)yi - a.ypre;
+    // lanes past the grid take its last column, so that every lane's ray stays inside the
+    // tile's footprint; what they and lanes outside the cylinder add up is dropped at the end
+    const float x = (float)min(xi, a.nx - 1) - a.xpre, y = (float)min(yi, a.ny - 1) - a.ypre;
     const bool incyl = colvol && (x * x + y * y < a.r2);
 
     const float cxa = (float)(tx * kTX) - a.xpre;
@@ -267,7 +305,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             b.x = us; b.y = vs; b.w = nr | (pitch << 16);
             // the fused vIndex of the fast path may round a hair below 0 at the top edge
             const int fast = vs0 >= 0 ? 1 : 0;
-            b.z = nc | (fast << 27) | ((nc * pitch <= a.cap ? 1 : 2) << 28);
+            // no voxel of the tile and run can fail a window test (by more than either
+            // expression's rounding), and no entry is clipped away
+            const bool in = fast && us0 >= 0 && umin - kBoxMargin >= a.ulo + a.upre &&
+                            umax + kBoxMargin <= fminf(a.uhi + a.upre, (float)(a.W - 1)) &&
+                            vmin - kBoxMargin >= a.vpre - a.vhi &&
+                            vmax + kBoxMargin <= fminf(a.vpre - a.vlo, (float)(a.H - 1));
+            b.z = nc | ((in ? 1 : 0) << 26) | (fast << 27) | ((nc * pitch <= a.cap ? 1 : 2) << 28);
             return b;
         };
 
@@ -312,66 +356,126 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             const float s = x * g.y + y * g.x;
             const float U = cone_magnification(a.fcd, s);
             const float u = t * U;
-            const bool cv = incyl && u >= a.ulo && u <= a.uhi;
             const float uIdx = u + a.upre;
             const int u0 = (int)uIdx;
             const float fu = uIdx - (float)u0;
             const float w = U * U * sc;
-            if (kind == 1) {
-                const int us = bx.x, vs = bx.y, nr = box_pitch(bx);
+            const float vA = det_row_anchor(zwa, g.z, U, a.vpre);
+            const int us = bx.x, vs = bx.y, pitch = box_pitch(bx);
+            const bool cv = incyl && u >= a.ulo && u <= a.uhi;
+            float Ue = U, we = w, fue = fu, vAe = vA;
+            const char* tile_b = reinterpret_cast<const char*>(tile) - (us * pitch + vs) * E::kBytes;
+            const char* col = tile_b + __mul24(u0, pitch * E::kBytes);
+            // a column that adds nothing reads the box's first entry with zero weight
+            auto idle = [&]() {
+                Ue = we = fue = 0.0f;
+                vAe = (float)vs;
+                col = reinterpret_cast<const char*>(tile) - vs * E::kBytes;
+            };
+            // how the step runs: 1 unmasked from LDS, 2 masked by groups of slices from LDS,
+            // 3 voxel by voxel from global memory
+            int mode = kind == 1 ? 1 : 3;
+            if (kind == 1 && !box_inside(bx)) {
                 const bool lane_full = !cv || ((zw0 + g.z) * U >= a.vlo && (zw1 + g.z) * U <= a.vhi);
-                if (box_fast(bx) && __all(lane_full)) {
-                    // every active column keeps all ZPL voxels inside the detector window;
-                    // inactive columns read entry 0 with zero weight
-                    const float Ue = cv ? U : 0.0f;
-                    const float we = cv ? w : 0.0f;
-                    const float fue = cv ? fu : 0.0f;
-                    const int base = cv ? (u0 - us) * nr - vs : -(int)floorf(a.vpre);
-                    const T* tb = tile + base;
-                    const float vA = det_row_anchor(zwa, g.z, Ue, a.vpre);
-                    // software pipeline in groups of kGrp: the LDS reads of group g+1 are
-                    // issued before the arithmetic of group g, and scheduling barriers
-                    // keep the compiler from trading those in-flight reads for hoisted
-                    // row-index arithmetic
-                    constexpr int kGrp = E::kGrp;
-                    T e[2][kGrp];
-                    float fv[2][kGrp];
-                    auto fetch = [&](int g0, int slot) {
+                if (!(box_fast(bx) && __all(lane_full))) mode = 2;
+                else if (!cv) idle();
+            }
+            // The three forms follow one another, each under its own opaque condition: as
+            // alternatives of one branch the compiler keeps the accumulators of each in
+            // registers of its own and copies them together on every step.
+            if (opaque_uniform(mode) == 1) {
+                const T* tb = reinterpret_cast<const T*>(col);
+                // software pipeline in groups of kGrp: the LDS reads of group g+1 are
+                // issued before the arithmetic of group g, and scheduling barriers
+                // keep the compiler from trading those in-flight reads for hoisted
+                // row-index arithmetic
+                constexpr int kGrp = E::kGrp;
+                T e[2][kGrp];
+                float fv[2][kGrp];
+                auto fetch = [&](int g0, int slot) {
 #pragma unroll
-                        for (int j = 0; j < kGrp; ++j) {
-                            const float vI = det_row_index((float)(g0 + j + koff), Ue, vA);
-                            e[slot][j] = tb[cvt_flr(vI)];
-                            fv[slot][j] = __builtin_amdgcn_fractf(vI);
-                        }
-                    };
-                    fetch(0, 0);
-#pragma unroll
-                    for (int g0 = 0; g0 < ZPL; g0 += kGrp) {
-                        const int slot = (g0 / kGrp) & 1;
-                        if (g0 + kGrp < ZPL) fetch(g0 + kGrp, slot ^ 1);
-#pragma unroll
-                        for (int j = 0; j < kGrp; ++j)
-                            acc[g0 + j] = fmaf(we, E::eval(e[slot][j], fue, fv[slot][j]), acc[g0 + j]);
-                        __builtin_amdgcn_sched_barrier(0);
+                    for (int j = 0; j < kGrp; ++j) {
+                        const float vI = det_row_index((float)(g0 + j + koff), Ue, vAe);
+                        e[slot][j] = tb[cvt_flr(vI)];
+                        fv[slot][j] = __builtin_amdgcn_fractf(vI);
                     }
-                } else {
-                    const T* tb = tile + ((u0 - us) * nr - vs);
-                    const float vA = det_row_anchor(zwa, g.z, U, a.vpre);
+                };
+                fetch(0, 0);
 #pragma unroll
-                    for (int k = 0; k < ZPL; ++k) {
-                        const float zk = zw0 + (float)k;
-                        const float v = (zk + g.z) * U;
-                        if (cv && v >= a.vlo && v <= a.vhi) {
-                            const float vI = det_row_index((float)(k + koff), U, vA);
+                for (int g0 = 0; g0 < ZPL; g0 += kGrp) {
+                    const int slot = (g0 / kGrp) & 1;
+                    if (g0 + kGrp < ZPL) fetch(g0 + kGrp, slot ^ 1);
+#pragma unroll
+                    for (int j = 0; j < kGrp; ++j)
+                        fmac(acc[g0 + j], we, E::eval(e[slot][j], fue, fv[slot][j]));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (opaque_uniform(mode) == 2) {
+                // Some column leaves the window within the run.  v = (z + h) U is
+                // non-decreasing in z (U > 0, monotone rounding), so the slices that pass the
+                // window test form an interval [lo, hi]: estimated by division, then settled
+                // with the test's own expression.
+                auto v_of = [&](int k) { return ((zw0 + (float)k) + g.z) * U; };
+                const float iU = __builtin_amdgcn_rcpf(U), zo = zw0 + g.z;
+                int lo = (int)ceilf(fminf(fmaxf(a.vlo * iU - zo, -4.0f), (float)(ZPL + 4)));
+                int hi = (int)floorf(fminf(fmaxf(a.vhi * iU - zo, -4.0f), (float)(ZPL + 4)));
+#pragma unroll
+                for (int it = 0; it < 2; ++it) {
+                    if (v_of(lo - 1) >= a.vlo) --lo;
+                    if (v_of(hi + 1) <= a.vhi) ++hi;
+                }
+#pragma unroll
+                for (int it = 0; it < 2; ++it) {
+                    if (!(v_of(lo) >= a.vlo)) ++lo;
+                    if (!(v_of(hi) <= a.vhi)) --hi;
+                }
+                lo = max(lo, 0);
+                hi = min(hi, ZPL - 1);
+                const bool act = cv && lo <= hi && v_of(lo) >= a.vlo && v_of(hi) <= a.vhi;
+                if (!act) idle();
+                const T* tb = reinterpret_cast<const T*>(col);
+                const int ve = vs + box_nr(bx) - 1;
+                // groups of four slices: skipped where no column is in the window, unmasked
+                // where every column is (by one slice at the upper end, where the fused row
+                // index may round a hair below row 0), else each voxel masked and its row
+                // clamped into the box
+#pragma unroll
+                for (int g0 = 0; g0 < ZPL; g0 += 4) {
+                    int form = 0;
+                    if (__any(act && lo <= g0 + 3 && hi >= g0)) form = __all(!act || (lo <= g0 && hi > g0 + 3)) ? 1 : 2;
+                    if (opaque_uniform(form) == 1) {
+                        T e[4];
+                        float fv[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float vI = det_row_index((float)(g0 + j + koff), Ue, vAe);
+                            e[j] = tb[cvt_flr(vI)];
+                            fv[j] = __builtin_amdgcn_fractf(vI);
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) fmac(acc[g0 + j], we, E::eval(e[j], fue, fv[j]));
+                    }
+                    if (opaque_uniform(form) == 2) {
+                        T e[4];
+                        float fv[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float vI = det_row_index((float)(g0 + j + koff), Ue, vAe);
                             const int v0 = (int)vI;
-                            const T e = tb[v0];
-                            acc[k] = fmaf(w, E::eval(e, fu, vI - (float)v0), acc[k]);
+                            e[j] = tb[min(max(v0, vs), ve)];
+                            fv[j] = vI - (float)v0;
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float q = E::eval(e[j], fue, fv[j]);
+                            fmac(acc[g0 + j], we, lo <= g0 + j && hi >= g0 + j ? q : 0.0f);
                         }
                     }
                 }
-            } else {
+            }
+            if (opaque_uniform(mode) == 3) {
                 const T* src = proj + ((size_t)p * a.W + u0) * a.H;
-                const float vA = det_row_anchor(zwa, g.z, U, a.vpre);
 #pragma unroll
                 for (int k = 0; k < ZPL; ++k) {
                     const float zk = zw0 + (float)k;
@@ -380,7 +484,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
                         const float vI = det_row_index((float)(k + koff), U, vA);
                         const int v0 = (int)vI;
                         const T e = src[v0];
-                        acc[k] = fmaf(w, E::eval(e, fu, vI - (float)v0), acc[k]);
+                        fmac(acc[k], w, E::eval(e, fu, vI - (float)v0));
                     }
                 }
             }
@@ -436,14 +540,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             __syncthreads();
             if ((p & 63) == 0 && tid < 64) fill_batch(((p >> 6) + 1) & 1, p + 64 + tid);
             const int q = p + 1;
-            const int4 bn = q < a.nproj ? uniform_box(boxes[(q >> 6) & 1][q & 63]) : make_int4(0, 0, 0, 0);
-            const float4 gn = q < a.nproj ? uniform_f4(params[(q >> 6) & 1][q & 63]) : g;
+            // (past the last projection the batch holds empty boxes)
+            const int4 bl = boxes[(q >> 6) & 1][q & 63];
+            const float4 gl = params[(q >> 6) & 1][q & 63];
+            const int4 bn = uniform_box(bl);
+            const float4 gn = uniform_f4(gl);
             step(reinterpret_cast<const T*>(buffer(p)), buffer(p + 1), p, bx, bn, g, g.w);
             bx = bn;
             g = gn;
         }
     }
 
+    if (!incyl) {
+#pragma unroll
+        for (int k = 0; k < ZPL; ++k) acc[k] = 0.0f;
+    }
     if (colvol) {
         float* col = vol + ((size_t)xi * a.ny + yi) * a.nzs;
         if (a.vec4 && zfirst <= 0 && zlast >= ZPL) {

@@ -854,3 +854,47 @@ def test_reconstruct_memory_plans_slabs_and_recomputation(gpu):
     assert calls == [0.5]
     ctx.reset_cancel()
     assert np.array_equal(recon(), ref)
+
+
+@pytest.mark.parametrize("store", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("nz,z0", [(1, 0), (31, 0), (33, 0), (100, 0), (100, 17)])
+def test_lds_forms_match_the_global_form(gpu, monkeypatch, store, nz, z0):
+    """The unmasked and the masked LDS forms of a backprojection step against the form that
+    tests voxel by voxel and reads global memory: the same expressions in the same order, so
+    the volumes agree bit for bit.  Height offsets of up to most of the detector, an axis
+    offset and a grid wider than the detector make runs leave the window at either end, in
+    the middle of a group of slices, and for some columns only.  Non-finite entries stay out
+    of the voxels outside the cylinder."""
+    import torch
+    import ct_amd
+    W, H, P = 70, 50, 11
+    g = ct_amd.geometry_grid(W, H, 1.3 * W, 5.0, 85, 83, nz)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    ctx.set_projections(np.linspace(0.0, 350.0, P), np.linspace(-40.0, 40.0, P))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    img = torch.randn((P, H, W), generator=gen, device="cuda")
+    entries = torch.empty(ctx.filtered_bytes(store, P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, dtype=torch.float32, device="cuda")
+    n = nz - z0
+
+    def volume():
+        v = torch.full((g.nx, g.ny, n), 0.5, dtype=torch.float32, device="cuda")
+        ctx.backproject(entries, store, scales, 0, P, v, z0, n, True)
+        torch.cuda.synchronize()
+        return v.cpu().numpy()
+
+    ctx.layout_projections(img, P, store, entries, scales)
+    got = volume()
+    # columns rounded up to 65536 rows fit no LDS buffer: every projection reads global memory
+    monkeypatch.setenv("CTG_BP_PITCH", "65536,0")
+    ref = volume()
+    assert np.isfinite(ref).all() and np.any(ref != 0.5)
+    np.testing.assert_array_equal(got, ref)
+    monkeypatch.delenv("CTG_BP_PITCH")
+    if store == "f32":
+        img.fill_(float("nan"))
+        ctx.layout_projections(img, P, store, entries, scales)
+        x = np.arange(g.nx)[:, None] - g.x_pre
+        y = np.arange(g.ny)[None, :] - g.y_pre
+        assert np.all(volume()[x * x + y * y >= g.radius ** 2] == 0.5)
