@@ -30,7 +30,7 @@ __global__ void maxabs_kernel(const float* __restrict__ img, size_t per_image, u
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < per_image; i += (size_t)gridDim.x * blockDim.x)
         m = fmaxf(m, fabsf(src[i]));
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(&out[p], __float_as_uint(m));
+    if ((threadIdx.x & 63) == 0) raise_max(&out[p], m);
 }
 }  // namespace
 
@@ -185,16 +185,20 @@ ctg_status preprocess_batched(ctg_context* ctx, const void* d_raw, ctg_pixel_typ
     const size_t budget = (size_t)1 << 30;  // 1 GiB of FP32 work images per batch
     int batch = (int)std::max<size_t>(1, std::min<size_t>((size_t)nproj, budget / (img * 4)));
     CTG_TRY(ctx->rows_f32.reserve(img * 4 * batch));
-    CTG_TRY(ctx->maxabs.reserve(sizeof(unsigned) * std::max(nproj, 1)));
-    CTG_TRY(fill_u32(ctx->maxabs.ptr, 0u, (size_t)nproj, st));
+    // only the 8-byte entries are scaled by their image's max |value|
+    const bool scaled = store != CTG_STORE_F32;
+    if (scaled) {
+        CTG_TRY(ctx->maxabs.reserve(sizeof(unsigned) * std::max(nproj, 1)));
+        CTG_TRY(fill_u32(ctx->maxabs.ptr, 0u, (size_t)nproj, st));
+    }
     for (int b0 = 0; b0 < nproj; b0 += batch) {
         if (ctx->cancel.load()) return fail(CTG_ERROR_INTERRUPTED, "interrupted");
         const int nb = std::min(batch, nproj - b0);
         const char* raw = (const char*)d_raw + (size_t)b0 * img * pixel_bytes(pixel);
-        CTG_TRY(launch_preprocess_rows(ctx, raw, pixel, nb, base, form, filter, ctx->rows_f32.as<float>(),
-                                       ctx->maxabs.as<unsigned>() + b0, true, true, true, st));
+        unsigned* mx = scaled ? ctx->maxabs.as<unsigned>() + b0 : nullptr;
+        CTG_TRY(launch_preprocess_rows(ctx, raw, pixel, nb, base, form, filter, ctx->rows_f32.as<float>(), mx, st));
         char* out = (char*)d_filtered + (size_t)b0 * img * store_bytes(store);
-        CTG_TRY(launch_layout(g, ctx->rows_f32.as<float>(), nb, store, ctx->maxabs.as<unsigned>() + b0, out,
+        CTG_TRY(launch_layout(g, ctx->rows_f32.as<float>(), nb, store, mx, out,
                               d_scales ? d_scales + b0 : nullptr, st));
     }
     return CTG_OK;
@@ -496,8 +500,7 @@ ctg_status ctg_feldkamp_weight(ctg_context* ctx, float* d_images, int32_t nproj,
     CTG_TRY(check_ctx(ctx));
     if (nproj < 0 || (nproj > 0 && !d_images)) return fail(CTG_ERROR_INVALID_ARGUMENT, "bad buffers");
     if (nproj == 0) return CTG_OK;
-    return launch_preprocess_rows(ctx, d_images, CTG_PIXEL_F32, nproj, 1.0f, CTG_LOG_CPU_FORM, CTG_FILTER_RAMLAK,
-                                  d_images, nullptr, false, true, false, (hipStream_t)stream);
+    return launch_feldkamp_weight(ctx->geom, d_images, nproj, (hipStream_t)stream);
 }
 
 ctg_status ctg_filter_rows(ctg_context* ctx, const float* d_in, float* d_out, int64_t rows, ctg_filter filter,
@@ -520,10 +523,14 @@ ctg_status ctg_layout_projections(ctg_context* ctx, const float* d_images, int32
     if (nproj == 0) return CTG_OK;
     hipStream_t st = (hipStream_t)stream;
     const size_t img = (size_t)ctx->geom.det_width * ctx->geom.det_height;
-    CTG_TRY(ctx->maxabs.reserve(sizeof(unsigned) * nproj));
-    CTG_TRY(fill_u32(ctx->maxabs.ptr, 0u, (size_t)nproj, st));
-    if (store != CTG_STORE_F32) CTG_TRY(launch_maxabs(d_images, img, nproj, ctx->maxabs.as<unsigned>(), st));
-    return launch_layout(ctx->geom, d_images, nproj, store, ctx->maxabs.as<unsigned>(), d_filtered, d_scales, st);
+    unsigned* mx = nullptr;
+    if (store != CTG_STORE_F32) {
+        CTG_TRY(ctx->maxabs.reserve(sizeof(unsigned) * nproj));
+        mx = ctx->maxabs.as<unsigned>();
+        CTG_TRY(fill_u32(mx, 0u, (size_t)nproj, st));
+        CTG_TRY(launch_maxabs(d_images, img, nproj, mx, st));
+    }
+    return launch_layout(ctx->geom, d_images, nproj, store, mx, d_filtered, d_scales, st);
 }
 
 ctg_status ctg_layout_projections_noalloc(ctg_context* ctx, const float* d_images, int32_t nproj, ctg_store store,
@@ -541,8 +548,10 @@ ctg_status ctg_layout_projections_noalloc(ctg_context* ctx, const float* d_image
     hipStream_t st = (hipStream_t)stream;
     const size_t img = (size_t)ctx->geom.det_width * ctx->geom.det_height;
     unsigned* mx = ctx->noalloc_scratch;  // the device address of `scratch`, never the host stand-in
-    CTG_TRY(fill_u32(mx, 0u, (size_t)nproj, st));
-    if (store != CTG_STORE_F32) CTG_TRY(launch_maxabs(d_images, img, nproj, mx, st));
+    if (store != CTG_STORE_F32) {
+        CTG_TRY(fill_u32(mx, 0u, (size_t)nproj, st));
+        CTG_TRY(launch_maxabs(d_images, img, nproj, mx, st));
+    }
     return launch_layout(ctx->geom, d_images, nproj, store, mx, d_filtered, d_scales, st);
 }
 
@@ -607,8 +616,7 @@ ctg_status ctg_fdk_backward(ctg_context* ctx, const float* d_grad_volume, int32_
     CTG_TRY(launch_forward_project(g, ctx->proj_dev.as<float4>() + p0, ctx->proj_host.data() + p0, d_grad_volume, z0,
                                    nz, nproj, d_grad_lineint, ctx->fp_work, st));
     CTG_TRY(launch_filter_rows_only(ctx, d_grad_lineint, d_grad_lineint, (int64_t)nproj * g.det_height, filter, st));
-    return launch_preprocess_rows(ctx, d_grad_lineint, CTG_PIXEL_F32, nproj, 1.0f, CTG_LOG_CPU_FORM, filter,
-                                  d_grad_lineint, nullptr, false, true, false, st);
+    return launch_feldkamp_weight(g, d_grad_lineint, nproj, st);
 }
 
 ctg_status ctg_fdk_f64(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel, int32_t nproj, float base_intensity,

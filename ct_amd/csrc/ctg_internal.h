@@ -54,6 +54,15 @@ constexpr int kRowAnchor = 32;
 __device__ inline float det_row_anchor(float zwa, float h, float U, float vpre) { return fmaf(-(zwa + h), U, vpre); }
 __device__ inline float det_row_index(float k, float U, float anchor) { return fmaf(-k, U, anchor); }
 
+// Raises the running maximum *m (bits of a non-negative float, which order like unsigned
+// integers) to v.  Atomics to one address run one after another (about 10 ns each here: the
+// one per wave of every row of an image took longer than the row's filter), so a value
+// that is already covered only reads: what it reads may be old, but then only lower.
+__device__ inline void raise_max(unsigned* m, float v) {
+    const unsigned b = __float_as_uint(v);
+    if (__hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < b) atomicMax(m, b);
+}
+
 // Grow-only device buffer owned by a context.
 struct DevBuf {
     void* ptr = nullptr;
@@ -72,7 +81,7 @@ struct HostBuf {
 };
 
 // Cached filter response for one (W, filter): full-length real even response
-// Htilde(k) (W values), twiddles of the transform length M (M/2 complex), and for
+// Htilde(k) (W values), twiddles of the transform length M (M complex), and for
 // widths that are not powers of two the M-point transform of the periodically extended
 // filter kernel (M complex); float and double copies.
 struct FilterTables {
@@ -125,8 +134,8 @@ ctg_status ensure_filter_tables(ctg_context* ctx, int W, int filter);
 // ---- preprocess.hip
 ctg_status launch_preprocess_rows(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel,
                                   int nproj, float base, ctg_log_form form, ctg_filter filter,
-                                  float* d_out, unsigned* d_maxabs, bool do_log, bool do_weight,
-                                  bool do_filter, hipStream_t st);
+                                  float* d_out, unsigned* d_maxabs, hipStream_t st);
+ctg_status launch_feldkamp_weight(const ctg_geometry& g, float* d_images, int nproj, hipStream_t st);
 ctg_status launch_filter_rows_only(ctg_context* ctx, const float* d_in, float* d_out, int64_t rows,
                                    ctg_filter filter, hipStream_t st);
 ctg_status launch_preprocess_rows_f64(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel,

@@ -10,15 +10,17 @@
 //
 // Design: two rows are filtered at once as the real and imaginary parts of one complex
 // sequence (the response is real and even, so real rows stay real).
-//  - W = 256..2048 (FP32): one wave per row pair, values in registers, Stockham
-//    radix-16/8/4 passes exchanging through the wave's LDS region (rows_fft_kernel).
-//  - Other powers of two, and the FP64 yardstick: one workgroup per row pair, the pair
-//    in LDS, a radix-2 DIT forward FFT (bit-reversed load), the response and a
-//    conjugation, then a DIF FFT whose bit-reversed output is read back in natural order.
-//  - Other W: the row's circular convolution with the filter kernel g (length W) is
-//    the middle of a linear convolution with g extended periodically to 2W - 1 taps,
-//    done in a power-of-two transform of length M >= 2W - 1 with the LDS radix-2 pair
-//    (no wrap-around reaches the W outputs kept).
+//  - Powers of two transform at their own length.  For other W the row's circular
+//    convolution with the filter kernel g (length W) is the middle of a linear convolution
+//    with g extended periodically to 2W - 1 taps, done in a power-of-two transform of
+//    length M >= 2W - 1 (no wrap-around reaches the W outputs kept).
+//  - W = 256..2048, powers of two (FP32): one wave per row pair, values in registers,
+//    Stockham radix-16/8/4 passes exchanging through the wave's LDS region
+//    (rows_fft_kernel).
+//  - Padded rows and W = 4096, 8192 (FP32, M from 256): radix-2 stages, decimation in time
+//    forward and in frequency back, several at a time in registers (rows_r2_kernel).
+//  - Shorter transforms and the FP64 yardstick: the same radix-2 stages one at a time in
+//    LDS, one workgroup per row pair (rows_kernel).
 #include "ctg_internal.h"
 
 #include <hip/hip_fp16.h>
@@ -44,7 +46,7 @@ struct PreArgs {
     float la, lb, lk;  // p = -log((I * la + lb) * lk)
     double dla, dlb, dlk;
     float fcd, upre, vpre;
-    int do_log, do_weight, do_filter, pow2;
+    int pow2;
     int M, log2M;  // transform length: W for powers of two, else the padded length
 };
 
@@ -53,33 +55,25 @@ __device__ inline double dlog(double x) { return log(x); }
 __device__ inline float dsqrt(float x) { return sqrtf(x); }
 __device__ inline double dsqrt(double x) { return sqrt(x); }
 
+// Feldkamp weight D / sqrt(D^2 + u^2 + v^2), u = column - uPre, v = vPre - row
+template <typename T>
+__device__ inline T feldkamp(const PreArgs& a, int r, int c) {
+    const T u = (T)c - (T)a.upre;
+    const T v = (T)(-r) + (T)a.vpre;
+    const T D = (T)a.fcd;
+    return D / dsqrt(D * D + u * u + v * v);
+}
+
+// an intensity's line integral, Feldkamp weighted, or the value of a filter-only row
 template <typename T, typename Tin>
 __device__ inline T load_pixel(const Tin* __restrict__ raw, const float* __restrict__ lin, size_t idx,
                                const PreArgs& a, int r, int c) {
+    if (raw == nullptr) return (T)lin[idx];
+    const T I = (T)raw[idx];
     T x;
-    if (raw != nullptr) {
-        T I = (T)raw[idx];
-        if (a.do_log) {
-            if constexpr (sizeof(T) == 4) {
-                float y = fmaf((float)I, a.la, a.lb);
-                x = -dlog(y * a.lk);
-            } else {
-                T y = I * (T)a.dla + (T)a.dlb;
-                x = -dlog(y * (T)a.dlk);
-            }
-        } else {
-            x = I;
-        }
-    } else {
-        x = (T)lin[idx];
-    }
-    if (a.do_weight) {
-        T u = (T)c - (T)a.upre;
-        T v = (T)(-r) + (T)a.vpre;
-        T D = (T)a.fcd;
-        x = x * (D / dsqrt(D * D + u * u + v * v));
-    }
-    return x;
+    if constexpr (sizeof(T) == 4) x = -dlog(fmaf((float)I, a.la, a.lb) * a.lk);
+    else x = -dlog((I * (T)a.dla + (T)a.dlb) * (T)a.dlk);
+    return x * feldkamp<T>(a, r, c);
 }
 
 template <typename T>
@@ -130,6 +124,22 @@ __device__ inline float wave_max(float v) {
     return v;
 }
 
+// The wave's maxima of rows a and b of images pa and pb (they may differ when H is odd).
+__device__ inline void pair_max(unsigned* maxabs, long long pa, long long pb, float ma, float mb) {
+    const bool first = (threadIdx.x & 63) == 0;
+    if (pa == pb) {
+        const float m = wave_max(fmaxf(ma, mb));
+        if (first) raise_max(&maxabs[pa], m);
+    } else {
+        ma = wave_max(ma);
+        mb = wave_max(mb);
+        if (first) {
+            raise_max(&maxabs[pa], ma);
+            raise_max(&maxabs[pb], mb);
+        }
+    }
+}
+
 // One workgroup per row pair.  Output rows (T) row-major; for float output the
 // per-image max |value| is folded into maxabs with an atomic max on the bits.
 template <typename T, typename Tin>
@@ -143,99 +153,65 @@ __global__ __launch_bounds__(kRowThreads) void rows_kernel(PreArgs a, const Tin*
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* re = reinterpret_cast<T*>(smem_raw);
     T* im = re + a.M;
-    const int W = a.W;
+    const int W = a.W, M = a.M;
     const long long ra = 2ll * blockIdx.x;
     const long long rb = ra + 1;
     const bool hasb = rb < a.nrows;
     const int rin_a = (int)(ra % a.H), rin_b = (int)(rb % a.H);
     const size_t offa = (size_t)ra * W, offb = (size_t)rb * W;
 
-    if (a.do_filter && a.pow2) {
-        for (int n = threadIdx.x; n < W; n += blockDim.x) {
-            T xa = load_pixel<T, Tin>(raw, lin, offa + n, a, rin_a, n);
-            T xb = hasb ? load_pixel<T, Tin>(raw, lin, offb + n, a, rin_b, n) : (T)0;
-            unsigned pos = bitrev((unsigned)n, a.log2W);
-            re[pos] = xa;
-            im[pos] = xb;
+    // padded: y[n] = sum_m x[m] g[(n - m) mod W] = (x * h)[n + W - 1] with h[j] = g[(j - W + 1)
+    // mod W], j < 2W - 1: x zero-padded to M, times the M-point transform of h (over M,
+    // precomputed), outputs read at n + W - 1
+    for (int n = threadIdx.x; n < M; n += blockDim.x) {
+        T xa = (T)0, xb = (T)0;
+        if (n < W) {
+            xa = load_pixel<T, Tin>(raw, lin, offa + n, a, rin_a, n);
+            if (hasb) xb = load_pixel<T, Tin>(raw, lin, offb + n, a, rin_b, n);
         }
-        fft_dit<T>(re, im, W, a.log2W, tw);
-        // multiply by the real even response and conjugate: IDFT(Z) = conj(DFT(conj Z))
-        for (int k = threadIdx.x; k < W; k += blockDim.x) {
-            T h = resp[k];
-            re[k] = re[k] * h;
-            im[k] = -im[k] * h;
-        }
-        fft_dif<T>(re, im, W, a.log2W, tw);
-    } else if (a.do_filter) {
-        // y[n] = sum_m x[m] g[(n - m) mod W] = (x * h)[n + W - 1] with h[j] = g[(j - W + 1)
-        // mod W], j < 2W - 1: x zero-padded to M, times the M-point transform of h (over M,
-        // precomputed), the same conjugate trick, outputs read at n + W - 1
-        const int M = a.M;
-        for (int n = threadIdx.x; n < M; n += blockDim.x) {
-            T xa = (T)0, xb = (T)0;
-            if (n < W) {
-                xa = load_pixel<T, Tin>(raw, lin, offa + n, a, rin_a, n);
-                if (hasb) xb = load_pixel<T, Tin>(raw, lin, offb + n, a, rin_b, n);
-            }
-            unsigned pos = bitrev((unsigned)n, a.log2M);
-            re[pos] = xa;
-            im[pos] = xb;
-        }
-        fft_dit<T>(re, im, M, a.log2M, tw);
-        for (int k = threadIdx.x; k < M; k += blockDim.x) {
+        unsigned pos = bitrev((unsigned)n, a.log2M);
+        re[pos] = xa;
+        im[pos] = xb;
+    }
+    fft_dit<T>(re, im, M, a.log2M, tw);
+    // multiply by the response (real and even, complex when padded) and conjugate:
+    // IDFT(Z) = conj(DFT(conj Z))
+    for (int k = threadIdx.x; k < M; k += blockDim.x) {
+        const T xr = re[k], xi = im[k];
+        if (a.pow2) {
+            const T h = resp[k];
+            re[k] = xr * h;
+            im[k] = -xi * h;
+        } else {
             const Cx<T> h = pad_resp[k];
-            const T xr = re[k], xi = im[k];
             re[k] = xr * h.re - xi * h.im;
             im[k] = -(xr * h.im + xi * h.re);
         }
-        fft_dif<T>(re, im, M, a.log2M, tw);
-    } else {
-        for (int n = threadIdx.x; n < W; n += blockDim.x) {
-            re[n] = load_pixel<T, Tin>(raw, lin, offa + n, a, rin_a, n);
-            im[n] = hasb ? -load_pixel<T, Tin>(raw, lin, offb + n, a, rin_b, n) : (T)0;
-        }
-        __syncthreads();
     }
+    fft_dif<T>(re, im, M, a.log2M, tw);
 
     // filtered outputs sit in bit-reversed order (at n + W - 1 for padded widths)
     const int out_shift = a.pow2 ? 0 : W - 1;
-    auto out_pos = [&](int n) -> unsigned {
-        return a.do_filter ? bitrev((unsigned)(n + out_shift), a.log2M) : (unsigned)n;
-    };
-    float mloc = 0.0f;
+    float ma = 0.0f, mb = 0.0f;
     for (int n = threadIdx.x; n < W; n += blockDim.x) {
-        unsigned pos = out_pos(n);
-        T ya = re[pos];
-        T yb = -im[pos];
+        const unsigned pos = bitrev((unsigned)(n + out_shift), a.log2M);
+        const T ya = re[pos];
+        const T yb = -im[pos];
         out[offa + n] = ya;
         if (hasb) out[offb + n] = yb;
-        if constexpr (sizeof(T) == 4) {
-            mloc = fmaxf(mloc, fabsf((float)ya));
-            if (hasb) mloc = fmaxf(mloc, fabsf((float)yb));
-        }
+        ma = fmaxf(ma, fabsf((float)ya));
+        if (hasb) mb = fmaxf(mb, fabsf((float)yb));
     }
-    if constexpr (sizeof(T) == 4) {
-        if (maxabs != nullptr) {
-            // rows a and b may belong to different images when H is odd
-            const long long pa = ra / a.H, pb = hasb ? rb / a.H : pa;
-            if (pa == pb) {
-                float m = wave_max(mloc);
-                if ((threadIdx.x & 63) == 0) atomicMax(&maxabs[pa], __float_as_uint(m));
-            } else {
-                float ma = 0.0f, mb = 0.0f;
-                for (int n = threadIdx.x; n < W; n += blockDim.x) {
-                    unsigned pos = out_pos(n);
-                    ma = fmaxf(ma, fabsf((float)re[pos]));
-                    mb = fmaxf(mb, fabsf((float)im[pos]));
-                }
-                ma = wave_max(ma);
-                mb = wave_max(mb);
-                if ((threadIdx.x & 63) == 0) {
-                    atomicMax(&maxabs[pa], __float_as_uint(ma));
-                    atomicMax(&maxabs[pb], __float_as_uint(mb));
-                }
-            }
-        }
+    if (sizeof(T) == 4 && maxabs != nullptr) pair_max(maxabs, ra / a.H, hasb ? rb / a.H : ra / a.H, ma, mb);
+}
+
+// Feldkamp weight in place, one lane per pixel.
+__global__ __launch_bounds__(256) void weight_kernel(PreArgs a, float* __restrict__ img) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= a.W) return;
+    for (long long r = blockIdx.y; r < a.nrows; r += gridDim.y) {
+        float* px = img + (size_t)r * a.W + c;
+        *px = *px * feldkamp<float>(a, (int)(r % a.H), c);
     }
 }
 
@@ -252,6 +228,11 @@ __global__ __launch_bounds__(kRowThreads) void rows_kernel(PreArgs a, const Tin*
 // filtered rows are the conjugate of the forward transform of conj(X * H), so the same
 // forward passes run twice; the first pass reads the raw pixels from global memory and
 // the last writes the filtered rows.
+//
+// What bounds it (MI355X, N = 2048): VALU issue 50 % busy and the vector memory unit 43 %
+// at 2 waves per SIMD.  A twiddle gather holds that unit about 16 cycles, so pass 1 takes
+// its twiddles from a table in LDS and short transforms keep the last pass's in registers
+// for both directions: 48 images of 2048 x 1536 in 0.38 ms instead of 0.53.
 namespace fftw {
 
 __host__ __device__ constexpr int passes(int N) { return N == 256 ? 4 : 3; }
@@ -259,6 +240,8 @@ __host__ __device__ constexpr int radix(int N, int i) {
     return N == 256 ? 4 : (N == 512 ? 8 : (i < 2 ? 16 : (N == 1024 ? 4 : 8)));
 }
 __host__ __device__ constexpr int stride(int N, int i) { return i == 0 ? 1 : stride(N, i - 1) * radix(N, i - 1); }
+// entries of pass 1's twiddle table
+__host__ __device__ constexpr int ltw_size(int N) { return radix(N, 0) * radix(N, 1); }
 // LDS position of element i: one float2 of padding per 16 spreads the strided writes
 __device__ inline int lds_pos(int i) { return i + (i >> 4); }
 
@@ -325,13 +308,6 @@ __device__ inline void dft(F2* a) {
     else dft16(a);
 }
 
-// exp(-2 pi i k / N) for 0 <= k < N from the half table exp(-2 pi i m / N), m < N/2
-template <int N>
-__device__ inline F2 twiddle(const Cx<float>* __restrict__ tw, int k) {
-    const Cx<float> t = tw[k & (N / 2 - 1)];
-    return (k & (N / 2)) ? F2{-t.re, -t.im} : F2{t.re, t.im};
-}
-
 // orders the wave's LDS stores and loads around a cross-lane exchange
 __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -339,59 +315,87 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// LDS element that value b*R + r of a pass's inputs (load) or outputs (store) lives at
 template <int N, int I>
-__device__ inline void load_pass(const F2* __restrict__ buf, F2 (&v)[N / 64], int lane) {
-    constexpr int R = radix(N, I), B = N / 64 / R;
-#pragma unroll
-    for (int b = 0; b < B; ++b)
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[b * R + r] = buf[lds_pos(lane + 64 * b + r * (N / R))];
+__device__ inline int load_at(int lane, int i) {
+    constexpr int R = radix(N, I);
+    return lds_pos(lane + 64 * (i / R) + (i % R) * (N / R));
+}
+template <int N, int I>
+__device__ inline int store_at(int lane, int i) {
+    constexpr int R = radix(N, I), NS = stride(N, I);
+    const int j = lane + 64 * (i / R);
+    return lds_pos((j / NS) * NS * R + (j % NS) + (i % R) * NS);
 }
 
+// Moves the values through LDS from where `from` puts them to where `to` takes them.
+template <int N, class From, class To>
+__device__ inline void exchange(F2* __restrict__ buf, F2 (&v)[N / 64], From from, To to) {
+    constexpr int P = N / 64;
+#pragma unroll
+    for (int i = 0; i < P; ++i) buf[from(i)] = v[i];
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < P; ++i) v[i] = buf[to(i)];
+    wave_sync();
+}
+
+// Twiddles of pass I: w[b*R + r] = exp(-2 pi i (j mod NS) r / (NS R)), r > 0.
 template <int N, int I>
-__device__ inline void store_pass(F2* __restrict__ buf, const F2 (&v)[N / 64], int lane) {
+__device__ inline void load_twiddles(F2 (&w)[N / 64], int lane, const Cx<float>* __restrict__ tw) {
     constexpr int R = radix(N, I), NS = stride(N, I), B = N / 64 / R;
 #pragma unroll
     for (int b = 0; b < B; ++b) {
-        const int j = lane + 64 * b;
-        const int base = (j / NS) * NS * R + (j % NS);
+        const int jm = (lane + 64 * b) % NS;
 #pragma unroll
-        for (int r = 0; r < R; ++r) buf[lds_pos(base + r * NS)] = v[b * R + r];
-    }
-}
-
-// Passes I.. of one forward transform.  On entry v holds pass I's inputs; on return
-// v holds the last pass's outputs: value b*R + r is X[lane + 64 b + r * NS_last].
-template <int N, int I>
-__device__ inline void passes_from(F2 (&v)[N / 64], F2* __restrict__ buf, int lane,
-                                   const Cx<float>* __restrict__ tw) {
-    constexpr int R = radix(N, I), NS = stride(N, I), B = N / 64 / R;
-    // an opaque zero offset per pass: the twiddles are then loaded where they are used
-    // instead of being hoisted and kept live across both transforms
-    int zero = 0;
-    asm volatile("" : "+s"(zero));
-    const Cx<float>* twp = tw + zero;
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-        if constexpr (NS > 1) {
-            const int jm = (lane + 64 * b) % NS;
-#pragma unroll
-            for (int r = 1; r < R; ++r) v[b * R + r] = mul(v[b * R + r], twiddle<N>(twp, jm * r * (N / (NS * R))));
+        for (int r = 1; r < R; ++r) {
+            const Cx<float> t = tw[jm * r * (N / (NS * R))];
+            w[b * R + r] = F2{t.re, t.im};
         }
-        dft<R>(v + b * R);
     }
+}
+
+// Passes I.. of one forward transform.  On entry v holds pass I's inputs; on return v holds
+// the last pass's outputs: value b*R + r is X[lane + 64 b + r * NS_last].  Twiddles: pass 1
+// reads the short table ltw (exp(-2 pi i q / (NS R)), in LDS), the last pass takes `last`
+// (KEEP: registers, the same for both transforms), other passes read the global table.
+template <int N, int I, bool KEEP>
+__device__ inline void passes_from(F2 (&v)[N / 64], const F2 (&last)[N / 64], F2* __restrict__ buf,
+                                   const F2* __restrict__ ltw, int lane, const Cx<float>* __restrict__ tw) {
+    constexpr int R = radix(N, I), NS = stride(N, I), B = N / 64 / R;
+    if constexpr (I == 1) {
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[b * R + r] = mul(v[b * R + r], ltw[(lane + 64 * b) % NS * r]);
+    } else if constexpr (KEEP && I == passes(N) - 1) {
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[b * R + r] = mul(v[b * R + r], last[b * R + r]);
+    } else if constexpr (I > 0) {
+        // an opaque zero offset: loaded where they are used instead of being hoisted and
+        // kept live across both transforms
+        int zero = 0;
+        asm volatile("" : "+s"(zero));
+        F2 w[N / 64];
+        load_twiddles<N, I>(w, lane, tw + zero);
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[b * R + r] = mul(v[b * R + r], w[b * R + r]);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) dft<R>(v + b * R);
     if constexpr (I + 1 < passes(N)) {
-        store_pass<N, I>(buf, v, lane);
-        wave_sync();
-        load_pass<N, I + 1>(buf, v, lane);
-        wave_sync();
-        passes_from<N, I + 1>(v, buf, lane, tw);
+        exchange<N>(buf, v, [=](int i) { return store_at<N, I>(lane, i); }, [=](int i) { return load_at<N, I + 1>(lane, i); });
+        passes_from<N, I + 1, KEEP>(v, last, buf, ltw, lane, tw);
     }
 }
 
 }  // namespace fftw
 
-// row pairs (waves) per workgroup; LDS is (N + N/16) float2 per wave
+// row pairs (waves) per workgroup; LDS is (N + N/16) float2 per wave, and pass 1's table
 __host__ __device__ constexpr int fft_waves(int N) { return N >= 2048 ? 2 : 4; }
 
 template <int N, typename Tin>
@@ -408,96 +412,386 @@ __global__ __launch_bounds__(64 * fft_waves(N)) void rows_fft_kernel(PreArgs a, 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     F2* buf = reinterpret_cast<F2*>(smem_raw) + (size_t)wave * (N + N / 16);
+    F2* ltw = reinterpret_cast<F2*>(smem_raw) + (size_t)fft_waves(N) * (N + N / 16);
+    constexpr int S = ltw_size(N);
+    for (int q = threadIdx.x; q < S; q += 64 * fft_waves(N)) {
+        const Cx<float> t = tw[q * (N / S)];
+        ltw[q] = F2{t.re, t.im};
+    }
+    __syncthreads();
     const long long pair = (long long)blockIdx.x * fft_waves(N) + wave;
     const long long ra = 2 * pair, rb = ra + 1;
-    if (ra >= a.nrows) return;  // waves share nothing, so a finished wave may leave
+    if (ra >= a.nrows) return;  // waves share nothing more, so a finished wave may leave
     const bool hasb = rb < a.nrows;
     const int rin_a = (int)(ra % a.H), rin_b = (int)(rb % a.H);
     const size_t offa = (size_t)ra * N, offb = (size_t)rb * N;
 
     F2 v[P];
     // pass 0 inputs straight from the images: x[lane + 64 b + r N/R0].  All loads are
-    // issued first (a missing row b re-reads row a and is zeroed below); the uniform
-    // log and weight flags are tested once, outside the per-pixel loops.
+    // issued first (a missing row b re-reads row a and is zeroed below).
     const size_t offb_ld = hasb ? offb : offa;
+    auto col = [&](int i) { return lane + 64 * (i / R0) + (i % R0) * (N / R0); };
     if (raw != nullptr) {
 #pragma unroll
         for (int i = 0; i < P; ++i) {
-            const int n = lane + 64 * (i / R0) + (i % R0) * (N / R0);
-            v[i].x = (float)raw[offa + n];
-            v[i].y = (float)raw[offb_ld + n];
+            v[i].x = (float)raw[offa + col(i)];
+            v[i].y = (float)raw[offb_ld + col(i)];
         }
-        if (a.do_log) {
 #pragma unroll
-            for (int i = 0; i < P; ++i) {
-                v[i].x = -logf(fmaf(v[i].x, a.la, a.lb) * a.lk);
-                v[i].y = -logf(fmaf(v[i].y, a.la, a.lb) * a.lk);
-            }
+        for (int i = 0; i < P; ++i) {
+            v[i].x = -logf(fmaf(v[i].x, a.la, a.lb) * a.lk) * feldkamp<float>(a, rin_a, col(i));
+            v[i].y = -logf(fmaf(v[i].y, a.la, a.lb) * a.lk) * feldkamp<float>(a, rin_b, col(i));
         }
     } else {
 #pragma unroll
         for (int i = 0; i < P; ++i) {
-            const int n = lane + 64 * (i / R0) + (i % R0) * (N / R0);
-            v[i].x = lin[offa + n];
-            v[i].y = lin[offb_ld + n];
-        }
-    }
-    if (a.do_weight) {
-        // D / sqrt(D^2 + u^2 + v^2), u = column - uPre, v = vPre - row
-        const float D = a.fcd;
-        const float va = (float)(-rin_a) + a.vpre, vb = (float)(-rin_b) + a.vpre;
-#pragma unroll
-        for (int i = 0; i < P; ++i) {
-            const int n = lane + 64 * (i / R0) + (i % R0) * (N / R0);
-            const float u = (float)n - a.upre;
-            const float du = D * D + u * u;
-            v[i].x = v[i].x * (D / sqrtf(du + va * va));
-            v[i].y = v[i].y * (D / sqrtf(du + vb * vb));
+            v[i].x = lin[offa + col(i)];
+            v[i].y = lin[offb_ld + col(i)];
         }
     }
     if (!hasb) {
 #pragma unroll
         for (int i = 0; i < P; ++i) v[i].y = 0.0f;
     }
-    passes_from<N, 0>(v, buf, lane, tw);
+    // where the registers hold them beside the values without spilling
+    constexpr bool KEEP = N <= 512;
+    F2 last[P];
+    if constexpr (KEEP) load_twiddles<N, LAST>(last, lane, tw);
+    passes_from<N, 0, KEEP>(v, last, buf, ltw, lane, tw);
     // multiply by the real even response and conjugate; back to pass 0's distribution
 #pragma unroll
-    for (int b = 0; b < P / RL; ++b)
-#pragma unroll
-        for (int r = 0; r < RL; ++r) {
-            const int k = lane + 64 * b + r * NSL;
-            const float h = resp[k];
-            const F2 z = v[b * RL + r];
-            buf[lds_pos(k)] = F2{z.x * h, -(z.y * h)};
-        }
-    wave_sync();
-    load_pass<N, 0>(buf, v, lane);
-    wave_sync();
-    passes_from<N, 0>(v, buf, lane, tw);
+    for (int i = 0; i < P; ++i) {
+        const float h = resp[lane + 64 * (i / RL) + (i % RL) * NSL];
+        v[i] = F2{v[i].x * h, -(v[i].y * h)};
+    }
+    exchange<N>(buf, v, [=](int i) { return lds_pos(lane + 64 * (i / RL) + (i % RL) * NSL); },
+                [=](int i) { return load_at<N, 0>(lane, i); });
+    passes_from<N, 0, KEEP>(v, last, buf, ltw, lane, tw);
 
-    float mloc = 0.0f, ma = 0.0f, mb = 0.0f;
+    float ma = 0.0f, mb = 0.0f;
 #pragma unroll
-    for (int b = 0; b < P / RL; ++b)
+    for (int i = 0; i < P; ++i) {
+        const int n = lane + 64 * (i / RL) + (i % RL) * NSL;
+        const float ya = v[i].x, yb = -v[i].y;
+        out[offa + n] = ya;
+        if (hasb) out[offb + n] = yb;
+        ma = fmaxf(ma, fabsf(ya));
+        mb = fmaxf(mb, fabsf(yb));
+    }
+    if (maxabs != nullptr) pair_max(maxabs, ra / a.H, hasb ? rb / a.H : ra / a.H, ma, hasb ? mb : 0.0f);
+}
+
+// ---------------------------------------------------------------------------------
+// Register-resident radix-2 row filter (FP32): padded rows, and W = 4096 ... 16384.
+//
+// The stages and their arithmetic are rows_kernel's (a radix-2 decimation in time, the
+// response, a decimation in frequency back), product by product, so the rows are the same
+// bit for bit whichever kernel filters them.  What differs is where values live: T lanes
+// hold P = M/T of them each and run s stages at a time in registers.  A pass over stages
+// [a, a + s) takes groups of 2^s elements pos = hi 2^(a+s) + m 2^a + k (m < 2^s, k < 2^a);
+// between passes the values move through LDS, within one wave without a workgroup barrier.
+//  - Pass 0 (s = log2 P, k = 0): lane t holds positions P rev(t) + m, whose natural
+//    indices rev(m) M/P + t are consecutive over the lanes, on the way in and out.
+//  - The last pass runs its stages, the response and its stages of the way back in one
+//    stay in registers, on one set of twiddles.
+//  - Padded rows fill less than half of M: odd m of pass 0 are zero, whatever W.
+// One float2 of padding per 2^(L-5) positions and, in pass 1, five low bits of hi before k
+// in the lane number make the LDS accesses conflict-free (up to two-way at 9, 13 and 14).
+//
+// What bounds it (MI355X, M = 4096): VALU issue and the vector memory unit, each about
+// half busy, at 16 waves per CU (35 KB of LDS per row pair).  40 images of 1944 x 1536:
+// 2.67 ms one stage at a time in LDS, 0.51 ms here.
+namespace r2 {
+
+using fftw::F2;
+
+__host__ __device__ constexpr int lanes(int L) { return L == 8 ? 16 : (L == 9 || L == 10) ? 64 : (1 << L) / 16; }
+__host__ __device__ constexpr int values(int L) { return (1 << L) / lanes(L); }
+__host__ __device__ constexpr int passes(int L) { return L == 8 ? 2 : (L <= 12 ? 3 : 4); }
+// stages of pass i
+__host__ __device__ constexpr int stages(int L, int i) {
+    return L == 9 ? 3 : i == 0 ? 4 : (L == 10 || L == 13) ? 3 : (L == 11 ? (i == 1 ? 4 : 3) : (L == 14 ? (i == 1 ? 4 : 3) : 4));
+}
+__host__ __device__ constexpr int first(int L, int i) { return i == 0 ? 0 : first(L, i - 1) + stages(L, i - 1); }
+__host__ __device__ constexpr int pad_shift(int L) { return L == 8 ? 3 : L == 9 ? 4 : (L <= 12 ? L - 5 : L - 6); }
+// row pairs and lanes per workgroup, LDS per pair (float2) and per workgroup (bytes; the
+// second part is pass 1's twiddle table)
+__host__ __device__ constexpr int pairs(int L) { return lanes(L) <= 64 ? 256 / lanes(L) : 1; }
+__host__ __device__ constexpr int threads(int L) { return lanes(L) * pairs(L); }
+__host__ __device__ constexpr int pair_lds(int L) { return (1 << L) + ((1 << L) >> pad_shift(L)); }
+__host__ __device__ constexpr int ltw_size(int L) { return 1 << (first(L, 1) + stages(L, 1) - 1); }
+__host__ __device__ constexpr int lds_bytes(int L) { return (pairs(L) * pair_lds(L) + ltw_size(L)) * 8; }
+
+__host__ __device__ constexpr int rev(int x, int bits) {
+    int r = 0;
+    for (int i = 0; i < bits; ++i) r |= ((x >> i) & 1) << (bits - 1 - i);
+    return r;
+}
+
+// k and hi of group b of a lane in pass I > 0
+template <int L, int I>
+__device__ inline void group_of(int lane, int b, int& k, int& hi) {
+    constexpr int a = first(L, I), nh = L - stages(L, I) - a;
+    const int g = lane + lanes(L) * b;
+    if constexpr (I == 1 && I < passes(L) - 1) {
+        constexpr int h1 = nh < 5 ? nh : 5;
+        hi = (g & ((1 << h1) - 1)) | ((g >> (h1 + a)) << h1);
+        k = (g >> h1) & ((1 << a) - 1);
+    } else {
+        k = g & ((1 << a) - 1);
+        hi = g >> a;
+    }
+}
+
+// LDS place of value i of a lane in pass I
+template <int L, int I>
+__device__ inline int place(int lane, int i) {
+    constexpr int s = stages(L, I), a = first(L, I);
+    int pos;
+    if constexpr (I == 0) {
+        pos = ((int)(__brev((unsigned)lane) >> (32 - (L - s))) << s) + i;
+    } else {
+        int k, hi;
+        group_of<L, I>(lane, i >> s, k, hi);
+        pos = (hi << (a + s)) + ((i & ((1 << s) - 1)) << a) + k;
+    }
+    return pos + (pos >> pad_shift(L));
+}
+
+template <int L>
+__device__ inline void pair_sync() {
+    if constexpr (lanes(L) > 64) __syncthreads();
+    else fftw::wave_sync();
+}
+
+template <int L, int I, int J>
+__device__ inline void exchange(F2 (&v)[values(L)], F2* __restrict__ buf, int lane) {
 #pragma unroll
-        for (int r = 0; r < RL; ++r) {
-            const int k = lane + 64 * b + r * NSL;
-            const float ya = v[b * RL + r].x, yb = -v[b * RL + r].y;
-            out[offa + k] = ya;
-            if (hasb) out[offb + k] = yb;
-            ma = fmaxf(ma, fabsf(ya));
+    for (int i = 0; i < values(L); ++i) buf[place<L, I>(lane, i)] = v[i];
+    pair_sync<L>();
+#pragma unroll
+    for (int i = 0; i < values(L); ++i) v[i] = buf[place<L, J>(lane, i)];
+    pair_sync<L>();
+}
+
+__device__ inline F2 cmul(F2 b, F2 w) { return {b.x * w.x - b.y * w.y, b.x * w.y + b.y * w.x}; }
+
+// b exp(-2 pi i mm / 2^(j+1)), the twiddles of pass 0 (those off the axes as the table
+// rounds them)
+template <int J>
+__device__ inline F2 cmul_const(F2 b, int mm) {
+    constexpr float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f, h = 0.70710678118654752440f;
+    switch (mm << (3 - J)) {  // sixteenths of a turn
+        case 0: return b;
+        case 1: return cmul(b, F2{c1, -s1});
+        case 2: return cmul(b, F2{h, -h});
+        case 3: return cmul(b, F2{s1, -c1});
+        case 4: return F2{b.y, -b.x};
+        case 5: return cmul(b, F2{-s1, -c1});
+        case 6: return cmul(b, F2{-h, -h});
+        default: return cmul(b, F2{-c1, -s1});
+    }
+}
+
+// stage J of a group of 2^S; twiddle mm of stage j is w[2^j - 1 + mm] (CONST: pass 0)
+template <int S, int J, bool CONST, bool HALF>
+__device__ inline void dit_from(F2* v, const F2* w) {
+    if constexpr (J < S) {
+#pragma unroll
+        for (int m = 0; m < (1 << S); ++m) {
+            if (m & (1 << J)) continue;
+            const int mm = m & ((1 << J) - 1);
+            F2 &x = v[m], &y = v[m + (1 << J)];
+            if constexpr (HALF && J == 0) {
+                y = x;  // y is zero
+            } else {
+                F2 t;
+                if constexpr (CONST) t = cmul_const<J>(y, mm);
+                else t = cmul(y, w[(1 << J) - 1 + mm]);
+                y = fftw::sub(x, t);
+                x = fftw::add(x, t);
+            }
+        }
+        dit_from<S, J + 1, CONST, HALF>(v, w);
+    }
+}
+template <int S, int J, bool CONST>
+__device__ inline void dif_from(F2* v, const F2* w) {
+    if constexpr (J >= 0) {
+#pragma unroll
+        for (int m = 0; m < (1 << S); ++m) {
+            if (m & (1 << J)) continue;
+            const int mm = m & ((1 << J) - 1);
+            F2 &x = v[m], &y = v[m + (1 << J)];
+            const F2 d = fftw::sub(x, y);
+            x = fftw::add(x, y);
+            if constexpr (CONST) y = cmul_const<J>(d, mm);
+            else y = cmul(d, w[(1 << J) - 1 + mm]);
+        }
+        dif_from<S, J - 1, CONST>(v, w);
+    }
+}
+
+// Twiddles of pass I > 0: the short LDS table for pass 1, else the global table.
+template <int L, int I>
+__device__ inline void load_twiddles(F2 (&w)[values(L)], int lane, const F2* __restrict__ ltw,
+                                     const Cx<float>* __restrict__ tw) {
+    constexpr int s = stages(L, I), a = first(L, I), B = values(L) >> s;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        int k, hi;
+        group_of<L, I>(lane, b, k, hi);
+#pragma unroll
+        for (int j = 0; j < s; ++j)
+#pragma unroll
+            for (int mm = 0; mm < (1 << j); ++mm) {
+                F2& d = w[(b << s) + (1 << j) - 1 + mm];
+                if constexpr (I == 1) {
+                    d = ltw[(k + (mm << a)) << (s - 1 - j)];
+                } else {
+                    const Cx<float> t = tw[(k + (mm << a)) << (L - 1 - a - j)];
+                    d = F2{t.re, t.im};
+                }
+            }
+    }
+}
+
+// Passes I.. there, the response, and back to pass I - 1's distribution.
+template <int L, int I, class Response>
+__device__ inline void passes_from(F2 (&v)[values(L)], F2* __restrict__ buf, const F2* __restrict__ ltw, int lane,
+                                   const Cx<float>* __restrict__ tw, Response response) {
+    constexpr int s = stages(L, I), B = values(L) >> s;
+    constexpr bool last = I == passes(L) - 1;
+    exchange<L, I - 1, I>(v, buf, lane);
+    {
+        F2 w[values(L)];
+        load_twiddles<L, I>(w, lane, ltw, tw);
+#pragma unroll
+        for (int b = 0; b < B; ++b) dit_from<s, 0, false, false>(v + (b << s), w + (b << s));
+        if constexpr (last) {
+            response(v);
+#pragma unroll
+            for (int b = 0; b < B; ++b) dif_from<s, s - 1, false>(v + (b << s), w + (b << s));
+        }
+    }
+    if constexpr (!last) {
+        passes_from<L, I + 1>(v, buf, ltw, lane, tw, response);
+        // an opaque zero offset: the twiddles are read again instead of being kept live
+        int zero = 0;
+        asm volatile("" : "+s"(zero));
+        F2 w[values(L)];
+        load_twiddles<L, I>(w, lane, ltw + zero, tw + zero);
+#pragma unroll
+        for (int b = 0; b < B; ++b) dif_from<s, s - 1, false>(v + (b << s), w + (b << s));
+    }
+    exchange<L, I, I - 1>(v, buf, lane);
+}
+
+}  // namespace r2
+
+template <int L, bool PAD, typename Tin>
+__global__ __launch_bounds__(r2::threads(L)) __attribute__((amdgpu_waves_per_eu(4))) void rows_r2_kernel(
+    PreArgs a, const Tin* __restrict__ raw, const float* __restrict__ lin, const float* __restrict__ resp,
+    const Cx<float>* __restrict__ pad_resp, const Cx<float>* __restrict__ tw, float* __restrict__ out,
+    unsigned* __restrict__ maxabs) {
+    using namespace r2;
+    constexpr int M = 1 << L, T = lanes(L), P = values(L), S0 = stages(L, 0), LAST = passes(L) - 1;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int slot = threadIdx.x / T, lane = threadIdx.x % T;
+    F2* buf = reinterpret_cast<F2*>(smem_raw) + (size_t)slot * pair_lds(L);
+    F2* ltw = reinterpret_cast<F2*>(smem_raw) + (size_t)pairs(L) * pair_lds(L);
+    for (int q = threadIdx.x; q < ltw_size(L); q += threads(L)) {
+        const Cx<float> t = tw[q * (M / (2 * ltw_size(L)))];
+        ltw[q] = F2{t.re, t.im};
+    }
+    __syncthreads();
+    // lanes of a pair past the end re-read the last row and store nothing
+    const long long ra0 = 2 * ((long long)blockIdx.x * pairs(L) + slot);
+    const bool hasa = ra0 < a.nrows, hasb = ra0 + 1 < a.nrows;
+    const long long ra = hasa ? ra0 : a.nrows - 1, rb = hasb ? ra0 + 1 : ra;
+    const int W = a.W;
+    const int rin_a = (int)(ra % a.H), rin_b = (int)(rb % a.H);
+    const size_t offa = (size_t)ra * W, offb = (size_t)rb * W;
+
+    // natural index of value m in pass 0
+    auto col = [&](int m) { return rev(m, S0) * (M / P) + lane; };
+    auto used = [](int m) { return !PAD || (m & 1) == 0; };
+    F2 v[P];
+    // all loads are issued first (columns past the row re-read its last one); what does not
+    // exist is zeroed below
+    if (raw != nullptr) {
+#pragma unroll
+        for (int m = 0; m < P; ++m) {
+            if (!used(m)) continue;
+            const int n = PAD ? min(col(m), W - 1) : col(m);
+            v[m].x = (float)raw[offa + n];
+            v[m].y = (float)raw[offb + n];
+        }
+#pragma unroll
+        for (int m = 0; m < P; ++m) {
+            if (!used(m)) continue;
+            v[m].x = -logf(fmaf(v[m].x, a.la, a.lb) * a.lk) * feldkamp<float>(a, rin_a, col(m));
+            v[m].y = -logf(fmaf(v[m].y, a.la, a.lb) * a.lk) * feldkamp<float>(a, rin_b, col(m));
+        }
+    } else {
+#pragma unroll
+        for (int m = 0; m < P; ++m) {
+            if (!used(m)) continue;
+            const int n = PAD ? min(col(m), W - 1) : col(m);
+            v[m].x = lin[offa + n];
+            v[m].y = lin[offb + n];
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+        if (!used(m) || (PAD && col(m) >= W)) v[m] = F2{0.0f, 0.0f};
+        if (!hasb) v[m].y = 0.0f;
+    }
+    dit_from<S0, 0, true, PAD>(v, nullptr);
+    passes_from<L, 1>(v, buf, ltw, lane, tw, [&](F2(&z)[P]) {
+        // multiply by the response (real and even, complex when padded) and conjugate
+        constexpr int s = stages(L, LAST), f = first(L, LAST);
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const int k = lane + T * (i >> s) + ((i & ((1 << s) - 1)) << f);
+            if constexpr (PAD) {
+                const Cx<float> h = pad_resp[k];
+                const F2 y = cmul(z[i], F2{h.re, h.im});
+                z[i] = F2{y.x, -y.y};
+            } else {
+                const float h = resp[k];
+                z[i] = F2{z[i].x * h, -z[i].y * h};
+            }
+        }
+    });
+    dif_from<S0, S0 - 1, true>(v, nullptr);
+
+    const int shift = PAD ? W - 1 : 0;
+    float ma = 0.0f, mb = 0.0f;
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+        const int n = col(m) - shift;
+        if (!hasa || (PAD && (n < 0 || n >= W))) continue;
+        const float ya = v[m].x, yb = -v[m].y;
+        out[offa + n] = ya;
+        ma = fmaxf(ma, fabsf(ya));
+        if (hasb) {
+            out[offb + n] = yb;
             mb = fmaxf(mb, fabsf(yb));
         }
+    }
     if (maxabs != nullptr) {
-        const long long pa = ra / a.H, pb = hasb ? rb / a.H : pa;
-        if (pa == pb) {
-            mloc = wave_max(fmaxf(ma, hasb ? mb : 0.0f));
-            if (lane == 0) atomicMax(&maxabs[pa], __float_as_uint(mloc));
+        if constexpr (T >= 64) {
+            if (hasa) pair_max(maxabs, ra / a.H, rb / a.H, ma, mb);
         } else {
-            ma = wave_max(ma);
-            mb = wave_max(mb);
-            if (lane == 0) {
-                atomicMax(&maxabs[pa], __float_as_uint(ma));
-                atomicMax(&maxabs[pb], __float_as_uint(mb));
+            // several pairs per wave
+            for (int off = T / 2; off > 0; off >>= 1) {
+                ma = fmaxf(ma, __shfl_xor(ma, off, 64));
+                mb = fmaxf(mb, __shfl_xor(mb, off, 64));
+            }
+            if (lane == 0 && hasa) {
+                raise_max(&maxabs[ra / a.H], ma);
+                if (hasb) raise_max(&maxabs[rb / a.H], mb);
             }
         }
     }
@@ -580,16 +874,16 @@ int filter_log2_length(int W) {
     return m;
 }
 
+// the LDS row buffer holds transforms of up to `most` points
+ctg_status check_transform(const PreArgs& a, int most) {
+    if (a.M <= most) return CTG_OK;
+    return fail(CTG_ERROR_UNSUPPORTED, "detector width %d (transform length %d) exceeds the LDS row buffer", a.W, a.M);
+}
+
 void set_transform(PreArgs& a) {
-    a.log2W = ilog2_exact(a.W);
-    a.pow2 = a.log2W >= 0;
-    if (a.do_filter) {
-        a.log2M = filter_log2_length(a.W);
-        a.M = 1 << a.log2M;
-    } else {
-        a.log2M = a.log2W;
-        a.M = a.W;
-    }
+    a.pow2 = ilog2_exact(a.W) >= 0;
+    a.log2M = filter_log2_length(a.W);
+    a.M = 1 << a.log2M;
 }
 
 void fill_log_params(PreArgs& a, ctg_pixel_type pixel, float base, ctg_log_form form) {
@@ -611,67 +905,92 @@ void fill_log_params(PreArgs& a, ctg_pixel_type pixel, float base, ctg_log_form 
     a.lk = (float)a.dlk;
 }
 
-template <int N>
-ctg_status launch_rows_fft(const void* raw, ctg_pixel_type pixel, const float* lin, long long nrows,
-                           const PreArgs& a, const float* resp, const Cx<float>* tw, float* out,
-                           unsigned* maxabs, hipStream_t st) {
-    constexpr int waves = fft_waves(N);
-    const long long pairs = (nrows + 1) / 2;
-    const long long blocks = (pairs + waves - 1) / waves;
+// Launches KERNEL<..., Tin> for the pixel type of `raw` (float for filter-only rows).
+#define CTG_ROWS_LAUNCH(KERNEL, ...)                                                                        \
+    do {                                                                                                    \
+        if (raw != nullptr && pixel == CTG_PIXEL_U8)                                                        \
+            hipLaunchKernelGGL((KERNEL(uint8_t)), grid, block, lds, st, a, (const uint8_t*)raw, __VA_ARGS__);   \
+        else if (raw != nullptr && pixel == CTG_PIXEL_U16)                                                  \
+            hipLaunchKernelGGL((KERNEL(uint16_t)), grid, block, lds, st, a, (const uint16_t*)raw, __VA_ARGS__); \
+        else                                                                                                \
+            hipLaunchKernelGGL((KERNEL(float)), grid, block, lds, st, a, (const float*)raw, __VA_ARGS__);   \
+    } while (0)
+
+// workgroups for `pairs` row pairs, `per` in each
+ctg_status row_blocks(long long pairs, int per, dim3& grid) {
+    const long long blocks = (pairs + per - 1) / per;
     if (blocks > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "too many detector rows in one call");
-    const size_t lds = (size_t)waves * (N + N / 16) * sizeof(fftw::F2);
-    const dim3 grid((unsigned)blocks), block(64 * waves);
-    if (raw == nullptr) {
-        hipLaunchKernelGGL((rows_fft_kernel<N, float>), grid, block, lds, st, a, (const float*)nullptr, lin, resp,
-                           tw, out, maxabs);
-    } else if (pixel == CTG_PIXEL_U8) {
-        hipLaunchKernelGGL((rows_fft_kernel<N, uint8_t>), grid, block, lds, st, a, (const uint8_t*)raw, lin, resp,
-                           tw, out, maxabs);
-    } else if (pixel == CTG_PIXEL_U16) {
-        hipLaunchKernelGGL((rows_fft_kernel<N, uint16_t>), grid, block, lds, st, a, (const uint16_t*)raw, lin,
-                           resp, tw, out, maxabs);
-    } else {
-        hipLaunchKernelGGL((rows_fft_kernel<N, float>), grid, block, lds, st, a, (const float*)raw, lin, resp, tw,
-                           out, maxabs);
-    }
+    grid = dim3((unsigned)blocks);
+    return CTG_OK;
+}
+
+template <int N>
+ctg_status launch_rows_fft(const FilterTables& ft, const void* raw, ctg_pixel_type pixel, const float* lin,
+                           const PreArgs& a, float* out, unsigned* maxabs, hipStream_t st) {
+    constexpr int waves = fft_waves(N);
+    dim3 grid;
+    CTG_TRY(row_blocks((a.nrows + 1) / 2, waves, grid));
+    const dim3 block(64 * waves);
+    const size_t lds = ((size_t)waves * (N + N / 16) + fftw::ltw_size(N)) * sizeof(fftw::F2);
+#define CTG_K(Tin) rows_fft_kernel<N, Tin>
+    CTG_ROWS_LAUNCH(CTG_K, lin, ft.resp_f.as<float>(), ft.tw_f.as<Cx<float>>(), out, maxabs);
+#undef CTG_K
     CTG_HIP(hipGetLastError());
     return CTG_OK;
 }
 
-template <typename T>
-ctg_status launch_rows(ctg_context* ctx, const void* raw, ctg_pixel_type pixel, const float* lin,
-                       long long nrows, const PreArgs& a, T* out, unsigned* maxabs, hipStream_t st) {
+template <int L, bool PAD>
+ctg_status launch_rows_r2(const FilterTables& ft, const void* raw, ctg_pixel_type pixel, const float* lin,
+                          const PreArgs& a, float* out, unsigned* maxabs, hipStream_t st) {
+    dim3 grid;
+    CTG_TRY(row_blocks((a.nrows + 1) / 2, r2::pairs(L), grid));
+    const dim3 block(r2::threads(L));
+    const size_t lds = r2::lds_bytes(L);
+#define CTG_K(Tin) rows_r2_kernel<L, PAD, Tin>
+    CTG_ROWS_LAUNCH(CTG_K, lin, ft.resp_f.as<float>(), ft.pad_f.as<Cx<float>>(), ft.tw_f.as<Cx<float>>(), out, maxabs);
+#undef CTG_K
+    CTG_HIP(hipGetLastError());
+    return CTG_OK;
+}
+
+// Filters a.nrows rows of raw images (log, weight) or of line integrals `lin` into `out`.
+// Every transform that fills a wave's registers takes a register kernel.  8192 rows of line
+// integrals, one stage at a time in LDS against here: W = 90 19 / 9 us, 250 33 / 12 us,
+// 1000 145 / 36 us, 1944 331 / 64 us, 3000 843 / 182 us; 4096 rows of 4096 191 / 42 us, of
+// 8191 1431 / 261 us.
+ctg_status launch_rows(ctg_context* ctx, const void* raw, ctg_pixel_type pixel, const float* lin, const PreArgs& a,
+                       float* out, unsigned* maxabs, hipStream_t st) {
     const FilterTables& ft = ctx->ftab;
-    const T* resp = sizeof(T) == 4 ? (const T*)ft.resp_f.ptr : (const T*)ft.resp_d.ptr;
-    const Cx<T>* tw = sizeof(T) == 4 ? (const Cx<T>*)ft.tw_f.ptr : (const Cx<T>*)ft.tw_d.ptr;
-    const Cx<T>* pad = sizeof(T) == 4 ? (const Cx<T>*)ft.pad_f.ptr : (const Cx<T>*)ft.pad_d.ptr;
-    const size_t lds = (size_t)a.M * sizeof(T) * 2;
-    if (lds > 160 * 1024)
-        return fail(CTG_ERROR_UNSUPPORTED, "detector width %d (transform length %d) exceeds the LDS row buffer", a.W, a.M);
-    if constexpr (sizeof(T) == 4) {
-        if (a.do_filter && a.pow2 && a.W >= 256 && a.W <= 2048) {
-            switch (a.W) {
-                case 256: return launch_rows_fft<256>(raw, pixel, lin, nrows, a, resp, tw, out, maxabs, st);
-                case 512: return launch_rows_fft<512>(raw, pixel, lin, nrows, a, resp, tw, out, maxabs, st);
-                case 1024: return launch_rows_fft<1024>(raw, pixel, lin, nrows, a, resp, tw, out, maxabs, st);
-                default: return launch_rows_fft<2048>(raw, pixel, lin, nrows, a, resp, tw, out, maxabs, st);
-            }
+    CTG_TRY(check_transform(a, 16384));
+    if (a.pow2) {
+        switch (a.W) {
+            case 256: return launch_rows_fft<256>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 512: return launch_rows_fft<512>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 1024: return launch_rows_fft<1024>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 2048: return launch_rows_fft<2048>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 4096: return launch_rows_r2<12, false>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 8192: return launch_rows_r2<13, false>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 16384: return launch_rows_r2<14, false>(ft, raw, pixel, lin, a, out, maxabs, st);
+        }
+    } else {
+        switch (a.M) {
+            case 256: return launch_rows_r2<8, true>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 512: return launch_rows_r2<9, true>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 1024: return launch_rows_r2<10, true>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 2048: return launch_rows_r2<11, true>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 4096: return launch_rows_r2<12, true>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 8192: return launch_rows_r2<13, true>(ft, raw, pixel, lin, a, out, maxabs, st);
+            case 16384: return launch_rows_r2<14, true>(ft, raw, pixel, lin, a, out, maxabs, st);
         }
     }
-    dim3 grid((unsigned)((nrows + 1) / 2));
-    if (raw == nullptr) {
-        hipLaunchKernelGGL((rows_kernel<T, float>), grid, dim3(kRowThreads), lds, st, a, (const float*)nullptr,
-                           lin, resp, tw, pad, out, maxabs);
-    } else if (pixel == CTG_PIXEL_U8) {
-        hipLaunchKernelGGL((rows_kernel<T, uint8_t>), grid, dim3(kRowThreads), lds, st, a, (const uint8_t*)raw,
-                           lin, resp, tw, pad, out, maxabs);
-    } else if (pixel == CTG_PIXEL_U16) {
-        hipLaunchKernelGGL((rows_kernel<T, uint16_t>), grid, dim3(kRowThreads), lds, st, a,
-                           (const uint16_t*)raw, lin, resp, tw, pad, out, maxabs);
-    } else {
-        hipLaunchKernelGGL((rows_kernel<T, float>), grid, dim3(kRowThreads), lds, st, a, (const float*)raw,
-                           lin, resp, tw, pad, out, maxabs);
-    }
+    // transforms of up to 128 points: a few LDS stages, not worth a register form
+    dim3 grid;
+    CTG_TRY(row_blocks((a.nrows + 1) / 2, 1, grid));
+    const dim3 block(kRowThreads);
+    const size_t lds = (size_t)a.M * sizeof(float) * 2;
+#define CTG_K(Tin) rows_kernel<float, Tin>
+    CTG_ROWS_LAUNCH(CTG_K, lin, ft.resp_f.as<float>(), ft.tw_f.as<Cx<float>>(), ft.pad_f.as<Cx<float>>(), out, maxabs);
+#undef CTG_K
     CTG_HIP(hipGetLastError());
     return CTG_OK;
 }
@@ -680,8 +999,7 @@ ctg_status launch_rows(ctg_context* ctx, const void* raw, ctg_pixel_type pixel, 
 
 ctg_status launch_preprocess_rows(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel, int nproj,
                                   float base, ctg_log_form form, ctg_filter filter, float* d_out,
-                                  unsigned* d_maxabs, bool do_log, bool do_weight, bool do_filter,
-                                  hipStream_t st) {
+                                  unsigned* d_maxabs, hipStream_t st) {
     const ctg_geometry& g = ctx->geom;
     PreArgs a{};
     a.W = g.det_width;
@@ -691,13 +1009,24 @@ ctg_status launch_preprocess_rows(ctg_context* ctx, const void* d_raw, ctg_pixel
     a.fcd = g.fcd;
     a.upre = g.u_pre;
     a.vpre = g.v_pre;
-    a.do_log = do_log;
-    a.do_weight = do_weight;
-    a.do_filter = do_filter;
     set_transform(a);
-    if (do_filter) CTG_TRY(ensure_filter_tables(ctx, a.W, filter));
-    return launch_rows<float>(ctx, do_log ? d_raw : nullptr, pixel, do_log ? nullptr : (const float*)d_raw,
-                              a.nrows, a, d_out, d_maxabs, st);
+    CTG_TRY(check_transform(a, 16384));
+    CTG_TRY(ensure_filter_tables(ctx, a.W, filter));
+    return launch_rows(ctx, d_raw, pixel, nullptr, a, d_out, d_maxabs, st);
+}
+
+ctg_status launch_feldkamp_weight(const ctg_geometry& g, float* d_images, int nproj, hipStream_t st) {
+    PreArgs a{};
+    a.W = g.det_width;
+    a.H = g.det_height;
+    a.nrows = (long long)nproj * a.H;
+    a.fcd = g.fcd;
+    a.upre = g.u_pre;
+    a.vpre = g.v_pre;
+    const dim3 grid((unsigned)((a.W + 255) / 256), (unsigned)std::min<long long>(a.nrows, 16384));
+    hipLaunchKernelGGL(weight_kernel, grid, dim3(256), 0, st, a, d_images);
+    CTG_HIP(hipGetLastError());
+    return CTG_OK;
 }
 
 ctg_status launch_filter_rows_only(ctg_context* ctx, const float* d_in, float* d_out, int64_t rows,
@@ -707,10 +1036,10 @@ ctg_status launch_filter_rows_only(ctg_context* ctx, const float* d_in, float* d
     a.W = g.det_width;
     a.H = g.det_height > 0 ? g.det_height : 1;
     a.nrows = rows;
-    a.do_filter = 1;
     set_transform(a);
+    CTG_TRY(check_transform(a, 16384));
     CTG_TRY(ensure_filter_tables(ctx, a.W, filter));
-    return launch_rows<float>(ctx, nullptr, CTG_PIXEL_F32, d_in, rows, a, d_out, nullptr, st);
+    return launch_rows(ctx, nullptr, CTG_PIXEL_F32, d_in, a, d_out, nullptr, st);
 }
 
 ctg_status launch_preprocess_rows_f64(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel, int nproj,
@@ -724,12 +1053,21 @@ ctg_status launch_preprocess_rows_f64(ctg_context* ctx, const void* d_raw, ctg_p
     a.fcd = g.fcd;
     a.upre = g.u_pre;
     a.vpre = g.v_pre;
-    a.do_log = 1;
-    a.do_weight = 1;
-    a.do_filter = 1;
     set_transform(a);
+    CTG_TRY(check_transform(a, 8192));
     CTG_TRY(ensure_filter_tables(ctx, a.W, filter));
-    return launch_rows<double>(ctx, d_raw, pixel, nullptr, a.nrows, a, d_out, nullptr, st);
+    const FilterTables& ft = ctx->ftab;
+    const size_t lds = (size_t)a.M * sizeof(double) * 2;
+    dim3 grid;
+    CTG_TRY(row_blocks((a.nrows + 1) / 2, 1, grid));
+    const dim3 block(kRowThreads);
+    const void* raw = d_raw;
+#define CTG_K(Tin) rows_kernel<double, Tin>
+    CTG_ROWS_LAUNCH(CTG_K, (const float*)nullptr, ft.resp_d.as<double>(), ft.tw_d.as<Cx<double>>(),
+                    ft.pad_d.as<Cx<double>>(), d_out, (unsigned*)nullptr);
+#undef CTG_K
+    CTG_HIP(hipGetLastError());
+    return CTG_OK;
 }
 
 ctg_status launch_layout(const ctg_geometry& g, const float* d_rows, int nproj, ctg_store store,
@@ -741,7 +1079,7 @@ ctg_status launch_layout(const ctg_geometry& g, const float* d_rows, int nproj, 
         const int np = std::min(65535, nproj - p0);
         dim3 grid((unsigned)((g.det_width + 31) / 32), (unsigned)((g.det_height + 31) / 32), (unsigned)np);
         const float* rows = d_rows + (size_t)p0 * img;
-        const unsigned* mx = d_maxabs + p0;
+        const unsigned* mx = d_maxabs ? d_maxabs + p0 : nullptr;  // not read for FP32 entries
         void* out = (char*)d_out + (size_t)p0 * img * ebytes;
         float* sc = d_scales ? d_scales + p0 : nullptr;
         if (store == CTG_STORE_F32) {
@@ -791,11 +1129,13 @@ ctg_status ensure_filter_tables(ctg_context* ctx, int W, int filter) {
     for (int k = 0; k < W; ++k) resp[k] = h[k <= W / 2 ? k : W - k];
     const bool pow2 = ilog2_exact(W) >= 0;
     const int log2M = filter_log2_length(W), M = 1 << log2M;
-    std::vector<double> tw(2 * (size_t)(M / 2 > 0 ? M / 2 : 1));
+    std::vector<double> tw(2 * (size_t)M, 0.0);
     for (int m = 0; m < M / 2; ++m) {
         double ang = 2.0 * kPi * (double)m / (double)M;
         tw[2 * m] = std::cos(ang);
         tw[2 * m + 1] = -std::sin(ang);
+        tw[2 * (m + M / 2)] = -tw[2 * m];
+        tw[2 * (m + M / 2) + 1] = -tw[2 * m + 1];
     }
     std::vector<double> pad(2 * (size_t)M, 0.0);  // complex, interleaved
     if (!pow2) {
@@ -803,7 +1143,11 @@ ctg_status ensure_filter_tables(ctg_context* ctx, int W, int filter) {
         for (int j = 0; j < W; ++j) cosw[j] = std::cos(2.0 * kPi * (double)j / (double)W);
         for (int m = 0; m < W; ++m) {
             double s = 0.0;
-            for (int k = 0; k < W; ++k) s += resp[k] * cosw[(int)(((long long)k * m) % W)];
+            for (int k = 0, j = 0; k < W; ++k) {  // j = k m mod W
+                s += resp[k] * cosw[j];
+                j += m;
+                if (j >= W) j -= W;
+            }
             g[m] = s;
         }
         std::vector<std::complex<double>> z(M);

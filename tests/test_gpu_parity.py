@@ -898,3 +898,37 @@ def test_lds_forms_match_the_global_form(gpu, monkeypatch, store, nz, z0):
         x = np.arange(g.nx)[:, None] - g.x_pre
         y = np.arange(g.ny)[None, :] - g.y_pre
         assert np.all(volume()[x * x + y * y >= g.radius ** 2] == 0.5)
+
+
+@pytest.mark.parametrize("W", [2, 33, 128, 129, 255, 257, 513, 1025, 2047, 2049, 4096, 4097])
+def test_row_filter_transform_lengths_match_oracle(gpu, oracle, W):
+    """The row filter at the ends of each transform length: the padded lengths 256 to 16384
+    at their smallest and largest widths, and the widest powers of two.  An odd row count
+    leaves the last pair without its second row and puts a pair across two images; rows of
+    another image or past the end stay as they are.  FP32 rows against the oracle's FP64
+    ones at the bar of the other widths; FP16 scales from the images' own maxima."""
+    import torch
+    import ct_amd
+    H, P = 3, 3
+    rng = np.random.default_rng(W)
+    g = ct_amd.geometry_grid(W, H, 3.0 * W, 0.0, 4, 4, 4)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    rows = rng.standard_normal((P * H, W)).astype(np.float32)
+    src = torch.from_numpy(rows).cuda()
+    out = torch.full((P * H + 1, W), 7.0, dtype=torch.float32, device="cuda")
+    for filt in ("ramlak", "hann"):
+        ctx.filter_rows(src, out, P * H, filt)
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert rel_rmse(got[:-1], oracle.filter_rows_f64(rows.astype(np.float64), filt)) < 1e-5
+        assert np.all(got[-1] == 7.0)
+    raw = torch.from_numpy(rng.integers(3000, 65535, size=(P, H, W)).astype(np.uint16)).cuda()
+    ent = torch.empty((P, W, H, 4), dtype=torch.float32, device="cuda")
+    f16 = torch.empty((P, W, H, 4), dtype=torch.float16, device="cuda")
+    scales = torch.empty(P, dtype=torch.float32, device="cuda")
+    ctx.preprocess(raw, "u16", P, 1.0, "cpu", "ramlak", "f16", f16, scales)
+    ctx.preprocess(raw, "u16", P, 1.0, "cpu", "ramlak", "f32", ent, None)
+    torch.cuda.synchronize()
+    m = np.abs(ent[..., 0].cpu().numpy()).reshape(P, -1).max(axis=1)
+    np.testing.assert_array_equal(scales.cpu().numpy(), np.ldexp(1.0, np.frexp(m)[1]).astype(np.float32))
