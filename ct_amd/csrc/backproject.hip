@@ -129,28 +129,6 @@ template <int B>
 __device__ inline void lds_dma(dma_rsrc, unsigned, int, void*) {}
 #endif
 
-// acc += w * q, in place.  Written as the two-address instruction because the accumulators
-// meet again after paths that differ per step: with fmaf() the compiler gives the fast
-// path's sums registers of their own and copies all ZPL of them back on every step (one
-// more VALU instruction per update, and 162 VGPRs instead of 127 for FP32 entries, 128
-// instead of 95 for 8-byte entries).
-__device__ inline void fmac(float& acc, float w, float q) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm("v_fmac_f32 %0, %1, %2" : "+v"(acc) : "v"(w), "v"(q));
-#else
-    acc = fmaf(w, q, acc);
-#endif
-}
-
-// A wave-uniform value that the optimiser knows nothing about.
-__device__ inline int opaque_uniform(int v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    v = __builtin_amdgcn_readfirstlane(v);
-    asm volatile("" : "+s"(v));
-#endif
-    return v;
-}
-
 __device__ inline int cvt_flr(float x) {
     int r;
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));

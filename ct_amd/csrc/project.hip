@@ -5,8 +5,9 @@
 // voxel-driven backprojection of Ct/CtVolume.cpp:979-1039 term by term: every voxel that
 // the backprojection would read through taps (u0,v0),(u0+1,v0),(u0,v0+1),(u0+1,v0+1) with
 // weight U^2 and bilinear weights instead adds U^2 * f * weight into those pixels, under
-// the same cylinder and window masks.  It is computed as a gather (fp_gather_kernel):
-// each detector pixel sums the taps that land on it.
+// the same cylinder and window masks.  A workgroup owns a pixel column of one projection and
+// collects the voxel columns that land on it: fp_rows_kernel, or fp_gather_kernel where the
+// geometry rules that one out.
 #include "ctg_internal.h"
 
 #include <algorithm>
@@ -375,79 +376,129 @@ __global__ __launch_bounds__(kGThreads) void fp_gather_kernel(FpArgs a, const fl
     }
 }
 
-// -------------------------------------------------------- entry-space projector
+// ------------------------------------------------------------ row-run projector
 //
-// The backprojection evaluates a voxel's value from ONE coefficient entry (A, dU, dV, dUV)
-// at (u0, v0): val = A + fu dU + fv (dV + fu dUV), weighted by w = U^2.  Its transpose
-// therefore adds (w x, w x fu, w x fv, w x fu fv) into one entry gradient per (voxel,
-// projection), and the transpose of the layout (A = q00, dU = q10 - q00, dV = q01 - q00,
-// dUV = q11 - q10 - q01 + q00) turns entry gradients into pixels:
-//     q00 += gA - gdU - gdV + gdUV,  q01 += gdV - gdUV,  q10 += gdU - gdUV,  q11 += gdUV.
-// Every voxel is visited once per projection (by the workgroup of its own u0), with one
-// LDS read and one write of 16 bytes, instead of twice with two row taps each.
+// Every voxel adds its two row taps to pixel columns c = u0 and c + 1, with weights
+// w (1 - fu) and w fu, w = U^2.  The voxel columns that feed one c lie along a ray, and from
+// one to the next the detector row of a given slice moves by (z + h) dU, a small part of a
+// pixel.  So a lane keeps one slice (per chunk of 64) and walks the candidates in depth
+// order: over a run of candidates whose rows of the window's outermost slice stay within one
+// pixel, its taps fall on three rows R, R + 1, R + 2, whose six sums (three rows, two pixel
+// columns) stay in registers.  Each row's weight is the hat 1 - |vIndex - row| clamped at 0,
+// from the backprojection's own vIndex (exactly 1 - fv and fv on the two rows of a tap).
+// Only the end of a run touches LDS.
 //
-// fp_entry_kernel<G>: a workgroup owns entry column c of one projection within one
+// fp_rows_kernel<G>: a workgroup owns pixel column c of one projection within one
 // window of 64 G slices (grid z [wz0, wz0 + 64 G), wz0 - zrb a multiple of 64).
 //  - Candidates are the voxel columns with u0 == c that pass the cylinder and u window
 //    tests, between the two fan rays through u = c - 0.05 and u = c + 1.05 (plus a
-//    0.01-voxel margin).  The lanes test the wedge's (depth, lateral) slots and compact
-//    the survivors (column, U, fu) into LDS; then one lane per survivor settles its z
-//    interval of the v-window test (exactly, with the backprojection's expression),
-//    intersected with the slab and the window, and writes the final record.
-//  - A candidate is one item of G chunks of 64 slices: lane l takes slices
-//    wz0 + 64 k + l, whose row anchor is (l & 32) slices past the chunk start and whose
-//    offset from it is l & 31, as in the backprojection.  The voxels come through a
-//    buffer resource covering the candidate's interval (zero outside it, which is the
-//    window, slab and v-window mask).
-//  - Each wave accumulates into two private copies of the window's entry rows (even and
-//    odd lanes).  Lanes two slices apart have rows at least 2U - 1e-3 > 1 apart (U > 2/3
-//    whenever the cylinder radius is below half the FCD, checked on the host), and chunks
-//    are 64 slices apart, so no two lanes of one copy touch one entry in an instruction
-//    and the read-modify-writes need no atomics.  The host bounds the rows that any slice
-//    of the window can reach for every candidate U and height, [rbase, rbase + span), so
-//    lanes outside their interval (adding zero) stay inside their own copy.
-//  - At the end the eight copies are summed in a fixed order and turned into pixel
-//    partials: own column c (q00, q01) and the next column (q10, q11), added into the
-//    workgroup's own float2 column ps[p][c][*] of a column-major buffer.  Windows run one
-//    after another on one stream; fp_finish_kernel then adds ps[p][c][r].x +
+//    0.01-voxel margin).  Each lane tests the lateral slots of one depth step and the
+//    survivors (column, U, fu) go compacted into LDS in depth order; then one lane each
+//    settles its z interval of the v-window test (exactly, with the backprojection's
+//    expression), intersected with the slab and the window, and writes the final record.
+//  - Each wave walks a quarter of the list.  A candidate is one item of G chunks of 64
+//    slices: lane l takes slices wz0 + 64 k + l, whose row anchor is (l & 32) slices past
+//    the chunk start and whose offset from it is l & 31, as in the backprojection.  The
+//    voxels come through a buffer resource covering the candidate's interval (zero outside
+//    it, which is the window, slab and v-window mask).
+//  - A run is the longest of 16, 8, 4, 2 or 1 next candidates whose magnifications span
+//    [Umin, Umax] with (Umax - Umin) |z + h| <= 0.98 over the window; R is the row below the
+//    smaller of vIndex(Umin) and vIndex(Umax), less 0.002 for the rounding of either.
+//  - At the end of a run each lane adds its sums into its wave's rows in LDS, kept in two
+//    copies (even and odd lanes): lanes two slices apart have rows at least 2U - 1e-3 > 1
+//    apart (U > 2/3 whenever the cylinder radius is below half the FCD, checked on the
+//    host), and chunks are 64 slices apart, so no two lanes of one copy touch one row in an
+//    instruction and the read-modify-writes need no atomics.  The host bounds the rows that
+//    any slice of the window can reach for every candidate U and height, [rbase, rbase +
+//    span), so lanes outside their interval (adding zero) stay inside their own copy.
+//  - At the end the eight copies are summed in a fixed order and added into the workgroup's
+//    own float2 column ps[p][c][*] of a column-major buffer (own column c, next column).
+//    Windows run one after another on one stream; fp_finish_kernel then adds ps[p][c][r].x +
 //    ps[p][c-1][r].y into the row-major image.
 // The order of every addition is fixed: the result does not depend on scheduling.
-constexpr int kESlots = 256;
-constexpr int kEMaxSpan = 256;  // entry rows per copy
+//
+// What bounds it: VALU issue.  At 512^3 x 360 projections of 512 x 512 (5.9e8 wave-updates
+// inside the cylinder) it issues 1.24e10 wave instructions, 21 per update of which 13 are the
+// update itself: 12.6 of the 18.3 ms at the measured 2.5 cycles each.  A form that added each
+// voxel's two rows to LDS as it came (one 16-byte read-modify-write per update, LDS-bound)
+// took 24.8 ms; with its column-by-column order 1 % of the voxel reads hit the L2, with
+// fp_item's units 53 %.
+constexpr int kJ = 3;  // lateral slots per lane and round
+constexpr int kESlots = (kJ + 1) * kGThreads;  // a round always fits behind 256 candidates
+constexpr int kEMaxSpan = 512;  // rows per copy
+constexpr int kAside = 1 << 30;  // mark in a candidate's z interval word (2 kFpZBits bits in use)
 
 struct FpWin {
     int wz0;     // first grid slice of the window (a multiple of 64 past the run base)
-    int rbase;   // first entry row any voxel of the window can reach
+    int rbase;   // first row any voxel of the window can reach
     int span;    // rows per copy
-    int stride;  // entries between copies: span rounded up to 8 mod 16 (see the kernel)
+    int stride;  // rows between copies
 };
 
-__device__ inline int flr_i32(float x) {
-    int r;
-    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
-    return r;
+// min and max over aligned groups of lanes, doubled by one step: the lane 1, 2, 7 - l (of
+// eight) or 15 - l (of sixteen) away.  On the bits of positive floats, which order like
+// integers (no canonicalisation).
+template <int CTRL>
+__device__ inline void dpp_minmax(int& mn, int& mx) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    mn = min(mn, __builtin_amdgcn_mov_dpp(mn, CTRL, 0xf, 0xf, true));
+    mx = max(mx, __builtin_amdgcn_mov_dpp(mx, CTRL, 0xf, 0xf, true));
+#endif
+}
+// A scalar that the optimiser knows nothing about.
+__device__ inline int opaque_scalar(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(v));
+#endif
+    return v;
+}
+// x = v, keeping x in its register (see fmac)
+__device__ inline void set_in_place(float& x, float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_mov_b32 %0, %1" : "+v"(x) : "v"(v));
+#else
+    x = v;
+#endif
+}
+__device__ inline float first_lane(int x) { return __int_as_float(__builtin_amdgcn_readfirstlane(x)); }
+
+// The workgroups that an XCD runs together (dispatch is round-robin over 8 XCDs) should read
+// the same voxels: a voxel column is read once per projection, by the column it falls on, and
+// for neighbouring projections by neighbouring columns.  So the work is cut into units of
+// kPBlock projections x kCBlock columns, dealt to the XCDs in turn (columns vary slowest, so
+// that short rays at the edges spread over the XCDs), and inside a unit the projections vary
+// fastest.  Units of the rounded-up grid beyond it exit.
+constexpr int kPBlock = 4, kCBlock = 64;
+__host__ __device__ inline unsigned fp_units(int W, int nproj) {
+    return (unsigned)((W + kCBlock - 1) / kCBlock) * (unsigned)((nproj + kPBlock - 1) / kPBlock);
+}
+__device__ inline bool fp_item(const FpArgs& a, int& c, int& p) {
+    constexpr unsigned per = kPBlock * kCBlock;
+    const unsigned xcd = blockIdx.x & 7u, k = blockIdx.x >> 3;
+    const unsigned unit = (k / per) * 8u + xcd, r = k % per;
+    const unsigned npb = (unsigned)((a.nproj + kPBlock - 1) / kPBlock);
+    const unsigned cb = unit / npb, pb = unit - cb * npb;
+    c = (int)(cb * kCBlock + r / kPBlock);
+    p = (int)(pb * kPBlock + r % kPBlock);
+    return c < a.W && p < a.nproj;
 }
 
 template <int G>
-__global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win, const float4* __restrict__ pp,
-                                                             const float* __restrict__ vol,
-                                                             float2* __restrict__ ps) {
+__global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win, const float4* __restrict__ pp,
+                                                            const float* __restrict__ vol,
+                                                            float2* __restrict__ ps) {
     // column, U, w fu and the z interval relative to the run base (w = U^2 is recomputed
     // from U): one 16-byte LDS read per item
     __shared__ int4 slots[kESlots];
     __shared__ int wave_cnt[kGWaves];
-    // [wave][parity][row], copies `stride` entries apart (a multiple of 16 entries unless
-    // the host is told otherwise).  On gfx950 a ds_write_b128 occupies the LDS for about
-    // 13.5 cycles per wave instruction whatever its lane mask and a conflict-free
-    // ds_read_b128 about 4 (16 lanes per cycle); of the copy offsets 0, 2, 5, 6, 8 and 13
-    // entries modulo 16, 0 was the fastest on the 512^3 x 360 workload.
-    extern __shared__ float4 acc_lds[];
-    const int c = blockIdx.x;
-    const int p = blockIdx.y;
+    // [wave][parity][row]: (own column, next column)
+    extern __shared__ float2 acc_lds[];
+    int c, p;
+    if (!fp_item(a, c, p)) return;
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int span = win.span, stride = win.stride;
-    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) acc_lds[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) acc_lds[i] = make_float2(0.0f, 0.0f);
 
     const float4 g = pp[p];
     const float sn = g.x, cs = g.y, h = g.z;
@@ -483,7 +534,6 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
         return fabsf((ow - So) * (k1 - k0));
     };
     const int jm = (int)fmaxf(width(o_lo), width(o_hi)) + 2;
-    const int nslot = (o_hi - o_lo + 1) * jm;
 
     // per lane and chunk: world z of the slice's row anchor plus the height (the
     // backprojection's zwa + h), and the slice's offset from the anchor
@@ -491,62 +541,77 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
 #pragma unroll
     for (int k = 0; k < G; ++k) zh[k] = ((float)(win.wz0 + 64 * k + (lane & 32)) - a.zpre) + h;
     const float lane_k = (float)(lane & 31);
-    // LDS byte address of entry row v0 in this lane's copy: v0 * 16 + lane_base
-    int lane_base = (wv * 2 + (lane & 1)) * stride * 16 - win.rbase * 16;
-    // opaque to the optimiser, so that v0 * 16 + lane_base stays one shift-and-add per
-    // voxel instead of being re-associated around rbase
-    asm volatile("" : "+v"(lane_base));
-    char* acc_bytes = reinterpret_cast<char*>(acc_lds);
-    const float* colbase = vol + (zrb - a.z0);
-    const int zc = win.wz0 - zrb;  // the window's first slice relative to the run base
-    const unsigned lane4 = (unsigned)lane * (unsigned)sizeof(float);
+    // the window's largest |z + h|
+    const float zm = fmaxf(fabsf(((float)win.wz0 - a.zpre) + h), fabsf(((float)(win.wz0 + 64 * G - 1) - a.zpre) + h));
+    float2* const my_rows = acc_lds + (wv * 2 + (lane & 1)) * stride - win.rbase;
+    // A candidate's voxels are read from the window's first slice inside the slab, zs (relative
+    // to the run base).  Lanes of chunk 0 before it wrap to a huge offset, past every
+    // resource; the later chunks' offsets are one register plus immediates.
+    const int zs = max(wlo - zrb, win.wz0 - zrb);
+    const float* colbase = vol + (zrb - a.z0) + zs;
+    const unsigned off0 = (unsigned)((lane - (zs - (win.wz0 - zrb))) * (int)sizeof(float));
+    const unsigned off1 = off0 + 256u;
     __syncthreads();
 
+    // Rounds: 256 depth steps (one per lane) times kJ lateral slots, all laterals of a block of
+    // depth steps before the next block.
     int ncand = 0;
-    for (int sbase = 0; sbase < nslot && wlo <= whi; sbase += kGThreads) {
-        // fill, step 1: the cheap tests for 256 slots, survivors compacted (ballot prefix
-        // within each wave, wave totals through LDS)
-        const int sidx = sbase + tid;
-        int4 rec = make_int4(-1, 0, 0, 0);
-        if (sidx < nslot) {
-            const int oi = sidx / jm, jj = sidx - oi * jm;
-            const int o = o_lo + oi;
+    for (int ob = o_lo, jb = 0; ob <= o_hi && wlo <= whi;) {
+        // fill, step 1: the cheap tests of this lane's slots; survivors are compacted in
+        // depth order (ballot prefix within each wave, wave totals through LDS)
+        int4 rec[kJ];
+        int cnt = 0;  // survivors of this lane: rec[0 .. cnt)
+        const int o = ob + tid;
+        if (o <= o_hi) {
             int jl, jh;
             jrange(o, jl, jh);
-            const int j = jl + jj;
-            if (j <= jh) {
+#pragma unroll
+            for (int jj = 0; jj < kJ; ++jj) {
+                const int j = jl + jb + jj;
+                if (j > jh) continue;
                 const int xi = xmajor ? o : j, yi = xmajor ? j : o;
                 // per-voxel arithmetic identical to the backprojection's
                 const float x = (float)xi - a.xpre, y = (float)yi - a.ypre;
-                if (x * x + y * y < a.r2) {
-                    float t = (-1.0f) * x * g.x + y * g.y;
-                    t += a.uoff;
-                    const float s = x * g.y + y * g.x;
-                    const float U = cone_magnification(a.fcd, s);
-                    const float u = t * U;
-                    if (u >= a.ulo && u <= a.uhi) {
-                        const float uIdx = u + a.upre;
-                        const int u0 = (int)uIdx;
-                        if (u0 == c) rec = make_int4(xi * a.ny + yi, __float_as_int(U), __float_as_int(uIdx - (float)u0), 0);
-                    }
-                }
+                if (!(x * x + y * y < a.r2)) continue;
+                float t = (-1.0f) * x * g.x + y * g.y;
+                t += a.uoff;
+                const float s = x * g.y + y * g.x;
+                const float U = cone_magnification(a.fcd, s);
+                const float u = t * U;
+                if (!(u >= a.ulo && u <= a.uhi)) continue;
+                const float uIdx = u + a.upre;
+                const int u0 = (int)uIdx;
+                if (u0 != c) continue;
+                const int4 r = make_int4(xi * a.ny + yi, __float_as_int(U), __float_as_int(uIdx - (float)u0), 0);
+#pragma unroll
+                for (int q = 0; q < kJ; ++q)
+                    if (q == cnt) rec[q] = r;
+                ++cnt;
             }
         }
+        const bool last_round = jb + kJ >= jm && ob + kGThreads > o_hi;
+        if (jb + kJ >= jm) {
+            jb = 0;
+            ob += kGThreads;
+        } else {
+            jb += kJ;
+        }
         {
-            const unsigned long long m = __ballot(rec.x >= 0);
-            const int below = __popcll(m & ((1ull << lane) - 1ull));
-            if (lane == 0) wave_cnt[wv] = __popcll(m);
+            static_assert(kJ <= 3, "two ballots count the survivors of a lane");
+            const unsigned long long m1 = __ballot(cnt & 1), m2 = __ballot(cnt & 2), lt = (1ull << lane) - 1ull;
+            if (lane == 0) wave_cnt[wv] = __popcll(m1) + 2 * __popcll(m2);
             __syncthreads();
-            int base = ncand;
+            int base = ncand + __popcll(m1 & lt) + 2 * __popcll(m2 & lt);
             for (int w = 0; w < wv; ++w) base += wave_cnt[w];
             int total = 0;
             for (int w = 0; w < kGWaves; ++w) total += wave_cnt[w];
-            if (rec.x >= 0) slots[base + below] = rec;
+#pragma unroll
+            for (int q = 0; q < kJ; ++q)
+                if (q < cnt) slots[base + q] = rec[q];
             __syncthreads();  // the slots are complete; wave_cnt is rewritten below
             // fill, step 2: one lane per new survivor settles its z interval and writes its
             // final record (candidates with an empty interval keep an empty one)
-            const int ci = ncand + tid;
-            if (tid < total) {
+            for (int ci = ncand + tid; ci < ncand + total; ci += kGThreads) {
                 const int4 r = slots[ci];
                 const float U = __int_as_float(r.y), fu = __int_as_float(r.z);
                 auto v_of = [&](int zi) { const float zk = (float)zi - a.zpre; return (zk + h) * U; };
@@ -582,10 +647,13 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
             __syncthreads();  // records complete; wave_cnt free again
         }
         // walk when another fill round might not fit, and after the last round
-        if (ncand > kESlots - kGThreads || sbase + kGThreads >= nslot) {
+        if (ncand > kESlots - kJ * kGThreads || last_round) {
+            // this wave's part of the list
+            const int per_wave = (ncand + kGWaves - 1) / kGWaves;
+            const int c_begin = min(wv * per_wave, ncand), c_end = min(c_begin + per_wave, ncand);
             struct Item {
                 vbuf rs;
-                float U, w, wfu;
+                float U, wo, ws;  // weights of the own and the next column
                 int lo;
             };
             // past the last candidate an item still issues its loads, over an empty
@@ -595,99 +663,210 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
                 const int zb = __builtin_amdgcn_readfirstlane(r.w);
                 Item it;
                 it.lo = zb & ((1 << kFpZBits) - 1);
-                const int hi1 = (zb >> kFpZBits) & ((1 << kFpZBits) - 1);  // one past the last slice
-                it.rs = make_vbuf(colbase + (size_t)__builtin_amdgcn_readfirstlane(r.x) * a.zstride + it.lo,
-                                  valid ? (hi1 - it.lo) * (int)sizeof(float) : 0);
+                const int hi1 = zb >> kFpZBits;  // one past the last slice
+                it.rs = make_vbuf(colbase + (size_t)__builtin_amdgcn_readfirstlane(r.x) * a.zstride,
+                                  valid && hi1 > it.lo ? (hi1 - zs) * (int)sizeof(float) : 0);
                 // the same value in every lane: kept in vector registers (operands of the
                 // per-voxel arithmetic), where moving them to scalars would cost a
                 // readfirstlane each
                 it.U = __int_as_float(r.y);
-                it.w = it.U * it.U;  // as in the fill: the weight is U^2
-                it.wfu = __int_as_float(r.z);
+                it.ws = __int_as_float(r.z);
+                it.wo = it.U * it.U - it.ws;
                 return it;
             };
-            // Candidate ci goes to wave ci mod 4.  Three named slots keep the next two
-            // candidates' voxels in flight while one is accumulated.
+            // Three named slots keep the next two candidates' voxels in flight while one is
+            // accumulated.
             struct Slot { Item it; float x[G]; };
-            int ci_f = wv;
-            auto next = [&](Slot& sl) -> bool {
-                const bool valid = ci_f < ncand;
-                sl.it = item_of(ci_f, valid);
+            int ci_f = c_begin;
+            auto next = [&](Slot& sl) {
+                sl.it = item_of(ci_f, ci_f < c_end);
 #pragma unroll
                 for (int k = 0; k < G; ++k)
-                    sl.x[k] = vbuf_load(sl.it.rs, vadd_sv((zc + 64 * k - sl.it.lo) * (int)sizeof(float), lane4));
-                ci_f += kGWaves;
+                    sl.x[k] = vbuf_load(sl.it.rs, k == 0 ? off0 : off1 + 256u * (unsigned)(k - 1));
+                ++ci_f;
                 __builtin_amdgcn_sched_barrier(0);  // keep the slots' loads in walk order
-                return valid;
             };
-            // The G chunks of one item touch distinct entries of each copy (same-parity
-            // lanes of the item are two or more slices apart, so their rows differ), so
-            // all G reads are issued before the first write: one LDS round trip per item
-            // instead of one per chunk.
-            auto process = [&](const Slot& sl) {
-                float4* e[G];
-                float4 v[G];
-                float fv[G];
+            // sums over a run of x, x e and x max(e, 0), e = vIndex - (R + 1), for the own and
+            // the next column: row R takes S2 - S1, row R + 2 S2, row R + 1 the rest of S0
+            float acc[G][6];
+            float row1[G];   // R + 1
+            float2* at[G];   // row R in this lane's copy
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                row1[k] = (float)(win.rbase + 1);
+                at[k] = my_rows + win.rbase;
+#pragma unroll
+                for (int j = 0; j < 6; ++j) acc[k][j] = 0.0f;
+            }
+            // The current run, and whether a run of this part was set aside.  Sums that are not
+            // finite (an infinite or NaN voxel) would spread over all three rows: such a run
+            // adds nothing here and its candidates are marked for the walk below, which adds
+            // each one's two taps by themselves.
+            int run_at = c_begin, run_n = 0, aside = 0;
+            auto flush = [&]() {
+                float t = 0.0f;
+#pragma unroll
+                for (int k = 0; k < G; ++k) t += acc[k][0] + acc[k][1];
+                if (__ballot(!(fabsf(t) <= 3.402823466e38f))) {
+                    if (lane < run_n && run_at + lane < c_end) slots[run_at + lane].w |= kAside;
+                    aside = 1;
+#pragma unroll
+                    for (int k = 0; k < G; ++k)
+#pragma unroll
+                        for (int j = 0; j < 6; ++j) set_in_place(acc[k][j], 0.0f);
+                }
+#pragma unroll
+                for (int k = 0; k < G; ++k)
+#pragma unroll
+                    for (int c2 = 0; c2 < 2; ++c2) {
+                        const float s2 = acc[k][4 + c2], r0 = s2 - acc[k][2 + c2];
+                        set_in_place(acc[k][2 + c2], acc[k][c2] - (r0 + s2));
+                        set_in_place(acc[k][c2], r0);
+                    }
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    // The G rows of a lane and those of the other lanes are distinct; row j + 1
+                    // of one lane may be row j of another, so the compiler must keep the
+                    // three steps apart (a wave's LDS operations then run in order).
+                    float2 o[G];
+#pragma unroll
+                    for (int k = 0; k < G; ++k) o[k] = at[k][j];
+#pragma unroll
+                    for (int k = 0; k < G; ++k) {
+                        o[k].x += acc[k][2 * j];
+                        o[k].y += acc[k][2 * j + 1];
+                        at[k][j] = o[k];
+                        set_in_place(acc[k][2 * j], 0.0f);
+                        set_in_place(acc[k][2 * j + 1], 0.0f);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                }
+            };
+            // starts a run at candidate ci; returns its length
+            auto start_run = [&](int ci) -> int {
+                const int U = slots[min(ci + (lane & 15), c_end - 1)].y;
+                int mn = U, mx = U, n = 1;
+                float umin = first_lane(U), umax = umin;
+                auto grow = [&](int m) {
+                    // lane 0 holds the extremes of the first m candidates
+                    const float lo = first_lane(mn), hi = first_lane(mx);
+                    if (n * 2 == m && (hi - lo) * zm <= 0.98f) {
+                        n = m;
+                        umin = lo;
+                        umax = hi;
+                    }
+                };
+                dpp_minmax<0xB1>(mn, mx);  // quad_perm 1,0,3,2
+                grow(2);
+                dpp_minmax<0x4E>(mn, mx);  // quad_perm 2,3,0,1
+                grow(4);
+                dpp_minmax<0x141>(mn, mx);  // row_half_mirror
+                grow(8);
+                dpp_minmax<0x140>(mn, mx);  // row_mirror
+                grow(16);
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const float v1 = det_row_index(lane_k, umin, fmaf(-zh[k], umin, a.vpre));
+                    const float v2 = det_row_index(lane_k, umax, fmaf(-zh[k], umax, a.vpre));
+                    const float R = floorf(fminf(v1, v2) - 0.002f);
+                    set_in_place(row1[k], R + 1.0f);
+                    at[k] = my_rows + (int)R;
+                }
+                return n;
+            };
+            int ci_p = c_begin, left = 0;
+            auto process = [&](Slot& sl) {
+                if (opaque_scalar(left) == 0) {
+                    flush();  // before the first run: zeros
+                    left = start_run(ci_p);
+                    run_at = ci_p;
+                    run_n = left;
+                }
+                --left;
+                ++ci_p;
+                if (sl.it.lo > zs) {
+                    // the v window starts inside the window: slices before it are masked
+                    // here (those past its end are past the resource's)
+#pragma unroll
+                    for (int k = 0; k < G; ++k)
+                        if (win.wz0 - zrb + 64 * k + lane < sl.it.lo) sl.x[k] = 0.0f;
+                }
 #pragma unroll
                 for (int k = 0; k < G; ++k) {
                     const float vA = fmaf(-zh[k], sl.it.U, a.vpre);  // det_row_anchor(zwa, h, U, vpre)
-                    const float vI = det_row_index(lane_k, sl.it.U, vA);
-                    const int v0 = flr_i32(vI);
-                    fv[k] = __builtin_amdgcn_fractf(vI);
-                    e[k] = reinterpret_cast<float4*>(acc_bytes + (v0 * 16 + lane_base));
-                    v[k] = *e[k];
-                }
-#pragma unroll
-                for (int k = 0; k < G; ++k) {
-                    const float t = sl.it.w * sl.x[k], tu = sl.it.wfu * sl.x[k];
-                    v[k].x += t;
-                    v[k].y += tu;
-                    v[k].z = fmaf(t, fv[k], v[k].z);
-                    v[k].w = fmaf(tu, fv[k], v[k].w);
-                    *e[k] = v[k];
+                    const float e = det_row_index(lane_k, sl.it.U, vA) - row1[k];
+                    const float xo = sl.it.wo * sl.x[k], xs = sl.it.ws * sl.x[k], h2 = fmaxf(e, 0.0f);
+                    acc[k][0] += xo;
+                    acc[k][1] += xs;
+                    fmac(acc[k][2], xo, e);
+                    fmac(acc[k][3], xs, e);
+                    fmac(acc[k][4], xo, h2);
+                    fmac(acc[k][5], xs, h2);
                 }
             };
-            Slot sa, sb, sc;
-            bool ha = next(sa), hb = next(sb), hc = next(sc);
-            while (ha) {
-                process(sa);
-                ha = next(sa);
-                if (!hb) break;
-                process(sb);
-                hb = next(sb);
-                if (!hc) break;
-                process(sc);
-                hc = next(sc);
+            // Three items at a time, whatever is left (items past the last add zeros): with
+            // a way out between them the compiler no longer knows which loads are older
+            // and waits for all of them at each item.
+            if (c_begin < c_end) {
+                Slot sa, sb, sc;
+                next(sa);
+                next(sb);
+                next(sc);
+                do {
+                    process(sa);
+                    next(sa);
+                    process(sb);
+                    next(sb);
+                    process(sc);
+                    next(sc);
+                } while (ci_p < c_end);
+                flush();
+                if (opaque_scalar(aside)) {
+                    for (int ci = c_begin; ci < c_end; ++ci) {
+                        const int4 r = slots[ci];
+                        const int zb = __builtin_amdgcn_readfirstlane(r.w);
+                        if (!(zb & kAside)) continue;
+                        const int lo = zb & ((1 << kFpZBits) - 1), hi1 = (zb & ~kAside) >> kFpZBits;
+                        const float U = __int_as_float(r.y), ws = __int_as_float(r.z), wo = U * U - ws;
+                        for (int k = 0; k < G; ++k) {
+                            const int z = win.wz0 - zrb + 64 * k + lane;
+                            const float zk = ((float)(win.wz0 + 64 * k + (lane & 32)) - a.zpre) + h;
+                            const float vI = det_row_index(lane_k, U, fmaf(-zk, U, a.vpre)), v0 = floorf(vI);
+                            const bool on = z >= lo && z < hi1;
+                            const float x = on ? colbase[(size_t)r.x * a.zstride + (z - zs)] : 0.0f;
+                            const float fv = vI - v0;
+                            float2* const at0 = my_rows + (int)v0;
+                            for (int j = 0; j < 2; ++j) {
+                                const float wv2 = j ? fv : 1.0f - fv;
+                                float2 o = at0[j];
+                                if (on) {
+                                    o.x += wo * wv2 * x;
+                                    o.y += ws * wv2 * x;
+                                    at0[j] = o;
+                                }
+                                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                                __builtin_amdgcn_wave_barrier();
+                            }
+                        }
+                    }
+                }
             }
             ncand = 0;
             __syncthreads();  // every wave is done with the slots
         }
     }
-    // sum the eight copies per entry row (waves in order, even before odd) and turn the
-    // entry gradients into pixel partials: own column (q00 at row v, q01 at v + 1) and
-    // the next column (q10 at v, q11 at v + 1); pixel row rbase + r takes entry rows r
-    // and r - 1
+    // sum the eight copies per row (waves in order, even before odd)
     float2* col = ps + ((size_t)p * a.W + c) * a.H;
-    auto entry = [&](int r) {
-        float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (r >= 0 && r < span) {
-            for (int w = 0; w < kGWaves; ++w)
-                for (int par = 0; par < 2; ++par) {
-                    const float4 e = acc_lds[(w * 2 + par) * stride + r];
-                    sum.x += e.x; sum.y += e.y; sum.z += e.z; sum.w += e.w;
-                }
-        }
-        return sum;
-    };
-    for (int r = tid; r <= span; r += kGThreads) {
+    for (int r = tid; r < span; r += kGThreads) {
         const int row = win.rbase + r;
         if (row < 0 || row >= a.H) continue;
-        const float4 e0 = entry(r), e1 = entry(r - 1);  // entries at rows v = row and v = row - 1
-        const float own = ((e0.x - e0.y) - e0.z + e0.w) + (e1.z - e1.w);
-        const float side = (e0.y - e0.w) + e1.w;
         float2 o = col[row];
-        o.x += own;
-        o.y += side;
+        for (int w = 0; w < 2 * kGWaves; ++w) {
+            const float2 e = acc_lds[w * stride + r];
+            o.x += e.x;
+            o.y += e.y;
+        }
         col[row] = o;
     }
 }
@@ -840,18 +1019,19 @@ __global__ __launch_bounds__(256) void copy_swap_kernel(const float* __restrict_
 
 namespace {
 
-// Entry rows that the slices [wz0, wz0 + nsl) of any voxel column can reach: vIndex =
+// Rows that the slices [wz0, wz0 + nsl) of any voxel column can reach: vIndex =
 // vPre - (z + h) U over every world z of the window, every height of the launch's
-// projections and every magnification of the cylinder, with two rows of margin for the
-// rounding of the kernel's anchored expression.
+// projections and every magnification of the cylinder.  A run's first row lies up to two
+// below and its last up to two above the rows that its voxels fall in; one more on either
+// side covers the rounding of the kernel's anchored expression.
 void window_rows(const ctg_geometry& g, double hmin, double hmax, double Umin, double Umax, int wz0, int nsl,
                  int& rbase, int& span) {
     const double ylo = (double)wz0 - g.z_pre + hmin, yhi = (double)(wz0 + nsl - 1) - g.z_pre + hmax;
     const double c[4] = {ylo * Umin, ylo * Umax, yhi * Umin, yhi * Umax};
     const double mn = std::min(std::min(c[0], c[1]), std::min(c[2], c[3]));
     const double mx = std::max(std::max(c[0], c[1]), std::max(c[2], c[3]));
-    rbase = (int)std::floor(g.v_pre - mx) - 2;
-    const int rtop = (int)std::floor(g.v_pre - mn) + 2;
+    rbase = (int)std::floor(g.v_pre - mx) - 3;
+    const int rtop = (int)std::floor(g.v_pre - mn) + 3;
     span = rtop - rbase + 1;
 }
 
@@ -883,7 +1063,7 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
     dim3 grid((unsigned)a.W, (unsigned)nproj);
     if (grid.y > 65535u) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
 
-    // Entry-space form (fp_entry_kernel) when the windows' rows fit the LDS copies: it
+    // Row-run form (fp_rows_kernel) when the windows' rows fit the LDS copies: it
     // needs U > 2/3 (radius below half the FCD) and host parameters for the row bounds.
     int G = 0;
     double hmin = 0.0, hmax = 0.0;
@@ -898,20 +1078,20 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
         }
         const int zrb = z0 & ~(kRowAnchor - 1);
         // CTG_FP_MAXSPAN overrides the rows per copy the window height may need (tuning;
-        // at most 400, which keeps the eight copies within 54 KB of LDS)
+        // at most 800, which keeps the eight copies within 52 KB of LDS)
         int max_span = kEMaxSpan;
-        if (const char* e = std::getenv("CTG_FP_MAXSPAN")) max_span = std::max(16, std::min(400, std::atoi(e)));
-        for (int cand : {4, 2, 1}) {
+        if (const char* e = std::getenv("CTG_FP_MAXSPAN")) max_span = std::max(16, std::min(800, std::atoi(e)));
+        // as few windows as chunks of 64 slices allow at four per window, equally deep
+        const int nch = (z0 + nz - zrb + 63) / 64;
+        const int deep = (nch + (nch + 3) / 4 - 1) / ((nch + 3) / 4);
+        for (int cand = deep; cand >= 1 && G == 0; --cand) {
             bool fits = true;
             for (int w0 = zrb; w0 < z0 + nz && fits; w0 += 64 * cand) {
                 int rb, sp;
                 window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * cand, rb, sp);
                 fits = sp <= max_span;
             }
-            if (fits) {
-                G = cand;
-                break;
-            }
+            if (fits) G = cand;
         }
     }
     if (G > 0 && nz <= kFpMaxSlab) {
@@ -920,19 +1100,19 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
         float2* ps = work.as<float2>();
         CTG_TRY(fill_u32(ps, 0u, cells * 2, st));
         const int zrb = z0 & ~(kRowAnchor - 1);
+        const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj) + 7) / 8) * 8 * kPBlock * kCBlock;
+        if (blocks > 0x7fffffffull) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
+        const dim3 rgrid((unsigned)blocks);
         for (int w0 = zrb; w0 < z0 + nz; w0 += 64 * G) {
             FpWin win{};
             win.wz0 = w0;
             window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * G, win.rbase, win.span);
-            // copies a multiple of 16 entries apart (CTG_FP_SPAD=r sets the remainder
-            // modulo 16 instead, tuning)
-            int pad = 0;
-            if (const char* e = std::getenv("CTG_FP_SPAD")) pad = std::atoi(e) & 15;
-            win.stride = win.span + ((pad - win.span) & 15);
-            const size_t lds = sizeof(float4) * 2 * kGWaves * (size_t)win.stride;
-            if (G == 4) hipLaunchKernelGGL(fp_entry_kernel<4>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-            else if (G == 2) hipLaunchKernelGGL(fp_entry_kernel<2>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-            else hipLaunchKernelGGL(fp_entry_kernel<1>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
+            win.stride = (win.span + 1) & ~1;
+            const size_t lds = sizeof(float2) * 2 * kGWaves * (size_t)win.stride;
+            if (G == 4) hipLaunchKernelGGL(fp_rows_kernel<4>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
+            else if (G == 3) hipLaunchKernelGGL(fp_rows_kernel<3>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
+            else if (G == 2) hipLaunchKernelGGL(fp_rows_kernel<2>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
+            else hipLaunchKernelGGL(fp_rows_kernel<1>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
             CTG_HIP(hipGetLastError());
         }
         dim3 fg((unsigned)((a.W + 31) / 32), (unsigned)((a.H + 31) / 32), (unsigned)nproj);

@@ -618,6 +618,63 @@ def test_forward_projector_entry_form_matches_gather_form(gpu, case):
     np.testing.assert_allclose(acc.cpu().numpy(), base.cpu().numpy() + out["entry"], rtol=1e-6, atol=1e-4)
 
 
+@pytest.mark.parametrize("shape", [(64, 0, 33), (300, 5, 64), (96, 37, 128), (128, 64, 192), (80, 31, 300)])
+@pytest.mark.parametrize("special", [False, True])
+def test_forward_projector_runs_match_gather_form(gpu, shape, special):
+    """fp_rows_kernel at the edges of its split: windows of one to four chunks of 64 slices
+    and a partial last one, slabs that start off a chunk, more depth steps than a fill round
+    has lanes, and two lateral rounds (views near 45 degrees).  Both forms add the same taps
+    in FP32 (n of them at most 1200, so a relative error of about sqrt(n) 6e-8 = 2e-6).
+    Voxels that are not finite reach the gather form's pixels and no others, and infinite
+    ones keep their sign where a 1 in their place is seen and no other such voxel."""
+    import os
+    import torch
+    import ct_amd
+    n, z0, nz = shape
+    rng = np.random.default_rng(n + nz + special)
+    g = ct_amd.geometry_grid(n, 96, 3.0 * n, 1.25, n, n, z0 + nz + 3)
+    P = 6
+    angles, heights = np.array([0.0, 44.0, 45.0, 91.0, 137.0, 290.0]), np.linspace(-4.0, 4.0, P)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    ctx.set_projections(angles, heights)
+    x = rng.standard_normal((n, n, nz)).astype(np.float32)
+    at = {np.inf: (n // 2, n // 2 + 3, nz // 2), -np.inf: (n // 3, n // 2, nz // 3), np.nan: (n // 2, n // 3, nz // 2 + 1)}
+
+    def project(x, form="rows"):
+        if form == "gather":
+            os.environ["CTG_FP_GATHER"] = "1"
+        try:
+            Ax = torch.empty((P, g.det_height, g.det_width), dtype=torch.float32, device="cuda")
+            ctx.forward_project(torch.from_numpy(x).cuda(), z0, nz, 0, P, Ax)
+            torch.cuda.synchronize()
+        finally:
+            os.environ.pop("CTG_FP_GATHER", None)
+        return Ax.cpu().numpy()
+
+    if not special:
+        want = project(x, "gather")
+        assert np.abs(want).max() > 0.0
+        assert rel_rmse(project(x), want) < 2e-6
+        return
+    hit = {}
+    for v, i in at.items():
+        one = np.zeros_like(x)
+        one[i] = 1.0
+        hit[str(v)] = project(one) != 0.0
+        x[i] = v
+    got = project(x)
+    any_hit = ~np.isfinite(project(x, "gather"))
+    assert any_hit.any() and (hit["inf"] & any_hit).any() and (hit["-inf"] & any_hit).any()
+    np.testing.assert_array_equal(~np.isfinite(got), any_hit)
+    assert (got[hit["inf"] & ~hit["-inf"] & ~hit["nan"]] == np.inf).all()
+    assert (got[hit["-inf"] & ~hit["inf"] & ~hit["nan"]] == -np.inf).all()
+    for i in at.values():
+        x[i] = 0.0
+    want = project(x, "gather")
+    assert rel_rmse(got[~any_hit], want[~any_hit]) < 2e-6
+
+
 def test_phantom_generator_matches_oracle(gpu, oracle):
     import torch
     scan = small_scan(W=64, H=48, P=6, seed=12)
