@@ -31,8 +31,8 @@
 //    a projection whose box exceeds the tile capacity reads entries from global memory
 //    instead, so any geometry stays correct;
 //  - workgroups are numbered so that each XCD (dispatch is round-robin over 8 XCDs)
-//    receives a contiguous range of tiles, in 4x4 blocks of tiles, and shares detector
-//    footprints in its own L2.
+//    receives contiguous ranges of tiles, in 4x4 blocks of tiles, and shares detector
+//    footprints in its own L2, with an equal part of every layer (tile_of).
 //
 // What bounds it (1024^3 x 720 x 1024^2, MI355X): with FP32 entries the traffic of boxes that
 // miss L2 (747 GB per launch, 4.6 TB/s; 137 ms instead of 162 when every staged line hits),
@@ -59,17 +59,79 @@ constexpr int kMaxTileBytes = 36 * 1024;  // per LDS buffer (two buffers per wor
 // expressions round differently by about 1e-4 pixel at most.
 constexpr float kBoxMargin = 0.05f;
 
+constexpr int kMaxStrips = 64;  // strips of a layer
+
 struct BpArgs {
     int W, H, nx, ny, nzs, z0;
     float xpre, ypre, zpre, upre, vpre;
     float r2, fcd, uoff, ulo, uhi, vlo, vhi;
     int nproj, ntx, nty, nzb, cap, accumulate, vec4;
-    int blk, ntxp, ntyp;     // tile blocks of blk x blk (0: rows of tiles); tile counts rounded up to blk
     int zshift;              // z0 mod ZPL: runs start at grid z multiples of ZPL, zshift voxels before the slab
     int dma16;               // 8-byte entries staged with 16-byte DMA (H even: rows start even)
     int pitch_mod, pitch_rem;  // LDS column pitch = rows rounded up to pitch_rem mod pitch_mod (a power of two)
     int pitch_adapt;           // per box, -pitch_rem mod pitch_mod where the footprint slants the other way
+    // numbering of the tiles (tile_of)
+    int strip_h, nstrips, blk;  // tile rows per strip, tile columns per block
+    unsigned nwork, nidle;     // tiles of one layer inside / outside the strips' ranges
+    unsigned per, chunk, extra;  // 8 nzb chunks, the first `extra` of chunk + 1 tiles, the others of chunk; the largest
+    unsigned before[kMaxStrips + 1];  // working tiles of the strips before each
+    int first[kMaxStrips];            // first working tile column of each strip
 };
+
+// Tile of this workgroup; false for the surplus of the rounded-up grid.  A layer (one run of
+// slices) is cut into strips of strip_h tile rows, each with the range of tile columns inside
+// the reconstruction cylinder; a strip is numbered in blocks of blk columns, so that
+// consecutive numbers are neighbours along every ray direction.  The working tiles of all
+// layers, in that order, are cut into chunks of equal size (to one tile), eight per layer, that
+// go to the XCDs in turn (dispatch is round-robin over 8 XCDs).  So an XCD works on a
+// contiguous region, whose footprints its own L2 holds, and yet has an equal share of every
+// layer and, since the turn shifts by three per layer, of every part of the layers: outer
+// layers and tiles leave the detector window and are cheaper.  The tiles outside the
+// cylinder only store; they come last.
+//
+// One contiguous range of all tiles per XCD (outer layers all on two of them) took 2.21 ms for
+// a 256^3 scan of 360 projections of 256 x 192 and 12.6 ms for 512^3 of 512 x 512, this
+// numbering 1.56 and 11.05 ms; 1024^3 does not depend on it (160 ms FP32, 130 FP16), nor on two
+// or half a chunk per layer, strips of 2 rows, by more than 3 %; single blocks dealt in turn
+// take 171 and 140 ms there, and blocks numbered column by column 132 with FP16.
+__device__ inline bool tile_of(const BpArgs& a, int& zbi, int& tx, int& ty) {
+    const unsigned xcd = blockIdx.x & 7u, k = blockIdx.x >> 3;
+    const bool work = k < (unsigned)a.nzb * a.per;
+    unsigned n;
+    if (work) {
+        const unsigned m = k / a.per, w = k - m * a.per, i = m * 8u + ((xcd + 3u * m) & 7u);
+        if (w >= a.chunk + (i < a.extra ? 1u : 0u)) return false;
+        n = i * a.chunk + min(i, a.extra) + w;
+    } else {
+        n = (k - (unsigned)a.nzb * a.per) * 8u + xcd;
+        if (n >= a.nidle * (unsigned)a.nzb) return false;
+    }
+    const unsigned layer = work ? a.nwork : a.nidle;
+    zbi = (int)(n / layer);
+    unsigned t = n - (unsigned)zbi * layer;
+    // the last strip that starts at or before t
+    auto start = [&](int s) { return work ? a.before[s] : (unsigned)(a.ntx * a.strip_h * s) - a.before[s]; };
+    int lo = 0, hi = a.nstrips;  // start(lo) <= t < start(hi)
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (start(mid) <= t) lo = mid;
+        else hi = mid;
+    }
+    t -= start(lo);
+    const int h = min(a.strip_h, a.nty - lo * a.strip_h);
+    const int n_in = (int)(a.before[lo + 1] - a.before[lo]) / h;  // working columns
+    if (work) {
+        const int hb = a.blk * h, b = (int)t / hb, w = (int)t - b * hb;
+        const int bw = min(a.blk, n_in - a.blk * b), y = w / bw;
+        tx = a.first[lo] + a.blk * b + (w - y * bw);
+        ty = lo * a.strip_h + y;
+    } else {
+        const int c = (int)t / h;
+        tx = c < a.first[lo] ? c : c + n_in;
+        ty = lo * a.strip_h + ((int)t - c * h);
+    }
+    return true;
+}
 
 // Entry formats: FP32 (16 B), FP16 and BF16 (8 B: {A,dU} {dV,dUV} as 16-bit pairs).
 struct EF32 {
@@ -161,30 +223,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     // per projection: sin, cos, height, and the entry scale in w (written with the boxes)
     __shared__ float4 params[2][64];
 
-    // XCD-aware numbering: dispatch sends workgroup L to XCD L%8; give each XCD a
-    // contiguous range of work items.
-    const unsigned N = gridDim.x, L = blockIdx.x;
-    const unsigned xcd = L & 7u, kk = L >> 3, q8 = N >> 3, r8 = N & 7u;
-    const unsigned item = xcd * q8 + min(xcd, r8) + kk;
     int zbi, tx, ty;
-    if (a.blk > 0) {
-        // consecutive items cover blk x blk squares of tiles, whose detector footprints
-        // overlap along every ray direction (the workgroups an XCD runs together then
-        // share their boxes in its L2); tiles of the rounded-up grid beyond it exit
-        const unsigned ntxy = (unsigned)(a.ntxp * a.ntyp), bb = (unsigned)(a.blk * a.blk);
-        zbi = (int)(item / ntxy);
-        const unsigned t = item - (unsigned)zbi * ntxy, b = t / bb, w = t - b * bb;
-        const unsigned sbx = (unsigned)(a.ntxp / a.blk), by = b / sbx;
-        tx = (int)((b - by * sbx) * a.blk + w % a.blk);
-        ty = (int)(by * a.blk + w / a.blk);
-        if (tx >= a.ntx || ty >= a.nty) return;
-    } else {
-        const unsigned ntxy = (unsigned)(a.ntx * a.nty);
-        zbi = (int)(item / ntxy);
-        const int txy = (int)(item - (unsigned)zbi * ntxy);
-        ty = txy / a.ntx;
-        tx = txy - ty * a.ntx;
-    }
+    if (!tile_of(a, zbi, tx, ty)) return;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int xi = tx * kTX + (tid & (kTX - 1));
@@ -634,6 +674,14 @@ BpArgs make_args(const ctg_geometry& g, int nproj, int z0, int nz, int accumulat
     return a;
 }
 
+bool tile_in_cylinder(const ctg_geometry& g, int tx, int ty) {
+    const float cxa = (float)(tx * kTX) - g.x_pre, cxb = (float)std::min(tx * kTX + kTX - 1, g.nx - 1) - g.x_pre;
+    const float cya = (float)(ty * kTY) - g.y_pre, cyb = (float)std::min(ty * kTY + kTY - 1, g.ny - 1) - g.y_pre;
+    const float ndx = cxa > 0.0f ? cxa : (cxb < 0.0f ? cxb : 0.0f);
+    const float ndy = cya > 0.0f ? cya : (cyb < 0.0f ? cyb : 0.0f);
+    return ndx * ndx + ndy * ndy < g.radius * g.radius;
+}
+
 // Largest footprint box (entries) over a sample of tiles and projections, with the
 // same construction as box_for on the device.  Boxes that exceed the resulting
 // capacity at run time take the global-memory path, so sampling only affects speed.
@@ -654,9 +702,7 @@ int sample_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, i
                 const float cxb = (float)std::min(tx * kTX + kTX - 1, g.nx - 1) - g.x_pre;
                 const float cya = (float)(ty * kTY) - g.y_pre;
                 const float cyb = (float)std::min(ty * kTY + kTY - 1, g.ny - 1) - g.y_pre;
-                const float ndx = cxa > 0.0f ? cxa : (cxb < 0.0f ? cxb : 0.0f);
-                const float ndy = cya > 0.0f ? cya : (cyb < 0.0f ? cyb : 0.0f);
-                if (!(ndx * ndx + ndy * ndy < g.radius * g.radius)) continue;
+                if (!tile_in_cylinder(g, tx, ty)) continue;
                 for (int p = 0; p < nproj; p += pstep) {
                     const float4 q = hp[p];
                     float umin = INFINITY, umax = -INFINITY, vmin = INFINITY, vmax = -INFINITY;
@@ -720,6 +766,37 @@ int cached_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, i
     return cap;
 }
 
+// Strips and chunks of the tile numbering (tile_of).
+void number_tiles(const ctg_geometry& g, BpArgs& a) {
+    // blocks of 4 x 4 tiles; CTG_BP_BLOCK=n sets their edge, 0 takes single rows (tuning)
+    int edge = 4;
+    if (const char* e = std::getenv("CTG_BP_BLOCK")) edge = std::max(0, std::min(64, std::atoi(e)));
+    a.strip_h = std::max(edge, 1);
+    a.blk = edge > 0 ? edge : a.ntx;
+    while ((a.nty + a.strip_h - 1) / a.strip_h > kMaxStrips) a.strip_h *= 2;
+    a.nstrips = (a.nty + a.strip_h - 1) / a.strip_h;
+    a.before[0] = 0;
+    for (int s = 0; s < a.nstrips; ++s) {
+        const int y0 = s * a.strip_h, h = std::min(a.strip_h, a.nty - y0);
+        int lo = a.ntx, hi = -1;
+        for (int ty = y0; ty < y0 + h; ++ty)
+            for (int tx = 0; tx < a.ntx; ++tx)
+                if (tile_in_cylinder(g, tx, ty)) {
+                    lo = std::min(lo, tx);
+                    hi = std::max(hi, tx);
+                }
+        if (hi < lo) lo = 0;
+        a.first[s] = lo;
+        a.before[s + 1] = a.before[s] + (unsigned)((hi - lo + 1) * h);
+    }
+    a.nwork = a.before[a.nstrips];
+    a.nidle = (unsigned)(a.ntx * a.nty) - a.nwork;
+    const unsigned total = a.nwork * (unsigned)a.nzb;
+    a.chunk = total / (8u * (unsigned)a.nzb);
+    a.extra = total - a.chunk * 8u * (unsigned)a.nzb;
+    a.per = a.chunk + (a.extra ? 1 : 0);
+}
+
 template <int ZPL>
 ctg_status launch_zpl(const BpLaunch& L, BpArgs a, hipStream_t st) {
     const ctg_geometry& g = *L.g;
@@ -759,13 +836,9 @@ ctg_status launch_zpl(const BpLaunch& L, BpArgs a, hipStream_t st) {
     cap &= ~7;  // keeps the second buffer and every column start 16-byte aligned
     a.cap = cap;
     const size_t lds = (size_t)2 * cap * ebytes;
-    // workgroups in 4 x 4 blocks of tiles (measured against rows of tiles and 8 x 8 and
-    // 16 x 16 blocks); CTG_BP_BLOCK=n sets the block edge, 0 for rows (tuning)
-    a.blk = 4;
-    if (const char* e = std::getenv("CTG_BP_BLOCK")) a.blk = std::max(0, std::min(64, std::atoi(e)));
-    a.ntxp = a.blk > 0 ? (a.ntx + a.blk - 1) / a.blk * a.blk : a.ntx;
-    a.ntyp = a.blk > 0 ? (a.nty + a.blk - 1) / a.blk * a.blk : a.nty;
-    const long long grid = (long long)a.ntxp * a.ntyp * a.nzb;
+    if ((long long)a.ntx * a.nty * a.nzb > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
+    number_tiles(g, a);
+    const long long grid = 8ll * ((long long)a.nzb * a.per + ((long long)a.nidle * a.nzb + 7) / 8);
     if (grid > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
 #define CTG_BP_LAUNCH(E, DMA)                                                                           \
     hipLaunchKernelGGL((bp_kernel<ZPL, E, DMA>), dim3((unsigned)grid), dim3(kThreads), lds, st, a, L.d_params, \

@@ -957,6 +957,46 @@ def test_lds_forms_match_the_global_form(gpu, monkeypatch, store, nz, z0):
         assert np.all(volume()[x * x + y * y >= g.radius ** 2] == 0.5)
 
 
+@pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
+                                        (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
+def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
+    """Every tile of a layer runs once, whatever part of it the cylinder covers: one tile,
+    narrow grids, strips without a working tile, more tile rows than strips of four, partial
+    last tiles.  Images of ones give the sum of U^2 over the projections whose u window holds
+    the voxel (every v window does), and 0 outside the cylinder; FP32 rounding of U and of
+    the sum leaves 1e-5.  The volume starts as NaN."""
+    import torch
+    import ct_amd
+    P = 3
+    g = ct_amd.geometry_grid(W, 2 * nz + 8, 4.0 * max(W, nx, ny), 0.0, nx, ny, nz)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    angles = np.array([0.0, 77.0, 200.0])
+    ctx.set_projections(angles, np.zeros(P))
+    img = torch.ones((P, g.det_height, W), device="cuda")
+    entries = torch.empty(ctx.filtered_bytes("f32", P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, dtype=torch.float32, device="cuda")
+    ctx.layout_projections(img, P, "f32", entries, scales)
+    v = torch.full((nx, ny, nz), float("nan"), device="cuda")
+    ctx.backproject(entries, "f32", scales, 0, P, v, 0, nz, False)
+    torch.cuda.synchronize()
+    x = np.arange(nx)[:, None] - float(g.x_pre)
+    y = np.arange(ny)[None, :] - float(g.y_pre)
+    a = np.deg2rad(angles)[:, None, None]
+    U = g.fcd / (g.fcd - (x * np.cos(a) + y * np.sin(a)))
+    u = (y * np.cos(a) - x * np.sin(a)) * U
+    want = (U ** 2 * ((u >= g.u_lo) & (u <= g.u_hi))).sum(0)
+    r2 = x * x + y * y
+    want[r2 >= g.radius ** 2] = 0.0
+    # not the voxels whose tests rounding may turn
+    sure = np.abs(r2 - g.radius ** 2) > 1e-4 * g.radius ** 2
+    sure &= ((np.abs(u - g.u_lo) > 1e-2) & (np.abs(u - g.u_hi) > 1e-2)).all(0)
+    got = v.cpu().numpy()
+    assert np.isfinite(got).all() and (want > 0).any()
+    err = np.abs(got - want[..., None])[sure]
+    assert err.max() <= 1e-5 * want.max()
+
+
 @pytest.mark.parametrize("W", [2, 33, 128, 129, 255, 257, 513, 1025, 2047, 2049, 4096, 4097])
 def test_row_filter_transform_lengths_match_oracle(gpu, oracle, W):
     """The row filter at the ends of each transform length: the padded lengths 256 to 16384
