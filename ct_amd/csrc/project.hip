@@ -401,8 +401,7 @@ __global__ __launch_bounds__(kGThreads) void fp_gather_kernel(FpArgs a, const fl
 //    the chunk start and whose offset from it is l & 31, as in the backprojection.  The
 //    voxels come through a buffer resource covering the candidate's interval (zero outside
 //    it, which is the window, slab and v-window mask).
-//  - A run is the longest of 16, 8, 4, 2 or 1 next candidates whose magnifications span
-//    [Umin, Umax] with (Umax - Umin) |z + h| <= 0.98 over the window; R is the row below the
+//  - A run is the most of the next 16 candidates whose magnifications span [Umin, Umax] with (Umax - Umin) |z + h| <= 0.98 over the window; R is the row below the
 //    smaller of vIndex(Umin) and vIndex(Umax), less 0.002 for the rounding of either.
 //  - At the end of a run each lane adds its sums into its wave's rows in LDS, kept in two
 //    copies (even and odd lanes): lanes two slices apart have rows at least 2U - 1e-3 > 1
@@ -411,22 +410,25 @@ __global__ __launch_bounds__(kGThreads) void fp_gather_kernel(FpArgs a, const fl
 //    instruction and the read-modify-writes need no atomics.  The host bounds the rows that
 //    any slice of the window can reach for every candidate U and height, [rbase, rbase +
 //    span), so lanes outside their interval (adding zero) stay inside their own copy.
-//  - At the end the eight copies are summed in a fixed order and added into the workgroup's
-//    own float2 column ps[p][c][*] of a column-major buffer (own column c, next column).
+//  - At the end the eight copies are summed in a fixed order (if a sum is infinite or NaN, the
+//    workgroup starts again and adds every voxel's two taps by themselves, so that such voxels
+//    reach their own two rows only) and added into the workgroup's own float2 column ps[p][c][*] of a column-major buffer (own column c, next column).
 //    Windows run one after another on one stream; fp_finish_kernel then adds ps[p][c][r].x +
 //    ps[p][c-1][r].y into the row-major image.
 // The order of every addition is fixed: the result does not depend on scheduling.
 //
-// What bounds it: VALU issue.  At 512^3 x 360 projections of 512 x 512 (5.9e8 wave-updates
-// inside the cylinder) it issues 1.24e10 wave instructions, 21 per update of which 13 are the
-// update itself: 12.6 of the 18.3 ms at the measured 2.5 cycles each.  A form that added each
-// voxel's two rows to LDS as it came (one 16-byte read-modify-write per update, LDS-bound)
-// took 24.8 ms; with its column-by-column order 1 % of the voxel reads hit the L2, with
-// fp_item's units 53 %.
+// What bounds it: VALU issue, then the memory: 92 % of the time remains at 512^3 when every
+// voxel read hits L2 (85 % of a 768^3 iteration with 60 projections per call).  At 512^3 x 360
+// projections of 512 x 512 (5.9e8 wave-updates inside the cylinder) it issues 1.07e10 VALU
+// instructions, 18 per update: 11 for the update, 2 for its candidate, 3 to end a run and
+// start the next (9.6 candidates per run), the rest to fill the list.  16.9 ms.  Twice the row
+// sums in LDS, |e| instead of max(e, 0) and runs of any length to 16 instead of powers of two
+// took 18.3 ms to that.  A form that added each voxel's two rows to LDS as it came (one 16-byte
+// read-modify-write per update, LDS-bound) took 24.8 ms; with its column-by-column order 1 %
+// of the voxel reads hit the L2, with fp_item's units 53 %.
 constexpr int kJ = 3;  // lateral slots per lane and round
 constexpr int kESlots = (kJ + 1) * kGThreads;  // a round always fits behind 256 candidates
 constexpr int kEMaxSpan = 512;  // rows per copy
-constexpr int kAside = 1 << 30;  // mark in a candidate's z interval word (2 kFpZBits bits in use)
 
 struct FpWin {
     int wz0;     // first grid slice of the window (a multiple of 64 past the run base)
@@ -435,14 +437,13 @@ struct FpWin {
     int stride;  // rows between copies
 };
 
-// min and max over aligned groups of lanes, doubled by one step: the lane 1, 2, 7 - l (of
-// eight) or 15 - l (of sixteen) away.  On the bits of positive floats, which order like
-// integers (no canonicalisation).
-template <int CTRL>
+// min and max over a lane and the `S` before it in its row of 16 lanes (fewer at the row's
+// start).  On the bits of positive floats, which order like integers (no canonicalisation).
+template <int S>
 __device__ inline void dpp_minmax(int& mn, int& mx) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    mn = min(mn, __builtin_amdgcn_mov_dpp(mn, CTRL, 0xf, 0xf, true));
-    mx = max(mx, __builtin_amdgcn_mov_dpp(mx, CTRL, 0xf, 0xf, true));
+    mn = min(mn, __builtin_amdgcn_update_dpp(mn, mn, 0x110 + S, 0xf, 0xf, false));  // row_shr:S
+    mx = max(mx, __builtin_amdgcn_update_dpp(mx, mx, 0x110 + S, 0xf, 0xf, false));
 #endif
 }
 // A scalar that the optimiser knows nothing about.
@@ -452,6 +453,14 @@ __device__ inline int opaque_scalar(int v) {
 #endif
     return v;
 }
+// acc += x |e|, in place (see fmac)
+__device__ inline void fma_abs(float& acc, float x, float e) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_fma_f32 %0, %1, |%2|, %0" : "+v"(acc) : "v"(x), "v"(e));
+#else
+    acc = fmaf(x, fabsf(e), acc);
+#endif
+}
 // x = v, keeping x in its register (see fmac)
 __device__ inline void set_in_place(float& x, float v) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -460,7 +469,7 @@ __device__ inline void set_in_place(float& x, float v) {
     x = v;
 #endif
 }
-__device__ inline float first_lane(int x) { return __int_as_float(__builtin_amdgcn_readfirstlane(x)); }
+__device__ inline float lane_value(int x, int lane) { return __int_as_float(__builtin_amdgcn_readlane(x, lane)); }
 
 // The workgroups that an XCD runs together (dispatch is round-robin over 8 XCDs) should read
 // the same voxels: a voxel column is read once per projection, by the column it falls on, and
@@ -498,8 +507,6 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int span = win.span, stride = win.stride;
-    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) acc_lds[i] = make_float2(0.0f, 0.0f);
-
     const float4 g = pp[p];
     const float sn = g.x, cs = g.y, h = g.z;
     const float Sx = a.fcd * cs + a.uoff * sn, Sy = a.fcd * sn - a.uoff * cs;
@@ -551,6 +558,12 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
     const float* colbase = vol + (zrb - a.z0) + zs;
     const unsigned off0 = (unsigned)((lane - (zs - (win.wz0 - zrb))) * (int)sizeof(float));
     const unsigned off1 = off0 + 256u;
+
+    // An infinite or NaN voxel makes all three rows of its run infinite or NaN: a column with
+    // such sums is computed again, tap by tap.
+    int by_tap = 0;
+again:
+    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) acc_lds[i] = make_float2(0.0f, 0.0f);
     __syncthreads();
 
     // Rounds: 256 depth steps (one per lane) times kJ lateral slots, all laterals of a block of
@@ -686,8 +699,10 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
                 ++ci_f;
                 __builtin_amdgcn_sched_barrier(0);  // keep the slots' loads in walk order
             };
-            // sums over a run of x, x e and x max(e, 0), e = vIndex - (R + 1), for the own and
-            // the next column: row R takes S2 - S1, row R + 2 S2, row R + 1 the rest of S0
+            const float vpre_run = a.vpre - 0.002f;
+            // sums S0, S1, S2 over a run of x, x e and x |e|, e = vIndex - (R + 1), for the own
+            // and the next column: row R takes (S2 - S1) / 2, R + 1 S0 - S2, R + 2 (S2 + S1) / 2
+            // (the LDS rows hold twice that)
             float acc[G][6];
             float row1[G];   // R + 1
             float2* at[G];   // row R in this lane's copy
@@ -698,31 +713,7 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
 #pragma unroll
                 for (int j = 0; j < 6; ++j) acc[k][j] = 0.0f;
             }
-            // The current run, and whether a run of this part was set aside.  Sums that are not
-            // finite (an infinite or NaN voxel) would spread over all three rows: such a run
-            // adds nothing here and its candidates are marked for the walk below, which adds
-            // each one's two taps by themselves.
-            int run_at = c_begin, run_n = 0, aside = 0;
             auto flush = [&]() {
-                float t = 0.0f;
-#pragma unroll
-                for (int k = 0; k < G; ++k) t += acc[k][0] + acc[k][1];
-                if (__ballot(!(fabsf(t) <= 3.402823466e38f))) {
-                    if (lane < run_n && run_at + lane < c_end) slots[run_at + lane].w |= kAside;
-                    aside = 1;
-#pragma unroll
-                    for (int k = 0; k < G; ++k)
-#pragma unroll
-                        for (int j = 0; j < 6; ++j) set_in_place(acc[k][j], 0.0f);
-                }
-#pragma unroll
-                for (int k = 0; k < G; ++k)
-#pragma unroll
-                    for (int c2 = 0; c2 < 2; ++c2) {
-                        const float s2 = acc[k][4 + c2], r0 = s2 - acc[k][2 + c2];
-                        set_in_place(acc[k][2 + c2], acc[k][c2] - (r0 + s2));
-                        set_in_place(acc[k][c2], r0);
-                    }
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     // The G rows of a lane and those of the other lanes are distinct; row j + 1
@@ -733,43 +724,35 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
                     for (int k = 0; k < G; ++k) o[k] = at[k][j];
 #pragma unroll
                     for (int k = 0; k < G; ++k) {
-                        o[k].x += acc[k][2 * j];
-                        o[k].y += acc[k][2 * j + 1];
+                        const float* S = acc[k];
+                        o[k].x = j == 0 ? o[k].x + (S[4] - S[2]) : j == 1 ? fmaf(2.0f, S[0] - S[4], o[k].x) : o[k].x + (S[4] + S[2]);
+                        o[k].y = j == 0 ? o[k].y + (S[5] - S[3]) : j == 1 ? fmaf(2.0f, S[1] - S[5], o[k].y) : o[k].y + (S[5] + S[3]);
                         at[k][j] = o[k];
-                        set_in_place(acc[k][2 * j], 0.0f);
-                        set_in_place(acc[k][2 * j + 1], 0.0f);
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                 }
+#pragma unroll
+                for (int k = 0; k < G; ++k)
+#pragma unroll
+                    for (int j = 0; j < 6; ++j) set_in_place(acc[k][j], 0.0f);
             };
             // starts a run at candidate ci; returns its length
             auto start_run = [&](int ci) -> int {
-                const int U = slots[min(ci + (lane & 15), c_end - 1)].y;
-                int mn = U, mx = U, n = 1;
-                float umin = first_lane(U), umax = umin;
-                auto grow = [&](int m) {
-                    // lane 0 holds the extremes of the first m candidates
-                    const float lo = first_lane(mn), hi = first_lane(mx);
-                    if (n * 2 == m && (hi - lo) * zm <= 0.98f) {
-                        n = m;
-                        umin = lo;
-                        umax = hi;
-                    }
-                };
-                dpp_minmax<0xB1>(mn, mx);  // quad_perm 1,0,3,2
-                grow(2);
-                dpp_minmax<0x4E>(mn, mx);  // quad_perm 2,3,0,1
-                grow(4);
-                dpp_minmax<0x141>(mn, mx);  // row_half_mirror
-                grow(8);
-                dpp_minmax<0x140>(mn, mx);  // row_mirror
-                grow(16);
+                // lane l of a row: the extremes of the next l + 1 magnitudes
+                int mn = slots[min(ci + (lane & 15), c_end - 1)].y, mx = mn;
+                dpp_minmax<1>(mn, mx);
+                dpp_minmax<2>(mn, mx);
+                dpp_minmax<4>(mn, mx);
+                dpp_minmax<8>(mn, mx);
+                const unsigned over = (unsigned)__ballot(!((__int_as_float(mx) - __int_as_float(mn)) * zm <= 0.98f));
+                const int n = __builtin_ctz((over & 0xfffeu) | 0x10000u);
+                const float umin = lane_value(mn, n - 1), umax = lane_value(mx, n - 1);
 #pragma unroll
                 for (int k = 0; k < G; ++k) {
-                    const float v1 = det_row_index(lane_k, umin, fmaf(-zh[k], umin, a.vpre));
-                    const float v2 = det_row_index(lane_k, umax, fmaf(-zh[k], umax, a.vpre));
-                    const float R = floorf(fminf(v1, v2) - 0.002f);
+                    // within 0.001 of vIndex of the lanes whose row is on the detector
+                    const float y = zh[k] + lane_k;
+                    const float R = floorf(fminf(fmaf(-y, umin, vpre_run), fmaf(-y, umax, vpre_run)));
                     set_in_place(row1[k], R + 1.0f);
                     at[k] = my_rows + (int)R;
                 }
@@ -780,8 +763,6 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
                 if (opaque_scalar(left) == 0) {
                     flush();  // before the first run: zeros
                     left = start_run(ci_p);
-                    run_at = ci_p;
-                    run_n = left;
                 }
                 --left;
                 ++ci_p;
@@ -796,19 +777,42 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
                 for (int k = 0; k < G; ++k) {
                     const float vA = fmaf(-zh[k], sl.it.U, a.vpre);  // det_row_anchor(zwa, h, U, vpre)
                     const float e = det_row_index(lane_k, sl.it.U, vA) - row1[k];
-                    const float xo = sl.it.wo * sl.x[k], xs = sl.it.ws * sl.x[k], h2 = fmaxf(e, 0.0f);
+                    const float xo = sl.it.wo * sl.x[k], xs = sl.it.ws * sl.x[k];
                     acc[k][0] += xo;
                     acc[k][1] += xs;
                     fmac(acc[k][2], xo, e);
                     fmac(acc[k][3], xs, e);
-                    fmac(acc[k][4], xo, h2);
-                    fmac(acc[k][5], xs, h2);
+                    fma_abs(acc[k][4], xo, e);
+                    fma_abs(acc[k][5], xs, e);
                 }
             };
             // Three items at a time, whatever is left (items past the last add zeros): with
             // a way out between them the compiler no longer knows which loads are older
             // and waits for all of them at each item.
-            if (c_begin < c_end) {
+            if (opaque_uniform(by_tap)) {
+                for (int ci = c_begin; ci < c_end; ++ci) {
+                    const int4 r = slots[ci];
+                    const int zb = r.w, lo = zb & ((1 << kFpZBits) - 1), hi1 = zb >> kFpZBits;
+                    const float U = __int_as_float(r.y), ws = __int_as_float(r.z), wo = U * U - ws;
+                    for (int k = 0; k < G; ++k) {
+                        const int z = win.wz0 - zrb + 64 * k + lane;
+                        const float zk = ((float)(win.wz0 + 64 * k + (lane & 32)) - a.zpre) + h;
+                        const float vI = det_row_index(lane_k, U, fmaf(-zk, U, a.vpre)), v0 = floorf(vI);
+                        const bool on = z >= lo && z < hi1;
+                        const float x = on ? 2.0f * colbase[(size_t)r.x * a.zstride + (z - zs)] : 0.0f;
+                        float2* const at0 = my_rows + (int)v0;
+                        for (int j = 0; j < 2; ++j) {
+                            const float wr = j ? vI - v0 : 1.0f - (vI - v0);
+                            float2 o = at0[j];
+                            o.x += wo * wr * x;
+                            o.y += ws * wr * x;
+                            if (on) at0[j] = o;
+                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                            __builtin_amdgcn_wave_barrier();
+                        }
+                    }
+                }
+            } else if (c_begin < c_end) {
                 Slot sa, sb, sc;
                 next(sa);
                 next(sb);
@@ -822,51 +826,37 @@ __global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win,
                     next(sc);
                 } while (ci_p < c_end);
                 flush();
-                if (opaque_scalar(aside)) {
-                    for (int ci = c_begin; ci < c_end; ++ci) {
-                        const int4 r = slots[ci];
-                        const int zb = __builtin_amdgcn_readfirstlane(r.w);
-                        if (!(zb & kAside)) continue;
-                        const int lo = zb & ((1 << kFpZBits) - 1), hi1 = (zb & ~kAside) >> kFpZBits;
-                        const float U = __int_as_float(r.y), ws = __int_as_float(r.z), wo = U * U - ws;
-                        for (int k = 0; k < G; ++k) {
-                            const int z = win.wz0 - zrb + 64 * k + lane;
-                            const float zk = ((float)(win.wz0 + 64 * k + (lane & 32)) - a.zpre) + h;
-                            const float vI = det_row_index(lane_k, U, fmaf(-zk, U, a.vpre)), v0 = floorf(vI);
-                            const bool on = z >= lo && z < hi1;
-                            const float x = on ? colbase[(size_t)r.x * a.zstride + (z - zs)] : 0.0f;
-                            const float fv = vI - v0;
-                            float2* const at0 = my_rows + (int)v0;
-                            for (int j = 0; j < 2; ++j) {
-                                const float wv2 = j ? fv : 1.0f - fv;
-                                float2 o = at0[j];
-                                if (on) {
-                                    o.x += wo * wv2 * x;
-                                    o.y += ws * wv2 * x;
-                                    at0[j] = o;
-                                }
-                                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                                __builtin_amdgcn_wave_barrier();
-                            }
-                        }
-                    }
-                }
             }
             ncand = 0;
             __syncthreads();  // every wave is done with the slots
         }
     }
     // sum the eight copies per row (waves in order, even before odd)
-    float2* col = ps + ((size_t)p * a.W + c) * a.H;
+    bool bad = false;
     for (int r = tid; r < span; r += kGThreads) {
         const int row = win.rbase + r;
         if (row < 0 || row >= a.H) continue;
-        float2 o = col[row];
-        for (int w = 0; w < 2 * kGWaves; ++w) {
+        float2 o = acc_lds[r];
+        for (int w = 1; w < 2 * kGWaves; ++w) {
             const float2 e = acc_lds[w * stride + r];
             o.x += e.x;
             o.y += e.y;
         }
+        bad |= !(fabsf(o.x) + fabsf(o.y) <= 3.402823466e38f);
+        acc_lds[r] = o;
+    }
+    if (__builtin_amdgcn_readfirstlane(__syncthreads_or(bad)) && !by_tap) {
+        by_tap = 1;
+        goto again;
+    }
+    float2* col = ps + ((size_t)p * a.W + c) * a.H;
+    for (int r = tid; r < span; r += kGThreads) {
+        const int row = win.rbase + r;
+        if (row < 0 || row >= a.H) continue;
+        const float2 s2 = acc_lds[r];
+        float2 o = col[row];
+        o.x = fmaf(0.5f, s2.x, o.x);
+        o.y = fmaf(0.5f, s2.y, o.y);
         col[row] = o;
     }
 }
