@@ -16,9 +16,12 @@ Volumes are ``(nx, ny, nz)`` FP32 tensors, z fastest (Common/Volume.h:260); dete
 stacks are ``(P, H, W)`` FP32 tensors.  All operators are linear, so the autograd
 Functions save no activations: the backward recomputes what it needs from the
 incoming gradient.  Memory for the backprojection layout (16 B per detector texel) is
-bounded by ``max_entry_bytes``: projections are then laid out and backprojected in
-batches, and re-laid out for every z-slab when the volume is processed in slabs of
-``slab_nz`` (per-slab recomputation instead of keeping the filtered projections).
+bounded by ``max_entry_bytes``: projections are then filtered, laid out and
+backprojected in batches, each over every slice, and recomputed where they are needed
+again instead of being kept.  The kernels take the whole z range in one call: a slab of
+its own would need a copy of its slices on either side (a z-fastest volume holds no slab
+contiguously), a layout of every batch per slab, and launches too small to fill the chip
+(512^3 from 360 projections in four slabs and batches of 64: 14.9 ms so, 11.4 ms whole).
 
 There is no CPU path: every call runs the HIP kernels and raises if the library or a
 GPU is missing.
@@ -39,7 +42,8 @@ class ConeBeamOperator:
 
     geometry: :class:`ct_amd.Geometry` (``ct_amd.geometry_grid`` / ``geometry_ctvolume``).
     angles_deg, heights_px: per-projection angle (degrees) and height offset (pixels).
-    slab_nz: process the volume in z-slabs of this many slices (None = whole volume).
+    slab_nz: slices per z-slab for callers that walk the volume slab by slab (checkpoints of
+        a refinement); None = one slab.  The operators themselves need no slabs.
     max_entry_bytes: cap on the backprojection layout buffer (None = all projections).
     filt: ramp-family window of the FDK operator ("ramlak", "shepplogan", "hann").
     """
@@ -85,33 +89,22 @@ class ConeBeamOperator:
         """A x: (nx, ny, nz) -> (P, H, W)."""
         volume = self._check(volume, self.volume_shape, "volume")
         out = torch.empty(self.proj_shape, dtype=torch.float32, device=self.device)
-        s = _stream()
-        for i, (z0, nz) in enumerate(self._slabs()):
-            slab = volume if nz == self.g.nz else volume[:, :, z0:z0 + nz].contiguous()
-            self.ctx.forward_project(slab, z0, nz, 0, self.nproj, out, accumulate=i > 0, stream=s)
+        if self.g.nz == 0:
+            return out
+        self.ctx.forward_project(volume, 0, self.g.nz, 0, self.nproj, out, stream=_stream())
         return out
 
     def _backproject_entries(self, make_entries, out: torch.Tensor):
         """Backprojects the layout produced by make_entries(p0, n, entries, scales) into out,
-        slab by slab; the layout is recomputed per slab unless all of it is resident."""
+        batch by batch."""
         s = _stream()
         per = self.ctx.filtered_bytes("f32", 1)
         entries = torch.empty(per * self.batch, dtype=torch.uint8, device=self.device)
         scales = torch.empty(self.batch, dtype=torch.float32, device=self.device)
-        resident = self.batch >= self.nproj
-        if resident:
-            make_entries(0, self.nproj, entries, scales)
-        for z0, nz in self._slabs():
-            whole = nz == self.g.nz
-            slab = out if whole else torch.empty((self.g.nx, self.g.ny, nz), dtype=torch.float32,
-                                                 device=self.device)
-            for p0 in range(0, self.nproj, self.batch):
-                n = min(self.batch, self.nproj - p0)
-                if not resident:
-                    make_entries(p0, n, entries, scales)
-                self.ctx.backproject(entries, "f32", scales, p0, n, slab, z0, nz, accumulate=p0 > 0, stream=s)
-            if not whole:
-                out[:, :, z0:z0 + nz] = slab
+        for p0 in range(0, self.nproj if self.g.nz else 0, self.batch):
+            n = min(self.batch, self.nproj - p0)
+            make_entries(p0, n, entries, scales)
+            self.ctx.backproject(entries, "f32", scales, p0, n, out, 0, self.g.nz, accumulate=p0 > 0, stream=s)
         return out
 
     def backproject(self, images: torch.Tensor) -> torch.Tensor:
@@ -147,16 +140,7 @@ class ConeBeamOperator:
         grad_volume = self._check(grad_volume, self.volume_shape, "grad_volume")
         s = _stream()
         out = torch.empty(self.proj_shape, dtype=torch.float32, device=self.device)
-        if self.slab_nz >= self.g.nz:
-            self.ctx.fdk_backward(grad_volume, 0, self.g.nz, 0, self.nproj, self.filt, out, stream=s)
-            return out
-        # slabs: A is accumulated over slabs first, then filtered and weighted once
-        for i, (z0, nz) in enumerate(self._slabs()):
-            slab = grad_volume[:, :, z0:z0 + nz].contiguous()
-            self.ctx.forward_project(slab, z0, nz, 0, self.nproj, out, accumulate=i > 0, stream=s)
-        H = self.g.det_height
-        self.ctx.filter_rows(out, out, self.nproj * H, self.filt, stream=s)
-        self.ctx.feldkamp_weight(out, self.nproj, stream=s)
+        self.ctx.fdk_backward(grad_volume, 0, self.g.nz, 0, self.nproj, self.filt, out, stream=s)
         return out
 
 

@@ -56,6 +56,7 @@ constexpr int kSlots = 512;  // candidate slots per pass (16 B each)
 constexpr int kMaxRowsFp = 4096;  // detector rows held in LDS per wave
 constexpr int kFpZBits = 14;      // z interval bounds in a candidate record (relative to the run base)
 constexpr int kFpMaxSlab = (1 << kFpZBits) - 2 * kRowAnchor;  // slices per launch
+static_assert(kFpMaxSlab % (2 * kRowAnchor) == 0, "the next launch starts on a chunk");
 
 // Raw buffer resource over `bytes` bytes of global memory: a 4-byte load at an offset at
 // or past the end returns zero.  The builtins exist only in the device pass.
@@ -1076,34 +1077,39 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
         const int deep = (nch + (nch + 3) / 4 - 1) / ((nch + 3) / 4);
         for (int cand = deep; cand >= 1 && G == 0; --cand) {
             bool fits = true;
-            for (int w0 = zrb; w0 < z0 + nz && fits; w0 += 64 * cand) {
-                int rb, sp;
-                window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * cand, rb, sp);
-                fits = sp <= max_span;
-            }
+            for (int s = 0; s < nz; s += kFpMaxSlab)
+                for (int w0 = zrb + s; w0 < z0 + std::min(s + kFpMaxSlab, nz) && fits; w0 += 64 * cand) {
+                    int rb, sp;
+                    window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * cand, rb, sp);
+                    fits = sp <= max_span;
+                }
             if (fits) G = cand;
         }
     }
-    if (G > 0 && nz <= kFpMaxSlab) {
+    if (G > 0) {
         const size_t cells = (size_t)nproj * a.W * a.H;
         CTG_TRY(work.reserve(cells * sizeof(float2)));
         float2* ps = work.as<float2>();
         CTG_TRY(fill_u32(ps, 0u, cells * 2, st));
-        const int zrb = z0 & ~(kRowAnchor - 1);
         const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj) + 7) / 8) * 8 * kPBlock * kCBlock;
         if (blocks > 0x7fffffffull) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
         const dim3 rgrid((unsigned)blocks);
-        for (int w0 = zrb; w0 < z0 + nz; w0 += 64 * G) {
-            FpWin win{};
-            win.wz0 = w0;
-            window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * G, win.rbase, win.span);
-            win.stride = (win.span + 1) & ~1;
-            const size_t lds = sizeof(float2) * 2 * kGWaves * (size_t)win.stride;
-            if (G == 4) hipLaunchKernelGGL(fp_rows_kernel<4>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-            else if (G == 3) hipLaunchKernelGGL(fp_rows_kernel<3>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-            else if (G == 2) hipLaunchKernelGGL(fp_rows_kernel<2>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-            else hipLaunchKernelGGL(fp_rows_kernel<1>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-            CTG_HIP(hipGetLastError());
+        // the candidate records hold z relative to the launch's run base in kFpZBits bits
+        for (int s = 0; s < nz; s += kFpMaxSlab) {
+            a.z0 = z0 + s;
+            a.nzs = std::min(kFpMaxSlab, nz - s);
+            for (int w0 = a.z0 & ~(kRowAnchor - 1); w0 < a.z0 + a.nzs; w0 += 64 * G) {
+                FpWin win{};
+                win.wz0 = w0;
+                window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * G, win.rbase, win.span);
+                win.stride = (win.span + 1) & ~1;
+                const size_t lds = sizeof(float2) * 2 * kGWaves * (size_t)win.stride;
+                if (G == 4) hipLaunchKernelGGL(fp_rows_kernel<4>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
+                else if (G == 3) hipLaunchKernelGGL(fp_rows_kernel<3>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
+                else if (G == 2) hipLaunchKernelGGL(fp_rows_kernel<2>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
+                else hipLaunchKernelGGL(fp_rows_kernel<1>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
+                CTG_HIP(hipGetLastError());
+            }
         }
         dim3 fg((unsigned)((a.W + 31) / 32), (unsigned)((a.H + 31) / 32), (unsigned)nproj);
         hipLaunchKernelGGL(fp_finish_kernel, fg, dim3(256), 0, st, ps, a.W, a.H, d_proj);
