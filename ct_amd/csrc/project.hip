@@ -6,8 +6,8 @@
 // the backprojection would read through taps (u0,v0),(u0+1,v0),(u0,v0+1),(u0+1,v0+1) with
 // weight U^2 and bilinear weights instead adds U^2 * f * weight into those pixels, under
 // the same cylinder and window masks.  A workgroup owns a pixel column of one projection and
-// collects the voxel columns that land on it: fp_rows_kernel, or fp_gather_kernel where the
-// geometry rules that one out.
+// collects the voxel columns that land on it: fp_rows_kernel, fp_entry_kernel for small
+// volumes, or fp_gather_kernel where the geometry rules those out.
 #include "ctg_internal.h"
 
 #include <algorithm>
@@ -377,6 +377,304 @@ __global__ __launch_bounds__(kGThreads) void fp_gather_kernel(FpArgs a, const fl
     }
 }
 
+struct FpWin {
+    int wz0;     // first grid slice of the window (a multiple of 64 past the run base)
+    int rbase;   // first row any voxel of the window can reach
+    int span;    // rows per copy
+    int stride;  // rows between copies
+};
+
+// -------------------------------------------------------- entry-space projector
+//
+// The backprojection evaluates a voxel's value from ONE coefficient entry (A, dU, dV, dUV)
+// at (u0, v0): val = A + fu dU + fv (dV + fu dUV), weighted by w = U^2.  Its transpose
+// therefore adds (w x, w x fu, w x fv, w x fu fv) into one entry gradient per (voxel,
+// projection), and the transpose of the layout (A = q00, dU = q10 - q00, dV = q01 - q00,
+// dUV = q11 - q10 - q01 + q00) turns entry gradients into pixels:
+//     q00 += gA - gdU - gdV + gdUV,  q01 += gdV - gdUV,  q10 += gdU - gdUV,  q11 += gdUV.
+//
+// fp_entry_kernel<G>: candidates, windows, lanes and voxel reads as in fp_rows_kernel below,
+// but every voxel is added into its entry as it comes, with one LDS read and one write of 16
+// bytes, in two private copies per wave (even and odd lanes: same-parity lanes of an item are
+// two or more slices apart, so their rows differ).  Each round of 256 slots is walked at once,
+// candidate ci by wave ci mod 4.  At the end the eight copies are summed in a fixed order.
+//
+// What bounds it: the LDS (a 16-byte read and write take 18 cycles per wave and CU), a third
+// more per update than fp_rows_kernel at 512^3, but it has no runs to begin and end.  It is the
+// faster one where columns are short (see the launch): 59 against 64 us at 96^2 x 72 from 48
+// projections of 103 x 83, 296 against 311 at 128^3 from 200, but 217 against 207 at 200^2 x
+// 128 from 60 and 428 against 302 at 160^3 from 100, where a third window is begun.
+constexpr int kEntryMaxSpan = 256;  // entry rows per copy
+constexpr int kEntryMaxSide = 160;  // voxels
+
+__device__ inline int flr_i32(float x) {
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
+template <int G>
+__global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win, const float4* __restrict__ pp,
+                                                             const float* __restrict__ vol,
+                                                             float2* __restrict__ ps) {
+    // column, U, w fu and the z interval relative to the run base (w = U^2 is recomputed
+    // from U): one 16-byte LDS read per item
+    __shared__ int4 slots[kGThreads];
+    __shared__ int wave_cnt[kGWaves];
+    // [wave][parity][row], copies `stride` entries apart, a multiple of 16.  On gfx950 a ds_write_b128 occupies the LDS for about
+    // 13.5 cycles per wave instruction whatever its lane mask and a conflict-free
+    // ds_read_b128 about 4 (16 lanes per cycle); of the copy offsets 0, 2, 5, 6, 8 and 13
+    // entries modulo 16, 0 was the fastest on the 512^3 x 360 workload.
+    extern __shared__ float4 entry_lds[];
+    const int c = blockIdx.x;
+    const int p = blockIdx.y;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int span = win.span, stride = win.stride;
+    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) entry_lds[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+
+    const float4 g = pp[p];
+    const float sn = g.x, cs = g.y, h = g.z;
+    const float Sx = a.fcd * cs + a.uoff * sn, Sy = a.fcd * sn - a.uoff * cs;
+    const float ulo = (float)c - 0.05f - a.upre, uhi = (float)c + 1.05f - a.upre;
+    const float q0x = -(ulo - a.uoff) * sn, q0y = (ulo - a.uoff) * cs;
+    const float q1x = -(uhi - a.uoff) * sn, q1y = (uhi - a.uoff) * cs;
+    const float umid = (float)c + 0.5f - a.upre - a.uoff;
+    const bool xmajor = fabsf(-umid * sn - Sx) >= fabsf(umid * cs - Sy);
+    const int n_out = xmajor ? a.nx : a.ny, n_in = xmajor ? a.ny : a.nx;
+    const float pre_out = xmajor ? a.xpre : a.ypre, pre_in = xmajor ? a.ypre : a.xpre;
+    const float So = xmajor ? Sx : Sy, Si = xmajor ? Sy : Sx;
+    const float k0 = ((xmajor ? q0y : q0x) - Si) / ((xmajor ? q0x : q0y) - So);
+    const float k1 = ((xmajor ? q1y : q1x) - Si) / ((xmajor ? q1x : q1y) - So);
+    const float R = sqrtf(a.r2);
+    const int o_lo = max(0, (int)floorf(pre_out - R) - 1), o_hi = min(n_out - 1, (int)ceilf(pre_out + R) + 1);
+    const int zend = a.z0 + a.nzs - 1;
+    const int zrb = a.z0 & ~(kRowAnchor - 1);
+    // the slices of this window inside the slab
+    const int wlo = max(a.z0, win.wz0), whi = min(zend, win.wz0 + 64 * G - 1);
+
+    auto jrange = [&](int o, int& jl, int& jh) {
+        const float ow = (float)o - pre_out;
+        const float i0 = Si + (ow - So) * k0, i1 = Si + (ow - So) * k1;
+        jl = max(0, (int)ceilf(fminf(i0, i1) + pre_in - 0.01f));
+        jh = min(n_in - 1, (int)floorf(fmaxf(i0, i1) + pre_in + 0.01f));
+    };
+    // lateral slots per depth step: the wedge width |i1 - i0| is linear in the depth and
+    // the source lies outside the volume, so it peaks at an end of the depth range; a
+    // window of width w + 0.02 holds at most floor(w) + 2 integers
+    auto width = [&](int o) {
+        const float ow = (float)o - pre_out;
+        return fabsf((ow - So) * (k1 - k0));
+    };
+    const int jm = (int)fmaxf(width(o_lo), width(o_hi)) + 2;
+    const int nslot = (o_hi - o_lo + 1) * jm;
+
+    // per lane and chunk: world z of the slice's row anchor plus the height (the
+    // backprojection's zwa + h), and the slice's offset from the anchor
+    float zh[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) zh[k] = ((float)(win.wz0 + 64 * k + (lane & 32)) - a.zpre) + h;
+    const float lane_k = (float)(lane & 31);
+    // LDS byte address of entry row v0 in this lane's copy: v0 * 16 + lane_base
+    int lane_base = (wv * 2 + (lane & 1)) * stride * 16 - win.rbase * 16;
+    // opaque to the optimiser, so that v0 * 16 + lane_base stays one shift-and-add per
+    // voxel instead of being re-associated around rbase
+    asm volatile("" : "+v"(lane_base));
+    char* acc_bytes = reinterpret_cast<char*>(entry_lds);
+    const float* colbase = vol + (zrb - a.z0);
+    const int zc = win.wz0 - zrb;  // the window's first slice relative to the run base
+    const unsigned lane4 = (unsigned)lane * (unsigned)sizeof(float);
+    __syncthreads();
+
+    int ncand = 0;
+    for (int sbase = 0; sbase < nslot && wlo <= whi; sbase += kGThreads) {
+        // fill, step 1: the cheap tests for 256 slots, survivors compacted (ballot prefix
+        // within each wave, wave totals through LDS)
+        const int sidx = sbase + tid;
+        int4 rec = make_int4(-1, 0, 0, 0);
+        if (sidx < nslot) {
+            const int oi = sidx / jm, jj = sidx - oi * jm;
+            const int o = o_lo + oi;
+            int jl, jh;
+            jrange(o, jl, jh);
+            const int j = jl + jj;
+            if (j <= jh) {
+                const int xi = xmajor ? o : j, yi = xmajor ? j : o;
+                // per-voxel arithmetic identical to the backprojection's
+                const float x = (float)xi - a.xpre, y = (float)yi - a.ypre;
+                if (x * x + y * y < a.r2) {
+                    float t = (-1.0f) * x * g.x + y * g.y;
+                    t += a.uoff;
+                    const float s = x * g.y + y * g.x;
+                    const float U = cone_magnification(a.fcd, s);
+                    const float u = t * U;
+                    if (u >= a.ulo && u <= a.uhi) {
+                        const float uIdx = u + a.upre;
+                        const int u0 = (int)uIdx;
+                        if (u0 == c) rec = make_int4(xi * a.ny + yi, __float_as_int(U), __float_as_int(uIdx - (float)u0), 0);
+                    }
+                }
+            }
+        }
+        {
+            const unsigned long long m = __ballot(rec.x >= 0);
+            const int below = __popcll(m & ((1ull << lane) - 1ull));
+            if (lane == 0) wave_cnt[wv] = __popcll(m);
+            __syncthreads();
+            int base = ncand;
+            for (int w = 0; w < wv; ++w) base += wave_cnt[w];
+            int total = 0;
+            for (int w = 0; w < kGWaves; ++w) total += wave_cnt[w];
+            if (rec.x >= 0) slots[base + below] = rec;
+            __syncthreads();  // the slots are complete; wave_cnt is rewritten below
+            // fill, step 2: one lane per new survivor settles its z interval and writes its
+            // final record (candidates with an empty interval keep an empty one)
+            const int ci = ncand + tid;
+            if (tid < total) {
+                const int4 r = slots[ci];
+                const float U = __int_as_float(r.y), fu = __int_as_float(r.z);
+                auto v_of = [&](int zi) { const float zk = (float)zi - a.zpre; return (zk + h) * U; };
+                int lo = wlo, hi = whi;
+                if (!(v_of(wlo) >= a.vlo && v_of(whi) <= a.vhi)) {
+                    // the passing z of v = (zk + h) U in [vLo, vHi] form an interval (v is
+                    // non-decreasing in z): estimate its ends, then settle them with the
+                    // backprojection's own expression
+                    const float iU = __builtin_amdgcn_rcpf(U);
+                    const float zlo_f = fminf(fmaxf(a.vlo * iU - h + a.zpre, (float)(wlo - 4)), (float)(whi + 4));
+                    const float zhi_f = fminf(fmaxf(a.vhi * iU - h + a.zpre, (float)(wlo - 4)), (float)(whi + 4));
+                    lo = (int)ceilf(zlo_f);
+                    hi = (int)floorf(zhi_f);
+#pragma unroll
+                    for (int it = 0; it < 2; ++it) {
+                        if (lo > wlo && v_of(lo - 1) >= a.vlo) --lo;
+                        if (hi < whi && v_of(hi + 1) <= a.vhi) ++hi;
+                    }
+#pragma unroll
+                    for (int it = 0; it < 2; ++it) {
+                        if (lo <= whi && !(v_of(lo) >= a.vlo)) ++lo;
+                        if (hi >= wlo && !(v_of(hi) <= a.vhi)) --hi;
+                    }
+                    lo = max(lo, wlo);
+                    hi = min(hi, whi);
+                }
+                const float w = U * U;
+                // an empty interval [lo, hi] with hi < lo becomes a zero-length resource
+                slots[ci] = make_int4(r.x, r.y, __float_as_int(w * fu),
+                                      (lo - zrb) | (max(hi, lo - 1) - zrb + 1) << kFpZBits);
+            }
+            ncand += total;
+            __syncthreads();  // records complete; wave_cnt free again
+        }
+        if (ncand > 0) {
+            struct Item {
+                vbuf rs;
+                float U, w, wfu;
+                int lo;
+            };
+            // past the last candidate an item still issues its loads, over an empty
+            // resource (they return zero without touching memory)
+            auto item_of = [&](int ci, bool valid) {
+                const int4 r = slots[valid ? ci : 0];
+                const int zb = __builtin_amdgcn_readfirstlane(r.w);
+                Item it;
+                it.lo = zb & ((1 << kFpZBits) - 1);
+                const int hi1 = (zb >> kFpZBits) & ((1 << kFpZBits) - 1);  // one past the last slice
+                it.rs = make_vbuf(colbase + (size_t)__builtin_amdgcn_readfirstlane(r.x) * a.zstride + it.lo,
+                                  valid ? (hi1 - it.lo) * (int)sizeof(float) : 0);
+                // the same value in every lane: kept in vector registers (operands of the
+                // per-voxel arithmetic), where moving them to scalars would cost a
+                // readfirstlane each
+                it.U = __int_as_float(r.y);
+                it.w = it.U * it.U;  // as in the fill: the weight is U^2
+                it.wfu = __int_as_float(r.z);
+                return it;
+            };
+            // Candidate ci goes to wave ci mod 4.  Three named slots keep the next two
+            // candidates' voxels in flight while one is accumulated.
+            struct Slot { Item it; float x[G]; };
+            int ci_f = wv;
+            auto next = [&](Slot& sl) -> bool {
+                const bool valid = ci_f < ncand;
+                sl.it = item_of(ci_f, valid);
+#pragma unroll
+                for (int k = 0; k < G; ++k)
+                    sl.x[k] = vbuf_load(sl.it.rs, vadd_sv((zc + 64 * k - sl.it.lo) * (int)sizeof(float), lane4));
+                ci_f += kGWaves;
+                __builtin_amdgcn_sched_barrier(0);  // keep the slots' loads in walk order
+                return valid;
+            };
+            // The G chunks of one item touch distinct entries of each copy (same-parity
+            // lanes of the item are two or more slices apart, so their rows differ), so
+            // all G reads are issued before the first write: one LDS round trip per item
+            // instead of one per chunk.
+            auto process = [&](const Slot& sl) {
+                float4* e[G];
+                float4 v[G];
+                float fv[G];
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const float vA = fmaf(-zh[k], sl.it.U, a.vpre);  // det_row_anchor(zwa, h, U, vpre)
+                    const float vI = det_row_index(lane_k, sl.it.U, vA);
+                    const int v0 = flr_i32(vI);
+                    fv[k] = __builtin_amdgcn_fractf(vI);
+                    e[k] = reinterpret_cast<float4*>(acc_bytes + (v0 * 16 + lane_base));
+                    v[k] = *e[k];
+                }
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const float t = sl.it.w * sl.x[k], tu = sl.it.wfu * sl.x[k];
+                    v[k].x += t;
+                    v[k].y += tu;
+                    v[k].z = fmaf(t, fv[k], v[k].z);
+                    v[k].w = fmaf(tu, fv[k], v[k].w);
+                    *e[k] = v[k];
+                }
+            };
+            Slot sa, sb, sc;
+            bool ha = next(sa), hb = next(sb), hc = next(sc);
+            while (ha) {
+                process(sa);
+                ha = next(sa);
+                if (!hb) break;
+                process(sb);
+                hb = next(sb);
+                if (!hc) break;
+                process(sc);
+                hc = next(sc);
+            }
+            ncand = 0;
+            __syncthreads();  // every wave is done with the slots
+        }
+    }
+    // sum the eight copies per entry row (waves in order, even before odd) and turn the
+    // entry gradients into pixel partials: own column (q00 at row v, q01 at v + 1) and
+    // the next column (q10 at v, q11 at v + 1); pixel row rbase + r takes entry rows r
+    // and r - 1
+    float2* col = ps + ((size_t)p * a.W + c) * a.H;
+    auto entry = [&](int r) {
+        float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (r >= 0 && r < span) {
+            for (int w = 0; w < kGWaves; ++w)
+                for (int par = 0; par < 2; ++par) {
+                    const float4 e = entry_lds[(w * 2 + par) * stride + r];
+                    sum.x += e.x; sum.y += e.y; sum.z += e.z; sum.w += e.w;
+                }
+        }
+        return sum;
+    };
+    for (int r = tid; r <= span; r += kGThreads) {
+        const int row = win.rbase + r;
+        if (row < 0 || row >= a.H) continue;
+        const float4 e0 = entry(r), e1 = entry(r - 1);  // entries at rows v = row and v = row - 1
+        const float own = ((e0.x - e0.y) - e0.z + e0.w) + (e1.z - e1.w);
+        const float side = (e0.y - e0.w) + e1.w;
+        float2 o = col[row];
+        o.x += own;
+        o.y += side;
+        col[row] = o;
+    }
+}
+
 // ------------------------------------------------------------ row-run projector
 //
 // Every voxel adds its two row taps to pixel columns c = u0 and c + 1, with weights
@@ -430,13 +728,6 @@ __global__ __launch_bounds__(kGThreads) void fp_gather_kernel(FpArgs a, const fl
 constexpr int kJ = 3;  // lateral slots per lane and round
 constexpr int kESlots = (kJ + 1) * kGThreads;  // a round always fits behind 256 candidates
 constexpr int kEMaxSpan = 512;  // rows per copy
-
-struct FpWin {
-    int wz0;     // first grid slice of the window (a multiple of 64 past the run base)
-    int rbase;   // first row any voxel of the window can reach
-    int span;    // rows per copy
-    int stride;  // rows between copies
-};
 
 // min and max over a lane and the `S` before it in its row of 16 lanes (fewer at the row's
 // start).  On the bits of positive floats, which order like integers (no canonicalisation).
@@ -1091,11 +1382,27 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
         CTG_TRY(work.reserve(cells * sizeof(float2)));
         float2* ps = work.as<float2>();
         CTG_TRY(fill_u32(ps, 0u, cells * 2, st));
+        bool entries = false;
         const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj) + 7) / 8) * 8 * kPBlock * kCBlock;
         if (blocks > 0x7fffffffull) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
         const dim3 rgrid((unsigned)blocks);
+        // Volumes of at most two chunks of slices (one window) and short rays go to the entry
+        // form: its time per update is larger, but it spends less per column (figures there).
+        if (z0 + nz - (z0 & ~(kRowAnchor - 1)) <= 128 && std::max(g.nx, g.ny) <= kEntryMaxSide && G <= 2) {
+            FpWin win{};
+            win.wz0 = z0 & ~(kRowAnchor - 1);
+            window_rows(g, hmin, hmax, Umin, Umax, win.wz0, 64 * G, win.rbase, win.span);
+            entries = win.wz0 + 64 * G >= z0 + nz && win.span <= kEntryMaxSpan;
+            win.stride = (win.span + 15) & ~15;
+            const size_t lds = sizeof(float4) * 2 * kGWaves * (size_t)win.stride;
+            if (entries) {
+                if (G == 2) hipLaunchKernelGGL(fp_entry_kernel<2>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
+                else hipLaunchKernelGGL(fp_entry_kernel<1>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
+                CTG_HIP(hipGetLastError());
+            }
+        }
         // the candidate records hold z relative to the launch's run base in kFpZBits bits
-        for (int s = 0; s < nz; s += kFpMaxSlab) {
+        for (int s = 0; s < nz && !entries; s += kFpMaxSlab) {
             a.z0 = z0 + s;
             a.nzs = std::min(kFpMaxSlab, nz - s);
             for (int w0 = a.z0 & ~(kRowAnchor - 1); w0 < a.z0 + a.nzs; w0 += 64 * G) {

@@ -618,15 +618,18 @@ def test_forward_projector_entry_form_matches_gather_form(gpu, case):
     np.testing.assert_allclose(acc.cpu().numpy(), base.cpu().numpy() + out["entry"], rtol=1e-6, atol=1e-4)
 
 
-@pytest.mark.parametrize("shape", [(64, 0, 33), (300, 5, 64), (96, 37, 128), (128, 64, 192), (80, 31, 300)])
-@pytest.mark.parametrize("special", [False, True])
+_ROW_RUNS = [(164, 0, 33), (300, 5, 64), (172, 37, 90), (128, 64, 192), (80, 31, 300)]
+_ENTRIES = [(16, 0, 1), (64, 0, 33), (160, 5, 64), (96, 37, 123), (130, 0, 128)]
+
+
+@pytest.mark.parametrize("shape,special", [(x, False) for x in _ROW_RUNS + _ENTRIES] + [(x, True) for x in _ROW_RUNS])
 def test_forward_projector_runs_match_gather_form(gpu, shape, special):
-    """fp_rows_kernel at the edges of its split: windows of one to four chunks of 64 slices
-    and a partial last one, slabs that start off a chunk, more depth steps than a fill round
-    has lanes, and two lateral rounds (views near 45 degrees).  Both forms add the same taps
-    in FP32 (n of them at most 1200, so a relative error of about sqrt(n) 6e-8 = 2e-6).
-    Voxels that are not finite reach the gather form's pixels and no others, and infinite
-    ones keep their sign where a 1 in their place is seen and no other such voxel."""
+    """fp_rows_kernel and fp_entry_kernel (small volumes) at the edges of their split: windows
+    of one to four chunks of 64 slices and a partial last one, slabs that start off a chunk,
+    more depth steps than a fill round has lanes, and two lateral rounds (views near 45
+    degrees).  All forms add the same taps in FP32 (n of them at most 1200, so a relative error of about sqrt(n) 6e-8 = 2e-6).
+    In a row run, voxels that are not finite reach the gather form's pixels and no others, and
+    infinite ones keep their sign where a 1 in their place is seen and no other such voxel."""
     import os
     import torch
     import ct_amd
@@ -955,6 +958,38 @@ def test_lds_forms_match_the_global_form(gpu, monkeypatch, store, nz, z0):
         x = np.arange(g.nx)[:, None] - g.x_pre
         y = np.arange(g.ny)[None, :] - g.y_pre
         assert np.all(volume()[x * x + y * y >= g.radius ** 2] == 0.5)
+
+
+@pytest.mark.parametrize("zpl", ["16", "32"])
+@pytest.mark.parametrize("nz,z0", [(2, 0), (10, 0), (11, 0), (21, 0), (22, 0), (53, 0), (54, 32), (60, 27)])
+def test_partial_runs_match_the_global_form(gpu, monkeypatch, zpl, nz, z0):
+    """Runs that the slab fills only in part step over its slices alone, or whole, by how many
+    they are (at either end of the slab): bit for bit the form that reads global memory voxel
+    by voxel, whatever the run length."""
+    import torch
+    import ct_amd
+    W, H, P = 60, 56, 9
+    g = ct_amd.geometry_grid(W, H, 1.5 * W, -2.0, 60, 52, nz)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    ctx.set_projections(np.linspace(0.0, 320.0, P), np.linspace(-9.0, 12.0, P))
+    img = torch.randn((P, H, W), generator=torch.Generator(device="cuda").manual_seed(nz), device="cuda")
+    entries = torch.empty(ctx.filtered_bytes("f32", P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, dtype=torch.float32, device="cuda")
+    ctx.layout_projections(img, P, "f32", entries, scales)
+
+    def volume():
+        v = torch.full((g.nx, g.ny, nz - z0), float("nan"), device="cuda")
+        ctx.backproject(entries, "f32", scales, 0, P, v, z0, nz - z0, False)
+        torch.cuda.synchronize()
+        return v.cpu().numpy()
+
+    monkeypatch.setenv("CTG_BP_ZPL", zpl)
+    got = volume()
+    monkeypatch.setenv("CTG_BP_PITCH", "65536,0")
+    ref = volume()
+    assert np.isfinite(ref).all() and np.any(ref != 0.0)
+    np.testing.assert_array_equal(got, ref)
 
 
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
