@@ -250,7 +250,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     static_assert(ZPL == kRowAnchor || ZPL == kRowAnchor / 2, "a run lies inside one row anchor block");
     const int zrun = a.z0 - a.zshift + zb;
     const float zw0 = (float)zrun - a.zpre;
-    const float zw1 = zw0 + (float)(ZPL - 1);
+    // The slices a step has to cover: the whole run, unless the slab holds so few of it that the
+    // masked form (by groups of four, about 1.5 times the time per slice) is cheaper on those:
+    // 72 slices in runs of 32 at 96^2 x 48 projections took 99 us with a whole last run of 8
+    // slices, 88 so.
+    const int valid = min(zlast, ZPL) - max(zfirst, 0);
+    const bool whole = valid * 3 > ZPL * 2;
+    const int kfirst = whole ? 0 : max(zfirst, 0), klast = whole ? ZPL - 1 : min(zlast, ZPL) - 1;
+    const float zwf = zw0 + (float)kfirst, zwl = zw0 + (float)klast;
     const int koff = ZPL == kRowAnchor ? 0 : (zrun & (kRowAnchor - 1));
     const float zwa = (float)(zrun - koff) - a.zpre;
 
@@ -282,8 +289,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
                 bad |= !(den > 0.0f);
                 const float U = a.fcd / den;
                 const float ui = t * U + a.upre;
-                const float va = fmaf(-(zw0 + g.z), U, a.vpre);
-                const float vb = fmaf(-(zw1 + g.z), U, a.vpre);
+                const float va = fmaf(-(zwf + g.z), U, a.vpre);
+                const float vb = fmaf(-(zwl + g.z), U, a.vpre);
                 umin = fminf(umin, ui); umax = fmaxf(umax, ui);
                 vmin = fminf(vmin, fminf(va, vb)); vmax = fmaxf(vmax, fmaxf(va, vb));
                 du += (c & 1) ? ui : -ui;
@@ -325,7 +332,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             const int fast = vs0 >= 0 ? 1 : 0;
             // no voxel of the tile and run can fail a window test (by more than either
             // expression's rounding), and no entry is clipped away
-            const bool in = fast && us0 >= 0 && umin - kBoxMargin >= a.ulo + a.upre &&
+            const bool in = whole && fast && us0 >= 0 && umin - kBoxMargin >= a.ulo + a.upre &&
                             umax + kBoxMargin <= fminf(a.uhi + a.upre, (float)(a.W - 1)) &&
                             vmin - kBoxMargin >= a.vpre - a.vhi &&
                             vmax + kBoxMargin <= fminf(a.vpre - a.vlo, (float)(a.H - 1));
@@ -394,8 +401,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             // 3 voxel by voxel from global memory
             int mode = kind == 1 ? 1 : 3;
             if (kind == 1 && !box_inside(bx)) {
-                const bool lane_full = !cv || ((zw0 + g.z) * U >= a.vlo && (zw1 + g.z) * U <= a.vhi);
-                if (!(box_fast(bx) && __all(lane_full))) mode = 2;
+                const bool lane_full = !cv || ((zw0 + g.z) * U >= a.vlo && (zwl + g.z) * U <= a.vhi);
+                if (!(whole && box_fast(bx) && __all(lane_full))) mode = 2;
                 else if (!cv) idle();
             }
             // The three forms follow one another, each under its own opaque condition: as
@@ -448,8 +455,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
                     if (!(v_of(lo) >= a.vlo)) ++lo;
                     if (!(v_of(hi) <= a.vhi)) --hi;
                 }
-                lo = max(lo, 0);
-                hi = min(hi, ZPL - 1);
+                lo = max(lo, kfirst);
+                hi = min(hi, klast);
                 const bool act = cv && lo <= hi && v_of(lo) >= a.vlo && v_of(hi) <= a.vhi;
                 if (!act) idle();
                 const T* tb = reinterpret_cast<const T*>(col);
@@ -766,7 +773,7 @@ int cached_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, i
     return cap;
 }
 
-// Strips and chunks of the tile numbering (tile_of).
+// Strips of the tile numbering (tile_of).
 void number_tiles(const ctg_geometry& g, BpArgs& a) {
     // blocks of 4 x 4 tiles; CTG_BP_BLOCK=n sets their edge, 0 takes single rows (tuning)
     int edge = 4;
@@ -791,6 +798,10 @@ void number_tiles(const ctg_geometry& g, BpArgs& a) {
     }
     a.nwork = a.before[a.nstrips];
     a.nidle = (unsigned)(a.ntx * a.nty) - a.nwork;
+}
+
+// Its chunks.
+void number_chunks(BpArgs& a) {
     const unsigned total = a.nwork * (unsigned)a.nzb;
     a.chunk = total / (8u * (unsigned)a.nzb);
     a.extra = total - a.chunk * 8u * (unsigned)a.nzb;
@@ -837,7 +848,7 @@ ctg_status launch_zpl(const BpLaunch& L, BpArgs a, hipStream_t st) {
     a.cap = cap;
     const size_t lds = (size_t)2 * cap * ebytes;
     if ((long long)a.ntx * a.nty * a.nzb > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
-    number_tiles(g, a);
+    number_chunks(a);
     const long long grid = 8ll * ((long long)a.nzb * a.per + ((long long)a.nidle * a.nzb + 7) / 8);
     if (grid > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
 #define CTG_BP_LAUNCH(E, DMA)                                                                           \
@@ -882,9 +893,15 @@ ctg_status launch_backproject(const BpLaunch& L, hipStream_t st) {
     BpArgs a = make_args(g, L.nproj, L.z0, L.nz, L.accumulate);
     a.ntx = (g.nx + kTX - 1) / kTX;
     a.nty = (g.ny + kTY - 1) / kTY;
-    // z per lane: 32 by default; CTG_BP_ZPL=16 selects the shorter run
+    number_tiles(g, a);
+    // Slices per lane: 32, but 16 where the working tiles are then still at most one per CU (256
+    // of them): every tile runs alone on its CU, so shorter ones end sooner (96^2 x 72 from 48
+    // projections: 88 us with 32, 75 with 16).  From there on both take the same (128^3: 95 and
+    // 86, 160^3: 89 and 89, 200^3: 187 and 185 us), and on a full chip 16 takes 15 % longer.
+    // CTG_BP_ZPL=16 or 32 overrides (tuning).
     const char* env = std::getenv("CTG_BP_ZPL");
-    const int zpl = (env && std::atoi(env) == 16) ? 16 : 32;
+    const long long short_runs = (long long)a.nwork * ((L.nz + (L.z0 & 15) + 15) / 16);
+    const int zpl = env ? (std::atoi(env) == 16 ? 16 : 32) : (short_runs <= 256 ? 16 : 32);
     return zpl == 16 ? launch_zpl<16>(L, a, st) : launch_zpl<32>(L, a, st);
 }
 
