@@ -89,6 +89,7 @@ SIGNATURES = {
     "ctg_preprocess": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_float, c_int32, c_int32, c_int32,
                                  c_void_p, c_void_p, c_void_p]),
     "ctg_feldkamp_weight": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p]),
+    "ctg_sum_squares": (c_int32, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     "ctg_filter_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
     "ctg_layout_projections": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p]),
     "ctg_layout_projections_noalloc": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p,
@@ -171,6 +172,9 @@ def device_info(device: int = 0) -> DeviceInfo:
     return info
 
 
+SUM_WORK = 1025  # CTG_SUM_WORK
+
+
 def _ptr(x):
     if x is None:
         return None
@@ -246,6 +250,10 @@ class Context:
 
     def feldkamp_weight(self, images, nproj, stream=0):
         check(self.lib.ctg_feldkamp_weight(self.handle, _ptr(images), nproj, c_void_p(stream)))
+
+    def sum_squares(self, x, n, work, stream=0):
+        """work[0] = sum of squares of the n floats x; work: SUM_WORK doubles on the device."""
+        check(self.lib.ctg_sum_squares(self.handle, _ptr(x), int(n), _ptr(work), c_void_p(stream)))
 
     def filter_rows(self, src, dst, rows, filt, stream=0):
         check(self.lib.ctg_filter_rows(self.handle, _ptr(src), _ptr(dst), int(rows), FILTER[filt],

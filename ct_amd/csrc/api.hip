@@ -503,6 +503,13 @@ ctg_status ctg_feldkamp_weight(ctg_context* ctx, float* d_images, int32_t nproj,
     return launch_feldkamp_weight(ctx->geom, d_images, nproj, (hipStream_t)stream);
 }
 
+ctg_status ctg_sum_squares(ctg_context* ctx, const float* d_x, int64_t n, double* d_work, void* stream) {
+    clear_error();
+    CTG_TRY(check_ctx(ctx));
+    if (n < 0 || !d_work || (n > 0 && !d_x)) return fail(CTG_ERROR_INVALID_ARGUMENT, "bad buffers");
+    return launch_sum_squares(d_x, (size_t)n, d_work, (hipStream_t)stream);
+}
+
 ctg_status ctg_filter_rows(ctg_context* ctx, const float* d_in, float* d_out, int64_t rows, ctg_filter filter,
                            void* stream) {
     clear_error();

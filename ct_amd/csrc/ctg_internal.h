@@ -194,6 +194,8 @@ ctg_status launch_phantom(const ctg_geometry& g, const double4* d_params, const 
                           int n_ell, int nproj, int p0, double photons, double full_scale,
                           uint64_t seed, uint16_t* d_img, float* d_lineint, DevBuf& ell_buf,
                           hipStream_t st);
+// work[0] = sum x[i]^2 in FP64; work holds CTG_SUM_WORK doubles.
+ctg_status launch_sum_squares(const float* d_x, size_t n, double* d_work, hipStream_t st);
 ctg_status launch_convert_volume(const ctg_geometry& g, const float* d_vol, int nz,
                                  ctg_index_order order, ctg_byte_order bo, void* d_out,
                                  hipStream_t st);

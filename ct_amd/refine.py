@@ -35,6 +35,7 @@ import time
 
 import torch
 
+from ._ctg import SUM_WORK
 from .autograd import ConeBeamOperator
 
 
@@ -42,8 +43,12 @@ class Interrupted(RuntimeError):
     """Raised by :func:`refine` when ``stop_after`` is reached (a simulated stop)."""
 
 
-def _sum_sq(t: torch.Tensor) -> float:
-    return float(torch.sum(t.double() * t.double()))
+def _sum_sq(t: torch.Tensor, op) -> float:
+    if not t.is_cuda:  # an operator on host tensors, as in the CPU tests of the checkpoint logic
+        return float(torch.sum(t.double() * t.double()))
+    work = torch.empty(SUM_WORK, dtype=torch.float64, device=t.device)
+    op.ctx.sum_squares(t, t.numel(), work, stream=torch.cuda.current_stream(t.device).cuda_stream)
+    return float(work[0])
 
 
 class SlabCheckpoint:
@@ -176,8 +181,8 @@ def refine(op: ConeBeamOperator, x0: torch.Tensor, measured: torch.Tensor, steps
             alpha, loss = mid[2], mid[3]
         else:
             ag = op.project(g)
-            alpha = _sum_sq(g) / _sum_sq(ag)
-            loss = 0.5 * _sum_sq(r)
+            alpha = _sum_sq(g, op) / _sum_sq(ag, op)
+            loss = 0.5 * _sum_sq(r, op)
             del ag
         del r
         sync()

@@ -172,6 +172,12 @@ ctg_status ctg_feldkamp_weight(ctg_context* ctx, float* d_images, int32_t nproj,
 ctg_status ctg_filter_rows(ctg_context* ctx, const float* d_in, float* d_out, int64_t rows,
                            ctg_filter filter, void* stream);
 
+/* Sum of squares of n floats in FP64, the norms of an iterative method's line search:
+ * d_work[0] = sum d_x[i]^2.  Every product is exact and the order of the additions is
+ * fixed.  d_work: device memory of CTG_SUM_WORK doubles. */
+#define CTG_SUM_WORK 1025
+ctg_status ctg_sum_squares(ctg_context* ctx, const float* d_x, int64_t n, double* d_work, void* stream);
+
 /* Row-major FP32 detector images -> backprojection layout in a store type, with
  * per-projection power-of-two scales in d_scales (may be null for F32 only; no
  * counterpart: the reference kept FP32). */

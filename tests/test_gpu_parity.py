@@ -992,6 +992,34 @@ def test_partial_runs_match_the_global_form(gpu, monkeypatch, zpl, nz, z0):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("n", [0, 1, 3, 255, 4097, 4194304 + 5, 20000003])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_sum_squares(gpu, n, offset):
+    """Exact products, FP64 sums: n additions of terms of one sign are within n 2^-53 of the
+    true sum, and far closer in partial sums; 1e-13 covers every n here.  An unaligned start
+    takes the scalar loads; infinite and NaN values come through."""
+    import torch
+    import ct_amd
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(8, 8, 40.0, 0.0, 4, 4, 4))
+    ctx.set_projections([0.0], [0.0])
+    x = torch.randn(n + offset, generator=torch.Generator(device="cuda").manual_seed(n + 1), device="cuda")[offset:]
+    work = torch.full((1025,), float("nan"), dtype=torch.float64, device="cuda")
+
+    def total():
+        ctx.sum_squares(x if n else 0, n, work)
+        torch.cuda.synchronize()
+        return float(work[0])
+
+    want = float((x.double() ** 2).sum())
+    assert abs(total() - want) <= 1e-13 * want
+    if n:
+        x[n // 2] = float("-inf")
+        assert total() == float("inf")
+        x[n - 1] = float("nan")
+        assert np.isnan(total())
+
+
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
                                         (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
 def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
