@@ -601,10 +601,8 @@ ctg_status ctg_forward_project(ctg_context* ctx, const float* d_volume, int32_t 
     if (!d_volume || (nproj > 0 && !d_proj)) return fail(CTG_ERROR_INVALID_ARGUMENT, "null buffers");
     if (nproj == 0) return CTG_OK;
     hipStream_t st = (hipStream_t)stream;
-    const size_t n = (size_t)nproj * ctx->geom.det_width * ctx->geom.det_height;
-    if (!accumulate) CTG_TRY(fill_u32(d_proj, 0u, n, st));
     return launch_forward_project(ctx->geom, ctx->proj_dev.as<float4>() + p0, ctx->proj_host.data() + p0, d_volume, z0,
-                                  nz, nproj, d_proj, ctx->fp_work, st);
+                                  nz, nproj, d_proj, ctx->fp_work, accumulate, st);
 }
 
 ctg_status ctg_fdk_backward(ctg_context* ctx, const float* d_grad_volume, int32_t z0, int32_t nz, int32_t p0,
@@ -618,10 +616,8 @@ ctg_status ctg_fdk_backward(ctg_context* ctx, const float* d_grad_volume, int32_
     if (nproj == 0) return CTG_OK;
     hipStream_t st = (hipStream_t)stream;
     const ctg_geometry& g = ctx->geom;
-    const size_t n = (size_t)nproj * g.det_width * g.det_height;
-    CTG_TRY(fill_u32(d_grad_lineint, 0u, n, st));
     CTG_TRY(launch_forward_project(g, ctx->proj_dev.as<float4>() + p0, ctx->proj_host.data() + p0, d_grad_volume, z0,
-                                   nz, nproj, d_grad_lineint, ctx->fp_work, st));
+                                   nz, nproj, d_grad_lineint, ctx->fp_work, 0, st));
     CTG_TRY(launch_filter_rows_only(ctx, d_grad_lineint, d_grad_lineint, (int64_t)nproj * g.det_height, filter, st));
     return launch_feldkamp_weight(g, d_grad_lineint, nproj, st);
 }

@@ -184,12 +184,13 @@ ctg_status launch_backproject_f64(const ctg_geometry& g, const double4* d_params
                                   int nproj, double* d_volume, int z0, int nz, hipStream_t st);
 
 // ---- project.hip
-// Adds the forward projection of the slab into d_proj (row-major nproj x H x W images).
+// Forward projection of the slab into d_proj (row-major nproj x H x W images), added to it or
+// in its place.
 // h_params: host copy of the projections' parameters (row bounds of the row-run
 // form; null selects the gather form); work: the context buffer for its column partials.
 ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params, const float4* h_params,
                                   const float* d_volume, int z0, int nz, int nproj, float* d_proj, DevBuf& work,
-                                  hipStream_t st);
+                                  int accumulate, hipStream_t st);
 ctg_status launch_phantom(const ctg_geometry& g, const double4* d_params, const double* h_ell,
                           int n_ell, int nproj, int p0, double photons, double full_scale,
                           uint64_t seed, uint16_t* d_img, float* d_lineint, DevBuf& ell_buf,

@@ -382,6 +382,7 @@ struct FpWin {
     int rbase;   // first row any voxel of the window can reach
     int span;    // rows per copy
     int stride;  // rows between copies
+    int first;   // 1: the workgroup's column of sums is written, 0: added to
 };
 
 // -------------------------------------------------------- entry-space projector
@@ -662,13 +663,13 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
         }
         return sum;
     };
-    for (int r = tid; r <= span; r += kGThreads) {
-        const int row = win.rbase + r;
-        if (row < 0 || row >= a.H) continue;
+    const int row0 = win.first ? 0 : max(win.rbase, 0), row1 = win.first ? a.H - 1 : min(win.rbase + span, a.H - 1);
+    for (int row = row0 + tid; row <= row1; row += kGThreads) {
+        const int r = row - win.rbase;
         const float4 e0 = entry(r), e1 = entry(r - 1);  // entries at rows v = row and v = row - 1
         const float own = ((e0.x - e0.y) - e0.z + e0.w) + (e1.z - e1.w);
         const float side = (e0.y - e0.w) + e1.w;
-        float2 o = col[row];
+        float2 o = win.first ? make_float2(0.0f, 0.0f) : col[row];
         o.x += own;
         o.y += side;
         col[row] = o;
@@ -720,9 +721,10 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
 // voxel read hits L2 (85 % of a 768^3 iteration with 60 projections per call).  At 512^3 x 360
 // projections of 512 x 512 (5.9e8 wave-updates inside the cylinder) it issues 1.07e10 VALU
 // instructions, 18 per update: 11 for the update, 2 for its candidate, 3 to end a run and
-// start the next (9.6 candidates per run), the rest to fill the list.  16.9 ms.  Twice the row
+// start the next (9.6 candidates per run), the rest to fill the list.  16.3 ms.  Twice the row
 // sums in LDS, |e| instead of max(e, 0) and runs of any length to 16 instead of powers of two
-// took 18.3 ms to that.  A form that added each voxel's two rows to LDS as it came (one 16-byte
+// took 18.3 ms to 16.9, column sums and images written instead of cleared and added to the rest
+// (at 4 waves per SIMD: 134 VGPRs, 6 too many without being told, cost 2 ms).  A form that added each voxel's two rows to LDS as it came (one 16-byte
 // read-modify-write per update, LDS-bound) took 24.8 ms; with its column-by-column order 1 %
 // of the voxel reads hit the L2, with fp_item's units 53 %.
 constexpr int kJ = 3;  // lateral slots per lane and round
@@ -785,7 +787,7 @@ __device__ inline bool fp_item(const FpArgs& a, int& c, int& p) {
 }
 
 template <int G>
-__global__ __launch_bounds__(kGThreads) void fp_rows_kernel(FpArgs a, FpWin win, const float4* __restrict__ pp,
+__global__ __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(4))) void fp_rows_kernel(FpArgs a, FpWin win, const float4* __restrict__ pp,
                                                             const float* __restrict__ vol,
                                                             float2* __restrict__ ps) {
     // column, U, w fu and the z interval relative to the run base (w = U^2 is recomputed
@@ -1142,21 +1144,21 @@ again:
         goto again;
     }
     float2* col = ps + ((size_t)p * a.W + c) * a.H;
-    for (int r = tid; r < span; r += kGThreads) {
-        const int row = win.rbase + r;
-        if (row < 0 || row >= a.H) continue;
-        const float2 s2 = acc_lds[r];
-        float2 o = col[row];
+    const int row0 = win.first ? 0 : max(win.rbase, 0), row1 = win.first ? a.H - 1 : min(win.rbase + span - 1, a.H - 1);
+    for (int row = row0 + tid; row <= row1; row += kGThreads) {
+        const int r = row - win.rbase;
+        const float2 s2 = r >= 0 && r < span ? acc_lds[r] : make_float2(0.0f, 0.0f);
+        float2 o = win.first ? make_float2(0.0f, 0.0f) : col[row];
         o.x = fmaf(0.5f, s2.x, o.x);
         o.y = fmaf(0.5f, s2.y, o.y);
         col[row] = o;
     }
 }
 
-// img[p][r][c] += ps[p][c][r].x + ps[p][c - 1][r].y: column-major partials into the
+// img[p][r][c] = or += ps[p][c][r].x + ps[p][c - 1][r].y: column-major partials into the
 // row-major images, through a 32 x 33 tile per (row, column) block.
 __global__ __launch_bounds__(256) void fp_finish_kernel(const float2* __restrict__ ps, int W, int H,
-                                                        float* __restrict__ img) {
+                                                        int accumulate, float* __restrict__ img) {
     __shared__ float2 tile[33][33];  // [column - c0 + 1][row - r0]
     const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
     const size_t p = blockIdx.z;
@@ -1168,7 +1170,10 @@ __global__ __launch_bounds__(256) void fp_finish_kernel(const float2* __restrict
     __syncthreads();
     for (int i = threadIdx.x >> 5; i < 32; i += 8) {
         const int r = r0 + i, cc = c0 + tl;
-        if (cc < W && r < H) img[(p * H + r) * W + cc] += tile[tl + 1][i].x + tile[tl][i].y;
+        if (cc < W && r < H) {
+            float* o = img + (p * H + r) * W + cc;
+            *o = (accumulate ? *o : 0.0f) + (tile[tl + 1][i].x + tile[tl][i].y);
+        }
     }
 }
 
@@ -1369,8 +1374,10 @@ void window_rows(const ctg_geometry& g, double hmin, double hmax, double Umin, d
 
 ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params, const float4* h_params,
                                   const float* d_volume, int z0, int nz, int nproj, float* d_proj, DevBuf& work,
-                                  hipStream_t st) {
-    if (nz <= 0 || nproj <= 0) return CTG_OK;
+                                  int accumulate, hipStream_t st) {
+    const size_t pixels = (size_t)nproj * g.det_width * g.det_height;
+    if (nproj <= 0) return CTG_OK;
+    if (nz <= 0) return accumulate ? CTG_OK : fill_u32(d_proj, 0u, pixels, st);
     FpArgs a{};
     a.W = g.det_width; a.H = g.det_height; a.nx = g.nx; a.ny = g.ny; a.nzs = nz; a.z0 = z0; a.nproj = nproj;
     a.xpre = g.x_pre; a.ypre = g.y_pre; a.zpre = g.z_pre; a.upre = g.u_pre; a.vpre = g.v_pre;
@@ -1426,10 +1433,10 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
         }
     }
     if (G > 0) {
-        const size_t cells = (size_t)nproj * a.W * a.H;
-        CTG_TRY(work.reserve(cells * sizeof(float2)));
+        // the first window writes the column sums and fp_finish_kernel the images, so neither is
+        // cleared first
+        CTG_TRY(work.reserve(pixels * sizeof(float2)));
         float2* ps = work.as<float2>();
-        CTG_TRY(fill_u32(ps, 0u, cells * 2, st));
         bool entries = false;
         const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj) + 7) / 8) * 8 * kPBlock * kCBlock;
         if (blocks > 0x7fffffffull) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
@@ -1442,6 +1449,7 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
             window_rows(g, hmin, hmax, Umin, Umax, win.wz0, 64 * G, win.rbase, win.span);
             entries = win.wz0 + 64 * G >= z0 + nz && win.span <= kEntryMaxSpan;
             win.stride = (win.span + 15) & ~15;
+            win.first = 1;
             const size_t lds = sizeof(float4) * 2 * kGWaves * (size_t)win.stride;
             if (entries) {
                 if (G == 2) hipLaunchKernelGGL(fp_entry_kernel<2>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
@@ -1458,6 +1466,7 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
                 win.wz0 = w0;
                 window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * G, win.rbase, win.span);
                 win.stride = (win.span + 1) & ~1;
+                win.first = s == 0 && w0 <= z0;
                 const size_t lds = sizeof(float2) * 2 * kGWaves * (size_t)win.stride;
                 if (G == 4) hipLaunchKernelGGL(fp_rows_kernel<4>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
                 else if (G == 3) hipLaunchKernelGGL(fp_rows_kernel<3>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
@@ -1467,11 +1476,12 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
             }
         }
         dim3 fg((unsigned)((a.W + 31) / 32), (unsigned)((a.H + 31) / 32), (unsigned)nproj);
-        hipLaunchKernelGGL(fp_finish_kernel, fg, dim3(256), 0, st, ps, a.W, a.H, d_proj);
+        hipLaunchKernelGGL(fp_finish_kernel, fg, dim3(256), 0, st, ps, a.W, a.H, accumulate, d_proj);
         CTG_HIP(hipGetLastError());
         return CTG_OK;
     }
 
+    if (!accumulate) CTG_TRY(fill_u32(d_proj, 0u, pixels, st));
     const size_t lds = sizeof(float) * (size_t)(2 * kGWaves) * (a.H + 4);
     // the candidate records hold z relative to the launch's run base in kFpZBits bits
     for (int s = 0; s < nz; s += kFpMaxSlab) {

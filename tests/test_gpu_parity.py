@@ -1020,6 +1020,40 @@ def test_sum_squares(gpu, n, offset):
         assert np.isnan(total())
 
 
+@pytest.mark.parametrize("n,nz,gather", [(40, 100, False), (170, 300, False), (40, 100, True)])
+def test_forward_projection_writes_every_pixel(gpu, monkeypatch, n, nz, gather):
+    """Without accumulate every pixel is written whatever the images and the context's column
+    sums held before (rows outside a window's reach and columns without a voxel too), with
+    accumulate the same values are added; an empty slab clears, or leaves, the images."""
+    import torch
+    import ct_amd
+    if gather:
+        monkeypatch.setenv("CTG_FP_GATHER", "1")
+    g = ct_amd.geometry_grid(2 * n, 2 * nz, 6.0 * n, 0.0, n, n, nz)
+    x = torch.randn((n, n, nz), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+
+    def make(dirty):
+        ctx = ct_amd.Context(0)
+        ctx.set_geometry(g)
+        ctx.set_projections([0.0, 50.0, 140.0], [0.0, 3.0, -3.0])
+        y = torch.full((3, g.det_height, g.det_width), float("nan"), device="cuda")
+        if dirty:
+            ctx.forward_project(torch.full_like(x, 7.0), 0, nz, 0, 3, torch.empty_like(y))
+        ctx.forward_project(x, 0, nz, 0, 3, y)
+        torch.cuda.synchronize()
+        return ctx, y
+
+    (_, a), (ctx, b) = make(False), make(True)
+    assert torch.isfinite(a).all() and torch.equal(a, b) and (a == 0).any() and (a != 0).any()
+    ctx.forward_project(x, 0, nz, 0, 3, b, accumulate=True)
+    ctx.forward_project(x, 5, 0, 0, 3, a, accumulate=True)
+    torch.cuda.synchronize()
+    assert torch.equal(b, 2 * a)
+    ctx.forward_project(x, 5, 0, 0, 3, b)
+    torch.cuda.synchronize()
+    assert (b == 0).all()
+
+
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
                                         (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
 def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
