@@ -1054,6 +1054,30 @@ def test_forward_projection_writes_every_pixel(gpu, monkeypatch, n, nz, gather):
     assert (b == 0).all()
 
 
+@pytest.mark.parametrize("store", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("W,H", [(64, 64), (65, 63), (63, 66), (130, 129), (2, 128)])
+@pytest.mark.parametrize("shift", [0, 8])
+def test_layout_tile_sizes_agree(gpu, store, W, H, shift):
+    """Many images are laid out in tiles of 64, one in tiles of 32: the same bytes, at even and
+    odd heights, partial tiles, and in a buffer that is not 16-byte aligned."""
+    import torch
+    import ct_amd
+    P = 1024
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, H, 5.0 * W, 0.0, 4, 4, 4))
+    ctx.set_projections(np.zeros(P), None)
+    img = torch.randn((P, H, W), generator=torch.Generator(device="cuda").manual_seed(W), device="cuda")
+    n = ctx.filtered_bytes(store, 1)
+    entries = torch.zeros(n * P + 8, dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, device="cuda")
+    ctx.layout_projections(img, P, store, entries[shift:], scales)
+    one, sc = torch.zeros(n, dtype=torch.uint8, device="cuda"), torch.empty(1, device="cuda")
+    for p in (0, 1, 511, P - 1):
+        ctx.layout_projections(img[p], 1, store, one, sc)
+        torch.cuda.synchronize()
+        assert torch.equal(entries[shift + p * n:shift + (p + 1) * n], one) and scales[p] == sc[0]
+
+
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
                                         (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
 def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
