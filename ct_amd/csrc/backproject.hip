@@ -55,6 +55,7 @@ namespace bp_detail {
 
 constexpr int kTX = 16, kTY = 16, kThreads = 256, kWaves = kThreads / 64;
 constexpr int kMaxTileBytes = 36 * 1024;  // per LDS buffer (two buffers per workgroup)
+constexpr int kStaticLds = 4096;
 // Detector pixels added around a footprint box's corner bounds: the corner and voxel
 // expressions round differently by about 1e-4 pixel at most.
 constexpr float kBoxMargin = 0.05f;
@@ -70,6 +71,7 @@ struct BpArgs {
     int dma16;               // 8-byte entries staged with 16-byte DMA (H even: rows start even)
     int pitch_mod, pitch_rem;  // LDS column pitch = rows rounded up to pitch_rem mod pitch_mod (a power of two)
     int pitch_adapt;           // per box, -pitch_rem mod pitch_mod where the footprint slants the other way
+    int pitch_alt;             // remainder for boxes that do not fit with pitch_rem (pitch_rem: none)
     // numbering of the tiles (tile_of)
     int strip_h, nstrips, blk;  // tile rows per strip, tile columns per block
     unsigned nwork, nidle;     // tiles of one layer inside / outside the strips' ranges
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     using T = typename E::T;
     const T* __restrict__ proj = reinterpret_cast<const T*>(proj_raw);
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int4 boxes[2][64];
+    __shared__ int4 boxes[2][64];  // with params kStaticLds bytes
     // per projection: sin, cos, height, and the entry scale in w (written with the boxes)
     __shared__ float4 params[2][64];
 
@@ -317,16 +319,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             // two, so a mask: a division here would raise the kernel's register peak), so
             // that neighbouring detector columns start in different LDS bank groups
             const int wr = (DMA == 16 && E::kBytes == 8) ? (nr + 1) & ~1 : nr;
-            int pitch = wr + ((a.pitch_rem - wr) & (a.pitch_mod - 1));
             // A 16-lane row of voxels reads entries whose column and row both drift along
             // x.  With the pitch at +1 mod 16 a lane's bank group is column + row, and two
             // lanes whose column step is undone by a row step share one; where the column
             // and row drift in opposite directions the pitch -1 mod 16 (row - column)
             // avoids that.  Taken only where the box still fits the buffer.
-            if (a.pitch_adapt && du * dv < 0.0f) {
-                const int pm = wr + ((a.pitch_mod - a.pitch_rem - wr) & (a.pitch_mod - 1));
-                if (nc * pm <= a.cap) pitch = pm;
-            }
+            const bool minus = a.pitch_adapt && du * dv < 0.0f;
+            auto pitch_of = [&](int rem) {
+                const int p = wr + ((rem - wr) & (a.pitch_mod - 1));
+                const int m = wr + ((a.pitch_mod - rem - wr) & (a.pitch_mod - 1));
+                return minus && nc * m <= a.cap ? m : p;
+            };
+            int pitch = pitch_of(a.pitch_rem);
+            if (nc * pitch > a.cap) pitch = pitch_of(a.pitch_alt);
             b.x = us; b.y = vs; b.w = nr | (pitch << 16);
             // the fused vIndex of the fast path may round a hair below 0 at the top edge
             const int fast = vs0 >= 0 ? 1 : 0;
@@ -692,13 +697,14 @@ bool tile_in_cylinder(const ctg_geometry& g, int tx, int ty) {
 // Largest footprint box (entries) over a sample of tiles and projections, with the
 // same construction as box_for on the device.  Boxes that exceed the resulting
 // capacity at run time take the global-memory path, so sampling only affects speed.
-int sample_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, int nz, int zpl, int dma16,
-                   int pmod, int prem) {
+// x: with the column pitch at prem mod pmod, y: at palt.
+int2 sample_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, int nz, int zpl, int dma16,
+                    int pmod, int prem, int palt) {
     const int ntx = (g.nx + kTX - 1) / kTX, nty = (g.ny + kTY - 1) / kTY, nzb = (nz + zpl - 1) / zpl;
     // about 16 projections: boxes change slowly with the angle, and the capacity keeps a
     // margin above the largest sampled box
     const int pstep = std::max(1, nproj / 16);
-    int best = 0;
+    int2 best = make_int2(0, 0);
     const int zblocks[3] = {0, nzb / 2, nzb - 1};
     for (int zi = 0; zi < 3; ++zi) {
         const int zb = zblocks[zi] * zpl;
@@ -736,8 +742,8 @@ int sample_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, i
                     if (ue >= us && ve >= vs) {
                         const int nr = ve - vs + 1;
                         const int wr = dma16 ? (nr + 1) & ~1 : nr;
-                        const int pitch = wr + ((prem - wr) & (pmod - 1));
-                        best = std::max(best, (ue - us + 1) * pitch);
+                        best.x = std::max(best.x, (ue - us + 1) * (wr + ((prem - wr) & (pmod - 1))));
+                        best.y = std::max(best.y, (ue - us + 1) * (wr + ((palt - wr) & (pmod - 1))));
                     }
                 }
             }
@@ -751,23 +757,23 @@ int sample_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, i
 // sampling once.  The key hashes the geometry, the projection parameters and the slab;
 // a collision can only mis-size the LDS tile, which costs speed, not correctness
 // (boxes beyond the capacity read global memory).
-int cached_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, int nz, int zpl, int dma16, int pmod,
-                   int prem) {
+int2 cached_max_box(const ctg_geometry& g, const float4* hp, int nproj, int z0, int nz, int zpl, int dma16, int pmod,
+                    int prem, int palt) {
     uint64_t h = 1469598103934665603ull;
     auto mix = [&](const void* p, size_t n) {
         const unsigned char* b = static_cast<const unsigned char*>(p);
         for (size_t i = 0; i < n; ++i) h = (h ^ b[i]) * 1099511628211ull;
     };
-    const int keys[7] = {nproj, z0, nz, zpl, dma16, pmod, prem};
+    const int keys[8] = {nproj, z0, nz, zpl, dma16, pmod, prem, palt};
     mix(&g, sizeof(g));
     mix(keys, sizeof(keys));
     mix(hp, sizeof(float4) * (size_t)nproj);
-    struct Entry { uint64_t key; int cap; bool used; };
+    struct Entry { uint64_t key; int2 cap; bool used; };
     static thread_local Entry cache[16] = {};
     static thread_local int next = 0;
     for (const Entry& e : cache)
         if (e.used && e.key == h) return e.cap;
-    const int cap = sample_max_box(g, hp, nproj, z0, nz, zpl, dma16, pmod, prem);
+    const int2 cap = sample_max_box(g, hp, nproj, z0, nz, zpl, dma16, pmod, prem, palt);
     cache[next] = {h, cap, true};
     next = (next + 1) % 16;
     return cap;
@@ -839,12 +845,21 @@ ctg_status launch_zpl(const BpLaunch& L, BpArgs a, hipStream_t st) {
             a.pitch_rem = r % m;
         }
     }
-    int cap = L.h_params ? cached_max_box(g, L.h_params, L.nproj, L.z0 - a.zshift, L.nz + a.zshift, ZPL, a.dma16,
-                                          a.pitch_mod, a.pitch_rem)
-                         : 0;
-    cap = cap + cap / 32 + 16;
-    cap = std::min(cap, kMaxTileBytes / ebytes);
-    cap &= ~7;  // keeps the second buffer and every column start 16-byte aligned
+    // Boxes that do not fit with the pitch at 1 mod 16 (1.11 passes per LDS read on average) may
+    // take 11 mod 16 (1.21 passes, up to 6 rows less on a column); the buffers are sized for that
+    // where it lets more workgroups into a CU's 160 KB.  512^3 x 360 in batches of 64, FP32: 3
+    // workgroups and 11.3 ms with 1, 4 and 10.0 with 11; 1024^3 x 720, where both leave 3: 164.3
+    // and 166.7 ms.
+    a.pitch_alt = a.pitch_mod == 16 && a.pitch_rem == 1 ? 11 : a.pitch_rem;
+    const int2 most = L.h_params ? cached_max_box(g, L.h_params, L.nproj, L.z0 - a.zshift, L.nz + a.zshift, ZPL,
+                                                  a.dma16, a.pitch_mod, a.pitch_rem, a.pitch_alt)
+                                 : make_int2(0, 0);
+    // keeps the second buffer and every column start 16-byte aligned
+    auto capacity = [&](int n) { return std::min(n + n / 32 + 16, kMaxTileBytes / ebytes) & ~7; };
+    auto per_cu = [&](int n) { return std::min((160 * 1024) / (2 * capacity(n) * ebytes + kStaticLds), ebytes == 16 ? EF32::kMinWaves : EF16::kMinWaves); };
+    const bool tight = per_cu(most.y) > per_cu(most.x);
+    if (!tight) a.pitch_alt = a.pitch_rem;
+    const int cap = capacity(tight ? most.y : most.x);
     a.cap = cap;
     const size_t lds = (size_t)2 * cap * ebytes;
     if ((long long)a.ntx * a.nty * a.nzb > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");

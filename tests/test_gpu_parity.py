@@ -1078,6 +1078,36 @@ def test_layout_tile_sizes_agree(gpu, store, W, H, shift):
         assert torch.equal(entries[shift + p * n:shift + (p + 1) * n], one) and scales[p] == sc[0]
 
 
+@pytest.mark.parametrize("fcd", [450.0, 700.0, 1500.0])
+@pytest.mark.parametrize("store", ["f32", "bf16"])
+def test_tight_column_pitch_keeps_the_volume(gpu, monkeypatch, fcd, store):
+    """Boxes that only fit with the tighter LDS column pitch, from a short to a long source
+    distance (more and fewer rows per box, footprints slanting either way): the same volume,
+    bit for bit, as with a fixed pitch and from global memory."""
+    import torch
+    import ct_amd
+    W, H, P, n = 150, 160, 40, 128
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, H, fcd, 3.0, n, n, n))
+    ctx.set_projections(np.linspace(0.0, 351.0, P), np.linspace(-6.0, 6.0, P))
+    img = torch.randn((P, H, W), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+    entries = torch.empty(ctx.filtered_bytes(store, P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, device="cuda")
+    ctx.layout_projections(img, P, store, entries, scales)
+
+    def volume():
+        v = torch.empty((n, n, n), device="cuda")
+        ctx.backproject(entries, store, scales, 0, P, v, 0, n, False)
+        torch.cuda.synchronize()
+        return v
+
+    got = volume()
+    assert (got != 0).any()
+    for pitch in ("16,11", "16,3", "65536,0"):
+        monkeypatch.setenv("CTG_BP_PITCH", pitch)
+        assert torch.equal(volume(), got), pitch
+
+
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
                                         (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
 def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
