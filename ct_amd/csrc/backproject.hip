@@ -56,6 +56,9 @@ namespace bp_detail {
 constexpr int kTX = 16, kTY = 16, kThreads = 256, kWaves = kThreads / 64;
 constexpr int kMaxTileBytes = 36 * 1024;  // per LDS buffer (two buffers per workgroup)
 constexpr int kStaticLds = 4096;
+// LDS reads per software-pipeline group: with 8-byte entries 4 takes 133.5 ms at 1024^3 x 720
+// where 2 takes 134.5 (both fit 96 VGPRs), with FP32 ones 4 is as much as fits.
+constexpr int kGrp = 4;
 // Detector pixels added around a footprint box's corner bounds: the corner and voxel
 // expressions round differently by about 1e-4 pixel at most.
 constexpr float kBoxMargin = 0.05f;
@@ -140,7 +143,6 @@ struct EF32 {
     using T = float4;
     static constexpr int kBytes = 16;
     static constexpr int kMinWaves = 4;  // 127 VGPRs; the LDS may allow only 3
-    static constexpr int kGrp = 4;       // LDS reads per software-pipeline group
     __device__ static float eval(const T& e, float fu, float fv) {
         return fmaf(fv, fmaf(fu, e.w, e.z), fmaf(fu, e.y, e.x));
     }
@@ -149,7 +151,6 @@ struct EF16 {
     using T = uint2;
     static constexpr int kBytes = 8;
     static constexpr int kMinWaves = 5;  // VALU-bound: 5 waves per SIMD (at most 96 VGPRs)
-    static constexpr int kGrp = 2;       // (groups of 4 need more registers: measured slower)
     __device__ static float lo(uint32_t e) { return __half2float(__ushort_as_half((unsigned short)(e & 0xffffu))); }
     __device__ static float hi(uint32_t e) { return __half2float(__ushort_as_half((unsigned short)(e >> 16))); }
     __device__ static float eval(const T& e, float fu, float fv) {
@@ -160,7 +161,6 @@ struct EBF16 {
     using T = uint2;
     static constexpr int kBytes = 8;
     static constexpr int kMinWaves = 5;
-    static constexpr int kGrp = 2;
     __device__ static float lo(uint32_t e) { return __uint_as_float(e << 16); }
     __device__ static float hi(uint32_t e) { return __uint_as_float(e & 0xffff0000u); }
     __device__ static float eval(const T& e, float fu, float fv) {
@@ -419,7 +419,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
                 // issued before the arithmetic of group g, and scheduling barriers
                 // keep the compiler from trading those in-flight reads for hoisted
                 // row-index arithmetic
-                constexpr int kGrp = E::kGrp;
                 T e[2][kGrp];
                 float fv[2][kGrp];
                 auto fetch = [&](int g0, int slot) {
