@@ -44,10 +44,13 @@ class Interrupted(RuntimeError):
 
 
 def _sum_sq(t: torch.Tensor, op) -> float:
-    if not t.is_cuda:  # an operator on host tensors, as in the CPU tests of the checkpoint logic
+    ctx = getattr(op, "ctx", None)
+    # other operators: host tensors, as in the CPU tests of the checkpoint logic, or their own
+    if ctx is None or not t.is_cuda or t.dtype != torch.float32:
         return float(torch.sum(t.double() * t.double()))
+    t = t.contiguous()
     work = torch.empty(SUM_WORK, dtype=torch.float64, device=t.device)
-    op.ctx.sum_squares(t, t.numel(), work, stream=torch.cuda.current_stream(t.device).cuda_stream)
+    ctx.sum_squares(t, t.numel(), work, stream=torch.cuda.current_stream(t.device).cuda_stream)
     return float(work[0])
 
 

@@ -1108,6 +1108,27 @@ def test_tight_column_pitch_keeps_the_volume(gpu, monkeypatch, fcd, store):
         assert torch.equal(volume(), got), pitch
 
 
+def test_line_search_norm_of_any_operator(gpu):
+    """The norm of a refinement step: strided tensors through the kernel, operators without a
+    context and other types through torch, all the same value (1e-13, as above)."""
+    import torch
+    import ct_amd
+    from ct_amd.refine import _sum_sq
+
+    class Op:
+        pass
+
+    bare, op = Op(), Op()
+    op.ctx = ct_amd.Context(0)
+    op.ctx.set_geometry(ct_amd.geometry_grid(8, 8, 40.0, 0.0, 4, 4, 4))
+    op.ctx.set_projections([0.0], [0.0])
+    x = torch.randn((30, 40, 50), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    for t in (x, x[:, ::3, 1:], x.transpose(0, 2), x.double(), x.cpu()):
+        want = float((t.double() ** 2).sum())
+        for o in (bare, op):
+            assert abs(_sum_sq(t, o) - want) <= 1e-13 * want
+
+
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
                                         (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
 def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
