@@ -70,6 +70,7 @@ struct BpArgs {
     float xpre, ypre, zpre, upre, vpre;
     float r2, fcd, uoff, ulo, uhi, vlo, vhi;
     int nproj, ntx, nty, nzb, cap, accumulate, vec4;
+    int resume;              // the sums go on from the volume's values
     int zshift;              // z0 mod ZPL: runs start at grid z multiples of ZPL, zshift voxels before the slab
     int dma16;               // 8-byte entries staged with 16-byte DMA (H even: rows start even)
     int pitch_mod, pitch_rem;  // LDS column pitch = rows rounded up to pitch_rem mod pitch_mod (a power of two)
@@ -266,6 +267,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     float acc[ZPL];
 #pragma unroll
     for (int k = 0; k < ZPL; ++k) acc[k] = 0.0f;
+    float* const col = vol + ((size_t)xi * a.ny + yi) * a.nzs;
+    const bool whole_vec = a.vec4 && zfirst <= 0 && zlast >= ZPL;
+    if (a.resume && colvol) {
+        // the sums of the launch before
+        if (whole_vec) {
+            const float4* s4 = reinterpret_cast<const float4*>(col + zb);
+#pragma unroll
+            for (int k = 0; k < ZPL; k += 4) {
+                const float4 v = s4[k >> 2];
+                acc[k] = v.x; acc[k + 1] = v.y; acc[k + 2] = v.z; acc[k + 3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < ZPL; ++k)
+                if (k >= zfirst && k < zlast) acc[k] = col[zb - a.zshift + k];
+        }
+    }
 
     // nearest point of the tile's xy rectangle to the axis
     const float ndx = cxa > 0.0f ? cxa : (cxb < 0.0f ? cxb : 0.0f);
@@ -585,8 +603,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
         for (int k = 0; k < ZPL; ++k) acc[k] = 0.0f;
     }
     if (colvol) {
-        float* col = vol + ((size_t)xi * a.ny + yi) * a.nzs;
-        if (a.vec4 && zfirst <= 0 && zlast >= ZPL) {
+        if (whole_vec) {
             float4* d4 = reinterpret_cast<float4*>(col + zb);
 #pragma unroll
             for (int k = 0; k < ZPL; k += 4) {
@@ -916,7 +933,27 @@ ctg_status launch_backproject(const BpLaunch& L, hipStream_t st) {
     const char* env = std::getenv("CTG_BP_ZPL");
     const long long short_runs = (long long)a.nwork * ((L.nz + (L.z0 & 15) + 15) / 16);
     const int zpl = env ? (std::atoi(env) == 16 ? 16 : 32) : (short_runs <= 256 ? 16 : 32);
-    return zpl == 16 ? launch_zpl<16>(L, a, st) : launch_zpl<32>(L, a, st);
+    // The tiles that run at one time are spread over all projections of the launch, so a large
+    // scan's entries pass through the Infinity Cache without being met again.  Launches of about
+    // 240 projections that go on from each other's sums (the same additions in the same order)
+    // keep to fewer images at a time: 1024^3 x 720 162.0 -> 160.1 ms (FP16 131.2 -> 129.1), 768^3
+    // x 720 72.8 -> 71.4, 512^3 x 1440 44.2 -> 42.6, though each writes and reads the volume;
+    // 512^3 x 720 does not change.  At least 8192 tiles, so that a launch's last ones are few, and
+    // not where the sums are to be added to the volume.
+    const bool large = (long long)a.nwork * ((L.nz + (L.z0 & 31) + 31) / 32) >= 8192;
+    const int parts = large && !L.accumulate ? std::max(1, L.nproj / 240) : 1;
+    const int step = std::max(1, (L.nproj + parts - 1) / parts);
+    for (int p = 0; p < std::max(L.nproj, 1); p += step) {
+        BpLaunch part = L;
+        part.nproj = a.nproj = std::min(step, L.nproj - p);
+        part.d_params = L.d_params + p;
+        if (L.h_params) part.h_params = L.h_params + p;
+        if (L.d_scales) part.d_scales = L.d_scales + p;
+        part.d_filtered = (const char*)L.d_filtered + (size_t)p * (size_t)img_bytes;
+        a.resume = p > 0;
+        CTG_TRY(zpl == 16 ? launch_zpl<16>(part, a, st) : launch_zpl<32>(part, a, st));
+    }
+    return CTG_OK;
 }
 
 ctg_status launch_backproject_f64(const ctg_geometry& g, const double4* d_params, const double* d_rows,

@@ -1129,6 +1129,29 @@ def test_line_search_norm_of_any_operator(gpu):
             assert abs(_sum_sq(t, o) - want) <= 1e-13 * want
 
 
+@pytest.mark.parametrize("nz,P,store", [(352, 480, "f32"), (351, 723, "f32"), (351, 481, "f16")])
+def test_large_scans_run_in_parts(gpu, nz, P, store):
+    """A large volume from many projections takes several launches that go on from each other's
+    sums; added to a cleared volume it takes one.  The same bits, with whole and with partial
+    runs of slices, and in a volume that held NaN before."""
+    import torch
+    import ct_amd
+    n = 512
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(520, 60, 2600.0, 0.0, n, n, nz))
+    ctx.set_projections(np.linspace(0.0, 359.0, P), np.linspace(-150.0, 150.0, P))
+    img = torch.randn((P, 60, 520), generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
+    entries = torch.empty(ctx.filtered_bytes(store, P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, device="cuda")
+    ctx.layout_projections(img, P, store, entries, scales)
+    v = torch.full((n, n, nz), float("nan"), device="cuda")
+    ctx.backproject(entries, store, scales, 0, P, v, 0, nz, False)
+    w = torch.zeros((n, n, nz), device="cuda")
+    ctx.backproject(entries, store, scales, 0, P, w, 0, nz, True)
+    torch.cuda.synchronize()
+    assert (w != 0).any() and torch.equal(v, w)
+
+
 @pytest.mark.parametrize("nx,ny,nz,W", [(1, 1, 1, 40), (16, 16, 33, 40), (300, 17, 65, 400), (17, 300, 1, 400),
                                         (129, 193, 40, 150), (24, 4200, 3, 5000), (200, 200, 300, 60)])
 def test_backprojection_covers_every_tile(gpu, nx, ny, nz, W):
