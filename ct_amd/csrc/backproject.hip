@@ -35,7 +35,7 @@
 //    footprints in its own L2, with an equal part of every layer (tile_of).
 //
 // What bounds it (1024^3 x 720 x 1024^2, MI355X): with FP32 entries the traffic of boxes that
-// miss L2 (747 GB per launch, 4.6 TB/s; 137 ms instead of 162 when every staged line hits),
+// miss L2 (658 GB per backprojection, 4.1 TB/s; 137 ms instead of 162 when every line hits),
 // then the LDS (a ds_read_b128 takes 4.8 cycles per wave and CU, a staging DMA instruction
 // 17 whatever its lane mask); with 8-byte entries VALU issue (116 of 133 ms remain without
 // any staging).  Accumulators updated in place, three forms per step and tests left out where
