@@ -197,7 +197,7 @@ def refine(op: ConeBeamOperator, x0: torch.Tensor, measured: torch.Tensor, steps
         t1 = time.perf_counter()
         for s in range(first, len(slabs)):
             z0, nz = slabs[s]
-            x[:, :, z0:z0 + nz] -= alpha * g[:, :, z0:z0 + nz]
+            x[:, :, z0:z0 + nz].sub_(g[:, :, z0:z0 + nz], alpha=alpha)
             if ckpt:
                 tc = time.perf_counter()
                 ck.write_next_slab(s, x[:, :, z0:z0 + nz])
