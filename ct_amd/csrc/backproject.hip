@@ -55,7 +55,7 @@ namespace bp_detail {
 
 constexpr int kTX = 16, kTY = 16, kThreads = 256, kWaves = kThreads / 64;
 constexpr int kMaxTileBytes = 36 * 1024;  // per LDS buffer (two buffers per workgroup)
-constexpr int kStaticLds = 4096;
+constexpr int kStaticLds = 4112;
 // LDS reads per software-pipeline group: with 8-byte entries 4 takes 133.5 ms at 1024^3 x 720
 // where 2 takes 134.5 (both fit 96 VGPRs), with FP32 ones 4 is as much as fits.
 constexpr int kGrp = 4;
@@ -222,9 +222,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     using T = typename E::T;
     const T* __restrict__ proj = reinterpret_cast<const T*>(proj_raw);
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int4 boxes[2][64];  // with params kStaticLds bytes
+    __shared__ int4 boxes[2][64];  // with params and zero_entry kStaticLds bytes
     // per projection: sin, cos, height, and the entry scale in w (written with the boxes)
     __shared__ float4 params[2][64];
+    __shared__ float4 zero_entry;  // what columns that add nothing read
 
     int zbi, tx, ty;
     if (!tile_of(a, zbi, tx, ty)) return;
@@ -414,11 +415,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             float Ue = U, we = w, fue = fu, vAe = vA;
             const char* tile_b = reinterpret_cast<const char*>(tile) - (us * pitch + vs) * E::kBytes;
             const char* col = tile_b + __mul24(u0, pitch * E::kBytes);
-            // a column that adds nothing reads the box's first entry with zero weight
+            // a column that adds nothing reads an entry of zeros for every slice, with zero weight
+            // (not an entry of the box, which may be infinite or NaN, and so its product with 0)
             auto idle = [&]() {
                 Ue = we = fue = 0.0f;
                 vAe = (float)vs;
-                col = reinterpret_cast<const char*>(tile) - vs * E::kBytes;
+                col = reinterpret_cast<const char*>(&zero_entry) - vs * E::kBytes;
             };
             // how the step runs: 1 unmasked from LDS, 2 masked by groups of slices from LDS,
             // 3 voxel by voxel from global memory
@@ -551,6 +553,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             params[slot][tid] = g;
         };
         if (tid < 64) fill_batch(0, tid);
+        if (tid == 0) zero_entry = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         __syncthreads();
         auto buffer = [&](int p) { return smem + (size_t)(p & 1) * a.cap * E::kBytes; };
         if (a.nproj > 0) {

@@ -1224,3 +1224,39 @@ def test_row_filter_transform_lengths_match_oracle(gpu, oracle, W):
     torch.cuda.synchronize()
     m = np.abs(ent[..., 0].cpu().numpy()).reshape(P, -1).max(axis=1)
     np.testing.assert_array_equal(scales.cpu().numpy(), np.ldexp(1.0, np.frexp(m)[1]).astype(np.float32))
+
+
+@pytest.mark.parametrize("store", ["f32", "f16"])
+@pytest.mark.parametrize("nz,z0", [(33, 0), (100, 17)])
+def test_lds_forms_keep_nonfinite_entries_to_their_voxels(gpu, monkeypatch, store, nz, z0):
+    """Entries that are not finite reach the voxels that see them and no others, inside the
+    cylinder too: the LDS forms give the volume of the form that tests voxel by voxel and
+    reads global memory, NaN for NaN.  One image is NaN throughout and another infinite in
+    every other row, in a scan whose grid is wider than the detector and whose height
+    offsets move runs out of the window, so that tiles hold columns that see such an image
+    beside columns that do not."""
+    import torch
+    import ct_amd
+    W, H, P = 70, 50, 11
+    g = ct_amd.geometry_grid(W, H, 1.3 * W, 5.0, 85, 83, nz)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    ctx.set_projections(np.linspace(0.0, 350.0, P), np.linspace(-40.0, 40.0, P))
+    img = torch.randn((P, H, W), generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+    img[4] = float("nan")
+    img[7, ::2] = float("inf")
+    entries = torch.empty(ctx.filtered_bytes(store, P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, dtype=torch.float32, device="cuda")
+    ctx.layout_projections(img, P, store, entries, scales)
+
+    def volume():
+        v = torch.empty((g.nx, g.ny, nz - z0), dtype=torch.float32, device="cuda")
+        ctx.backproject(entries, store, scales, 0, P, v, z0, nz - z0, False)
+        torch.cuda.synchronize()
+        return v.cpu().numpy()
+
+    got = volume()
+    monkeypatch.setenv("CTG_BP_PITCH", "65536,0")
+    ref = volume()
+    assert np.isnan(ref).any() and np.any(np.isfinite(ref) & (ref != 0.0))
+    np.testing.assert_array_equal(got, ref)
