@@ -812,10 +812,11 @@ __global__ __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(4))) 
     const int n_out = xmajor ? a.nx : a.ny, n_in = xmajor ? a.ny : a.nx;
     const float pre_out = xmajor ? a.xpre : a.ypre, pre_in = xmajor ? a.ypre : a.xpre;
     const float So = xmajor ? Sx : Sy, Si = xmajor ? Sy : Sx;
-    // (the hardware's reciprocal and root, good to 1e-7: the fan's margins are far wider)
-    const float k0 = ((xmajor ? q0y : q0x) - Si) * __builtin_amdgcn_rcpf((xmajor ? q0x : q0y) - So);
-    const float k1 = ((xmajor ? q1y : q1x) - Si) * __builtin_amdgcn_rcpf((xmajor ? q1x : q1y) - So);
-    const float R = __builtin_amdgcn_sqrtf(a.r2);
+    // (divided: the slopes' error is multiplied by the distance to the source, and a hardware
+    // reciprocal one ulp off its rounded value loses voxel columns from 6e5 pixels on)
+    const float k0 = ((xmajor ? q0y : q0x) - Si) / ((xmajor ? q0x : q0y) - So);
+    const float k1 = ((xmajor ? q1y : q1x) - Si) / ((xmajor ? q1x : q1y) - So);
+    const float R = sqrtf(a.r2);
     const int o_lo = max(0, (int)floorf(pre_out - R) - 1), o_hi = min(n_out - 1, (int)ceilf(pre_out + R) + 1);
     const int zend = a.z0 + a.nzs - 1;
     const int zrb = a.z0 & ~(kRowAnchor - 1);

@@ -1260,3 +1260,27 @@ def test_lds_forms_keep_nonfinite_entries_to_their_voxels(gpu, monkeypatch, stor
     ref = volume()
     assert np.isnan(ref).any() and np.any(np.isfinite(ref) & (ref != 0.0))
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("fcd", [1.0e4, 1.0e6])
+def test_forward_projector_takes_every_voxel_of_a_distant_source(gpu, fcd):
+    """Every voxel that the backprojection reads is projected, however near to parallel the
+    rays: <A 1, 1> = <1, A^T 1> for each projection.  The grid holds about 50000 voxel
+    columns inside the cylinder, so one that the fan bounds miss is 2e-5 of the sum; FP32
+    rounding of pixels that sum a few hundred voxels averages to well below the 5e-6 allowed."""
+    import torch
+    import ct_amd
+    W, H, P, n, nz = 260, 16, 60, 256, 4
+    g = ct_amd.geometry_grid(W, H, fcd, 0.0, n, n, nz)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    ctx.set_projections(np.linspace(0.0, 360.0, P, endpoint=False) + 0.3, None)
+    y = torch.empty((P, H, W), device="cuda")
+    ctx.forward_project(torch.ones((n, n, nz), device="cuda"), 0, nz, 0, P, y)
+    entries = torch.empty(ctx.filtered_bytes("f32", 1), dtype=torch.uint8, device="cuda")
+    ctx.layout_projections(torch.ones((1, H, W), device="cuda"), 1, "f32", entries, None)
+    v = torch.empty((n, n, nz), device="cuda")
+    for p in range(P):
+        ctx.backproject(entries, "f32", None, p, 1, v, 0, nz, False)
+        want = float(v.double().sum())
+        assert abs(float(y[p].double().sum()) - want) <= 5e-6 * want, p
