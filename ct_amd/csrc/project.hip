@@ -855,8 +855,9 @@ __global__ __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(4))) 
     const unsigned off0 = (unsigned)((lane - (zs - (win.wz0 - zrb))) * (int)sizeof(float));
     const unsigned off1 = off0 + 256u;
 
-    // An infinite or NaN voxel makes all three rows of its run infinite or NaN: a column with
-    // such sums is computed again, tap by tap.
+    // An infinite or NaN voxel makes all three rows of its run infinite or NaN, and sums past half
+    // the largest float overflow where they are held twice: a column with such sums is computed
+    // again, tap by tap, into rows that hold the sums once.
     int by_tap = 0;
 again:
     for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) acc_lds[i] = make_float2(0.0f, 0.0f);
@@ -1095,7 +1096,7 @@ again:
                         const float zk = ((float)(win.wz0 + 64 * k + (lane & 32)) - a.zpre) + h;
                         const float vI = det_row_index(lane_k, U, fmaf(-zk, U, a.vpre)), v0 = floorf(vI);
                         const bool on = z >= lo && z < hi1;
-                        const float x = on ? 2.0f * colbase[(size_t)r.x * a.zstride + (z - zs)] : 0.0f;
+                        const float x = on ? colbase[(size_t)r.x * a.zstride + (z - zs)] : 0.0f;
                         float2* const at0 = my_rows + (int)v0;
                         for (int j = 0; j < 2; ++j) {
                             const float wr = j ? vI - v0 : 1.0f - (vI - v0);
@@ -1145,14 +1146,15 @@ again:
         by_tap = 1;
         goto again;
     }
+    const float share = by_tap ? 1.0f : 0.5f;
     float2* col = ps + ((size_t)p * a.W + c) * a.H;
     const int row0 = win.first ? 0 : max(win.rbase, 0), row1 = win.first ? a.H - 1 : min(win.rbase + span - 1, a.H - 1);
     for (int row = row0 + tid; row <= row1; row += kGThreads) {
         const int r = row - win.rbase;
         const float2 s2 = r >= 0 && r < span ? acc_lds[r] : make_float2(0.0f, 0.0f);
         float2 o = win.first ? make_float2(0.0f, 0.0f) : col[row];
-        o.x = fmaf(0.5f, s2.x, o.x);
-        o.y = fmaf(0.5f, s2.y, o.y);
+        o.x = fmaf(share, s2.x, o.x);
+        o.y = fmaf(share, s2.y, o.y);
         col[row] = o;
     }
 }
