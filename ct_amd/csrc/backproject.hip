@@ -833,8 +833,11 @@ void number_chunks(BpArgs& a) {
     a.per = a.chunk + (a.extra ? 1 : 0);
 }
 
+// Launches of `step` projections that go on from each other's sums.  One set of tiles and buffers
+// serves all of them: boxes are sampled over the whole scan, once (sampled launch by launch, a
+// scan of more launches than cached_max_box keeps took its samples anew on every call).
 template <int ZPL>
-ctg_status launch_zpl(const BpLaunch& L, BpArgs a, hipStream_t st) {
+ctg_status launch_zpl(const BpLaunch& L, BpArgs a, int step, hipStream_t st) {
     const ctg_geometry& g = *L.g;
     const int ebytes = L.store == CTG_STORE_F32 ? 16 : 8;
     a.zshift = L.z0 & (ZPL - 1);
@@ -885,26 +888,33 @@ ctg_status launch_zpl(const BpLaunch& L, BpArgs a, hipStream_t st) {
     number_chunks(a);
     const long long grid = 8ll * ((long long)a.nzb * a.per + ((long long)a.nidle * a.nzb + 7) / 8);
     if (grid > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
-#define CTG_BP_LAUNCH(E, DMA)                                                                           \
-    hipLaunchKernelGGL((bp_kernel<ZPL, E, DMA>), dim3((unsigned)grid), dim3(kThreads), lds, st, a, L.d_params, \
-                       L.d_scales, L.d_filtered, L.d_volume)
-    switch (L.store) {
-        case CTG_STORE_F32:
-            CTG_BP_LAUNCH(EF32, 16);
-            break;
-        case CTG_STORE_F16:
-            if (a.dma16) CTG_BP_LAUNCH(EF16, 16);
-            else CTG_BP_LAUNCH(EF16, 4);
-            break;
-        case CTG_STORE_BF16:
-            if (a.dma16) CTG_BP_LAUNCH(EBF16, 16);
-            else CTG_BP_LAUNCH(EBF16, 4);
-            break;
-        default:
-            return fail(CTG_ERROR_INVALID_ARGUMENT, "unknown store type %d", (int)L.store);
-    }
+    const size_t img_bytes = (size_t)g.det_width * g.det_height * ebytes;
+    for (int p = 0; p < std::max(L.nproj, 1); p += step) {
+        a.nproj = std::min(step, L.nproj - p);
+        a.resume = p > 0;
+        const float* scales = L.d_scales ? L.d_scales + p : nullptr;
+        const void* filtered = (const char*)L.d_filtered + p * img_bytes;
+#define CTG_BP_LAUNCH(E, DMA)                                                                                  \
+    hipLaunchKernelGGL((bp_kernel<ZPL, E, DMA>), dim3((unsigned)grid), dim3(kThreads), lds, st, a, L.d_params + p, \
+                       scales, filtered, L.d_volume)
+        switch (L.store) {
+            case CTG_STORE_F32:
+                CTG_BP_LAUNCH(EF32, 16);
+                break;
+            case CTG_STORE_F16:
+                if (a.dma16) CTG_BP_LAUNCH(EF16, 16);
+                else CTG_BP_LAUNCH(EF16, 4);
+                break;
+            case CTG_STORE_BF16:
+                if (a.dma16) CTG_BP_LAUNCH(EBF16, 16);
+                else CTG_BP_LAUNCH(EBF16, 4);
+                break;
+            default:
+                return fail(CTG_ERROR_INVALID_ARGUMENT, "unknown store type %d", (int)L.store);
+        }
 #undef CTG_BP_LAUNCH
-    CTG_HIP(hipGetLastError());
+        CTG_HIP(hipGetLastError());
+    }
     return CTG_OK;
 }
 
@@ -946,17 +956,7 @@ ctg_status launch_backproject(const BpLaunch& L, hipStream_t st) {
     const bool large = (long long)a.nwork * ((L.nz + (L.z0 & 31) + 31) / 32) >= 8192;
     const int parts = large && !L.accumulate ? std::max(1, L.nproj / 240) : 1;
     const int step = std::max(1, (L.nproj + parts - 1) / parts);
-    for (int p = 0; p < std::max(L.nproj, 1); p += step) {
-        BpLaunch part = L;
-        part.nproj = a.nproj = std::min(step, L.nproj - p);
-        part.d_params = L.d_params + p;
-        if (L.h_params) part.h_params = L.h_params + p;
-        if (L.d_scales) part.d_scales = L.d_scales + p;
-        part.d_filtered = (const char*)L.d_filtered + (size_t)p * (size_t)img_bytes;
-        a.resume = p > 0;
-        CTG_TRY(zpl == 16 ? launch_zpl<16>(part, a, st) : launch_zpl<32>(part, a, st));
-    }
-    return CTG_OK;
+    return zpl == 16 ? launch_zpl<16>(L, a, step, st) : launch_zpl<32>(L, a, step, st);
 }
 
 ctg_status launch_backproject_f64(const ctg_geometry& g, const double4* d_params, const double* d_rows,

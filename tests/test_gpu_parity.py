@@ -1312,3 +1312,29 @@ def test_forward_projector_sums_of_the_largest_voxels(gpu, monkeypatch, value):
     want = project()
     assert np.isfinite(want).all() and np.abs(want).max() > 0.5 * abs(value)
     assert rel_rmse(got, want) < 2e-6
+
+
+def test_large_scans_sample_their_boxes_once(gpu):
+    """The largest footprint box is sampled on the host once per scan, however many launches it
+    takes (18 here, more than the host keeps samples of): a repeated call does not sample
+    again, so its host time stays below that of sampling for a few launches."""
+    import time
+    import torch
+    import ct_amd
+    n, nz, P, H, W = 512, 352, 4320, 8, 520
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, H, 2600.0, 0.0, n, n, nz))
+    ctx.set_projections(np.linspace(0.0, 360.0, P, endpoint=False), None)
+    entries = torch.zeros(ctx.filtered_bytes("f32", P), dtype=torch.uint8, device="cuda")
+    v = torch.empty((n, n, nz), device="cuda")
+
+    def host_time(p0, np_, accumulate):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        ctx.backproject(entries, "f32", None, p0, np_, v, 0, nz, accumulate)
+        return time.perf_counter() - t
+
+    ctx.backproject(entries, "f32", None, 0, 1, v, 0, nz, True)  # the module is loaded
+    sample = min(host_time(p, 240, True) for p in range(1, 6))  # one launch, sampled each time
+    host_time(0, P, False)
+    assert min(host_time(0, P, False) for _ in range(3)) < 4.0 * sample
