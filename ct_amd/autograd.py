@@ -88,9 +88,9 @@ class ConeBeamOperator:
     def project(self, volume: torch.Tensor) -> torch.Tensor:
         """A x: (nx, ny, nz) -> (P, H, W)."""
         volume = self._check(volume, self.volume_shape, "volume")
+        if self.g.nz == 0:  # an empty tensor has no address to pass
+            return torch.zeros(self.proj_shape, dtype=torch.float32, device=self.device)
         out = torch.empty(self.proj_shape, dtype=torch.float32, device=self.device)
-        if self.g.nz == 0:
-            return out
         self.ctx.forward_project(volume, 0, self.g.nz, 0, self.nproj, out, stream=_stream())
         return out
 
@@ -138,6 +138,8 @@ class ConeBeamOperator:
     def fdk_adjoint(self, grad_volume: torch.Tensor) -> torch.Tensor:
         """F^T g = Wf H A g: (nx, ny, nz) -> (P, H, W)."""
         grad_volume = self._check(grad_volume, self.volume_shape, "grad_volume")
+        if self.g.nz == 0:
+            return torch.zeros(self.proj_shape, dtype=torch.float32, device=self.device)
         s = _stream()
         out = torch.empty(self.proj_shape, dtype=torch.float32, device=self.device)
         self.ctx.fdk_backward(grad_volume, 0, self.g.nz, 0, self.nproj, self.filt, out, stream=s)

@@ -1338,3 +1338,16 @@ def test_large_scans_sample_their_boxes_once(gpu):
     sample = min(host_time(p, 240, True) for p in range(1, 6))  # one launch, sampled each time
     host_time(0, P, False)
     assert min(host_time(0, P, False) for _ in range(3)) < 4.0 * sample
+
+
+def test_operators_on_a_grid_without_slices(gpu):
+    """A of an empty volume, and F's adjoint, are images of zeros, whatever their memory held."""
+    import torch
+    import ct_amd
+    from ct_amd.autograd import ConeBeamOperator
+    op = ConeBeamOperator(ct_amd.geometry_grid(40, 30, 200.0, 0.0, 20, 20, 0), [0.0, 90.0], slab_nz=8)
+    x = torch.empty(op.volume_shape, device="cuda")
+    for apply in (op.project, op.fdk_adjoint):
+        dirty = torch.full(op.proj_shape, float("nan"), device="cuda")
+        del dirty
+        assert torch.equal(apply(x), torch.zeros(op.proj_shape, device="cuda"))
