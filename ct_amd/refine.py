@@ -35,7 +35,7 @@ import time
 
 import torch
 
-from ._ctg import SUM_WORK
+from ._ctg import SUM_WORK, Context
 from .autograd import ConeBeamOperator
 
 
@@ -46,7 +46,7 @@ class Interrupted(RuntimeError):
 def _sum_sq(t: torch.Tensor, op) -> float:
     ctx = getattr(op, "ctx", None)
     # other operators: host tensors, as in the CPU tests of the checkpoint logic, or their own
-    if ctx is None or not t.is_cuda or t.dtype != torch.float32:
+    if not isinstance(ctx, Context) or not t.is_cuda or t.dtype != torch.float32:
         return float(torch.sum(t.double() * t.double()))
     t = t.contiguous()
     work = torch.empty(SUM_WORK, dtype=torch.float64, device=t.device)

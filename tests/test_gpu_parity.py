@@ -1351,3 +1351,17 @@ def test_operators_on_a_grid_without_slices(gpu):
         dirty = torch.full(op.proj_shape, float("nan"), device="cuda")
         del dirty
         assert torch.equal(apply(x), torch.zeros(op.proj_shape, device="cuda"))
+
+
+def test_line_search_norm_of_an_operator_with_another_context(gpu):
+    """An operator of the caller's own may keep anything under the name ctx: the norm of a
+    refinement step then comes from torch (1e-13, as above)."""
+    import torch
+    from ct_amd.refine import _sum_sq
+
+    class Op:
+        ctx = {"device": 0}
+
+    x = torch.randn((30, 40, 50), generator=torch.Generator(device="cuda").manual_seed(4), device="cuda")
+    want = float((x.double() ** 2).sum())
+    assert abs(_sum_sq(x, Op()) - want) <= 1e-13 * want
