@@ -17,7 +17,7 @@
 //  - W = 256..2048, powers of two (FP32): one wave per row pair, values in registers,
 //    Stockham radix-16/8/4 passes exchanging through the wave's LDS region
 //    (rows_fft_kernel).
-//  - Padded rows and W = 4096, 8192 (FP32, M from 256): radix-2 stages, decimation in time
+//  - Padded rows and W = 4096, 8192, 16384 (FP32, M from 256): radix-2 stages, decimation in time
 //    forward and in frequency back, several at a time in registers (rows_r2_kernel).
 //  - Shorter transforms and the FP64 yardstick: the same radix-2 stages one at a time in
 //    LDS, one workgroup per row pair (rows_kernel).

@@ -1365,3 +1365,11 @@ def test_line_search_norm_of_an_operator_with_another_context(gpu):
     x = torch.randn((30, 40, 50), generator=torch.Generator(device="cuda").manual_seed(4), device="cuda")
     want = float((x.double() ** 2).sum())
     assert abs(_sum_sq(x, Op()) - want) <= 1e-13 * want
+
+
+@pytest.mark.parametrize("W", [65, 127, 511, 1023, 4095, 8192, 16384])
+def test_row_filter_remaining_transform_lengths_match_oracle(gpu, oracle, W):
+    """The other ends of the transform lengths: the shortest padded one (256 points, several
+    row pairs to a wave), the largest widths of 1024, 2048 and 8192, and the widest powers of
+    two.  Rows and maxima as in the test of the lengths above."""
+    test_row_filter_transform_lengths_match_oracle(gpu, oracle, W)
