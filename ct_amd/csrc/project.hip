@@ -849,11 +849,13 @@ __global__ __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(4))) 
     float2* const my_rows = acc_lds + (wv * 2 + (lane & 1)) * stride - win.rbase;
     // A candidate's voxels are read from the window's first slice inside the slab, zs (relative
     // to the run base).  Lanes of chunk 0 before it wrap to a huge offset, past every
-    // resource; the later chunks' offsets are one register plus immediates.
+    // resource; an immediate added to that was measured to read zeros where the sum lands inside
+    // it, so the later chunks start from a register of their own, which the compiler may add
+    // immediates to but not fold into chunk 0's.
     const int zs = max(wlo - zrb, win.wz0 - zrb);
     const float* colbase = vol + (zrb - a.z0) + zs;
     const unsigned off0 = (unsigned)((lane - (zs - (win.wz0 - zrb))) * (int)sizeof(float));
-    const unsigned off1 = off0 + 256u;
+    const unsigned off1 = vadd_sv(256, off0);
 
     // An infinite or NaN voxel makes all three rows of its run infinite or NaN, and sums past half
     // the largest float overflow where they are held twice: a column with such sums is computed
