@@ -1373,3 +1373,32 @@ def test_row_filter_remaining_transform_lengths_match_oracle(gpu, oracle, W):
     row pairs to a wave), the largest widths of 1024, 2048 and 8192, and the widest powers of
     two.  Rows and maxima as in the test of the lengths above."""
     test_row_filter_transform_lengths_match_oracle(gpu, oracle, W)
+
+
+@pytest.mark.parametrize("z0", [0, 7, 32])
+def test_forward_projector_slabs_longer_than_a_launch(gpu, monkeypatch, z0):
+    """A slab of more than 16320 slices takes a second launch of the row runs, which starts on a
+    chunk and adds to the first one's sums: the gather form's images (2e-6, as above), with
+    the detector at the seam, at either end of the slab and in its middle."""
+    import torch
+    import ct_amd
+    n, nz = 12, 16401
+    g = ct_amd.geometry_grid(24, 96, 150.0, 0.5, n, n, z0 + nz + 5)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    at = [z0 + 16320, z0, z0 + nz, z0 + 8000]
+    ctx.set_projections([10.0, 100.0, 190.0, 280.0], [float(g.z_pre) - z for z in at])
+    x = torch.randn((n, n, nz), generator=torch.Generator(device="cuda").manual_seed(z0), device="cuda")
+
+    def project(p):
+        y = torch.empty((g.det_height, g.det_width), device="cuda")
+        ctx.forward_project(x, z0, nz, p, 1, y)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    got = [project(p) for p in range(4)]
+    monkeypatch.setenv("CTG_FP_GATHER", "1")
+    for p in range(4):
+        want = project(p)
+        assert np.abs(want).max() > 0.0
+        assert rel_rmse(got[p], want) < 2e-6
