@@ -30,7 +30,8 @@ __global__ void maxabs_kernel(const float* __restrict__ img, size_t per_image, u
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < per_image; i += (size_t)gridDim.x * blockDim.x)
         m = fmaxf(m, fabsf(src[i]));
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) raise_max(&out[p], m);
+    // (no look at the maximum first: the waves of an image end together, so it would only add a wait)
+    if ((threadIdx.x & 63) == 0) atomicMax(&out[p], __float_as_uint(m));
 }
 }  // namespace
 
