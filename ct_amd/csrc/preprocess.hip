@@ -808,6 +808,12 @@ __global__ __launch_bounds__(r2::threads(L)) __attribute__((amdgpu_waves_per_eu(
 // contiguous run of a column's stores (512 bytes of 8-byte entries) and halves the texels read
 // twice, and 8-byte entries go out two rows per lane.  48 images of 2048 x 1536 to FP16: 0.48
 // -> 0.41 ms (4.4 TB/s), 359 of 1001 x 763 (odd height, one row per lane): 0.80 -> 0.73 ms.
+//
+// The tiles of an image are rotated by its number, except large images (over 64 tiles) in tiles of
+// 64: dispatch deals workgroups to the 8 XCDs in turn, and where the tiles of an image are a
+// multiple of 4 or 8 the same XCDs would take the partly filled ones at the edge of every image
+// (FP32, 300 images of 250 x 201 in 4 x 4 tiles: 91 us, 78 rotated; 120 of 341 x 196 in 6 x 4: 34
+// and 29; 240 of 1024 x 1024 in tiles of 32: 1035 and 1001).
 __device__ inline uint32_t pack_f16(float a, float b) {
     __half ha = __float2half_rn(a), hb = __float2half_rn(b);
     return (uint32_t)__half_as_ushort(ha) | ((uint32_t)__half_as_ushort(hb) << 16);
@@ -825,19 +831,32 @@ __global__ __launch_bounds__(256) void layout_kernel(const float* __restrict__ r
                                                      void* __restrict__ out, float* __restrict__ scales) {
     __shared__ float tile[TS + 1][TS + 1];
     constexpr int kStep = 256 / TS;  // rows loaded, then columns stored, at a time
-    const int u0 = blockIdx.x * TS, v0 = blockIdx.y * TS;
     const size_t p = blockIdx.z;
+    unsigned tx = blockIdx.x, ty = blockIdx.y;
+    if (blockIdx.z > 0 && (TS == 32 || gridDim.x * gridDim.y <= 64)) {
+        tx = (tx + blockIdx.z) % gridDim.x;
+        ty = (ty + blockIdx.z / gridDim.x) % gridDim.y;
+    }
+    const int u0 = tx * TS, v0 = ty * TS;
     const float* img = rows + p * (size_t)W * H;
     const int tl = threadIdx.x & (TS - 1), tr = threadIdx.x / TS;
     auto texel = [&](int vl, int ul) {
         const int v = v0 + vl, u = u0 + ul;
         return v < H && u < W ? img[(size_t)v * W + u] : 0.0f;
     };
+    // (a small tile in one go over its 33 x 33 texels: as below it takes 2 to 10 % longer)
+    if constexpr (TS == 32) {
+        for (int i = threadIdx.x; i < (TS + 1) * (TS + 1); i += 256) {
+            const int vl = i / (TS + 1), ul = i - vl * (TS + 1);
+            tile[vl][ul] = texel(vl, ul);
+        }
+    } else {
 #pragma unroll
-    for (int i = 0; i < TS / kStep; ++i) tile[tr + i * kStep][tl] = texel(tr + i * kStep, tl);
-    // the row below and the column to the right
-    if (threadIdx.x < TS) tile[TS][threadIdx.x] = texel(TS, threadIdx.x);
-    else if (threadIdx.x < 2 * TS + 1) tile[threadIdx.x - TS][TS] = texel(threadIdx.x - TS, TS);
+        for (int i = 0; i < TS / kStep; ++i) tile[tr + i * kStep][tl] = texel(tr + i * kStep, tl);
+        // the row below and the column to the right
+        if (threadIdx.x < TS) tile[TS][threadIdx.x] = texel(TS, threadIdx.x);
+        else if (threadIdx.x < 2 * TS + 1) tile[threadIdx.x - TS][TS] = texel(threadIdx.x - TS, TS);
+    }
     __syncthreads();
     float scale = 1.0f, inv = 1.0f;
     if (STORE != CTG_STORE_F32) {
@@ -849,7 +868,7 @@ __global__ __launch_bounds__(256) void layout_kernel(const float* __restrict__ r
             inv = ldexpf(1.0f, -e);
         }
     }
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && scales != nullptr) scales[p] = scale;
+    if (tx == 0 && ty == 0 && threadIdx.x == 0 && scales != nullptr) scales[p] = scale;
     auto coeffs = [&](int vl, int ul) {
         const float A = tile[vl][ul] * inv, B = tile[vl][ul + 1] * inv;
         const float C = tile[vl + 1][ul] * inv, D = tile[vl + 1][ul + 1] * inv;
@@ -1107,13 +1126,19 @@ ctg_status launch_layout(const ctg_geometry& g, const float* d_rows, int nproj, 
         const unsigned* mx = d_maxabs ? d_maxabs + p0 : nullptr;  // not read for FP32 entries
         void* out = (char*)d_out + (size_t)p0 * img * ebytes;
         float* sc = d_scales ? d_scales + p0 : nullptr;
-        const dim3 big = tiles(64);
+        const dim3 big = tiles(64), small = tiles(32);
         // 64 x 64 tiles where at least four per CU are left (one image of 256 x 192 takes 4.1 us
-        // with its 48 tiles of 32, 7.6 with 12 of 64)
-        const bool wide = (long long)big.x * big.y * big.z >= 1024;
+        // with its 48 tiles of 32, 7.6 with 12 of 64), where they cover at most 1.45 times the area
+        // that tiles of 32 do (FP32, 600 images of 129 x 129, 1.44 times: 41 us and 42 in tiles of
+        // 32; 720 of 70 x 70, 1.78 times: 23 and 16) and, with FP32 entries, where these about fit
+        // the 256 MB Infinity Cache (in tiles of 64 and 32: 270 MiB, 360 of 256 x 192, 79 and 91 us;
+        // 291 MiB, 107 of 1038 x 172, 95 and 91; 1144 MiB, 100 of 1000 x 750, 348 and 315; 8-byte
+        // entries gain 2 to 9 % at all of these sizes)
+        const bool wide = (long long)big.x * big.y * big.z >= 1024 && 400ll * big.x * big.y <= 145ll * small.x * small.y &&
+                          (store != CTG_STORE_F32 || np * img * ebytes <= (size_t)280 << 20);
         // columns of an even height start 16-byte aligned if the buffer does
         const int pairs = g.det_height % 2 == 0 && (uintptr_t)out % 16 == 0;
-        const dim3 grid = wide ? big : tiles(32);
+        const dim3 grid = wide ? big : small;
 #define CTG_LAYOUT(S, TS) \
     hipLaunchKernelGGL((layout_kernel<S, TS>), grid, dim3(256), 0, st, rows, g.det_width, g.det_height, mx, pairs, out, sc)
         if (store == CTG_STORE_F32) {

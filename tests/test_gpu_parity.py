@@ -1402,3 +1402,24 @@ def test_forward_projector_slabs_longer_than_a_launch(gpu, monkeypatch, z0):
         want = project(p)
         assert np.abs(want).max() > 0.0
         assert rel_rmse(got[p], want) < 2e-6
+
+
+@pytest.mark.parametrize("W,H,P", [(129, 129, 130), (70, 70, 300), (250, 8, 300), (64, 2, 1100), (2, 600, 1200)])
+def test_layout_covers_every_tile_of_every_image(gpu, W, H, P):
+    """The tiles of an image are numbered anew for every image: 3 x 3 of 64, 3 x 3 of 32, 4 x 1,
+    one, and one column of ten, each entry written once, from its own texels.  Entries and
+    scales as the definition gives them: the same FP32 differences, so bit for bit."""
+    import torch
+    import ct_amd
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, H, 5.0 * W, 0.0, 4, 4, 4))
+    ctx.set_projections(np.zeros(P), None)
+    img = torch.randn((P, H, W), generator=torch.Generator(device="cuda").manual_seed(H), device="cuda")
+    q = torch.nn.functional.pad(img, (0, 1, 0, 1)).transpose(1, 2)
+    A, B, C, D = q[:, :-1, :-1], q[:, 1:, :-1], q[:, :-1, 1:], q[:, 1:, 1:]
+    want = torch.stack((A, B - A, C - A, (D - C) - (B - A)), dim=-1)
+    entries = torch.full((P, W, H, 4), float("nan"), device="cuda")
+    scales = torch.full((P,), float("nan"), device="cuda")
+    ctx.layout_projections(img, P, "f32", entries, scales)
+    torch.cuda.synchronize()
+    assert torch.equal(entries, want) and (scales == 1.0).all()
