@@ -189,17 +189,17 @@ ctg_status preprocess_batched(ctg_context* ctx, const void* d_raw, ctg_pixel_typ
     // only the 8-byte entries are scaled by their image's max |value|
     const bool scaled = store != CTG_STORE_F32;
     if (scaled) {
-        CTG_TRY(ctx->maxabs.reserve(sizeof(unsigned) * std::max(nproj, 1)));
-        CTG_TRY(fill_u32(ctx->maxabs.ptr, 0u, (size_t)nproj, st));
+        CTG_TRY(ctx->maxabs.reserve(sizeof(unsigned) * kMaxStride * std::max(nproj, 1)));
+        CTG_TRY(fill_u32(ctx->maxabs.ptr, 0u, (size_t)nproj * kMaxStride, st));
     }
     for (int b0 = 0; b0 < nproj; b0 += batch) {
         if (ctx->cancel.load()) return fail(CTG_ERROR_INTERRUPTED, "interrupted");
         const int nb = std::min(batch, nproj - b0);
         const char* raw = (const char*)d_raw + (size_t)b0 * img * pixel_bytes(pixel);
-        unsigned* mx = scaled ? ctx->maxabs.as<unsigned>() + b0 : nullptr;
+        unsigned* mx = scaled ? ctx->maxabs.as<unsigned>() + (size_t)b0 * kMaxStride : nullptr;
         CTG_TRY(launch_preprocess_rows(ctx, raw, pixel, nb, base, form, filter, ctx->rows_f32.as<float>(), mx, st));
         char* out = (char*)d_filtered + (size_t)b0 * img * store_bytes(store);
-        CTG_TRY(launch_layout(g, ctx->rows_f32.as<float>(), nb, store, mx, out,
+        CTG_TRY(launch_layout(g, ctx->rows_f32.as<float>(), nb, store, mx, kMaxStride, out,
                               d_scales ? d_scales + b0 : nullptr, st));
     }
     return CTG_OK;
@@ -538,7 +538,7 @@ ctg_status ctg_layout_projections(ctg_context* ctx, const float* d_images, int32
         CTG_TRY(fill_u32(mx, 0u, (size_t)nproj, st));
         CTG_TRY(launch_maxabs(d_images, img, nproj, mx, st));
     }
-    return launch_layout(ctx->geom, d_images, nproj, store, mx, d_filtered, d_scales, st);
+    return launch_layout(ctx->geom, d_images, nproj, store, mx, 1, d_filtered, d_scales, st);
 }
 
 ctg_status ctg_layout_projections_noalloc(ctg_context* ctx, const float* d_images, int32_t nproj, ctg_store store,
@@ -560,7 +560,7 @@ ctg_status ctg_layout_projections_noalloc(ctg_context* ctx, const float* d_image
         CTG_TRY(fill_u32(mx, 0u, (size_t)nproj, st));
         CTG_TRY(launch_maxabs(d_images, img, nproj, mx, st));
     }
-    return launch_layout(ctx->geom, d_images, nproj, store, mx, d_filtered, d_scales, st);
+    return launch_layout(ctx->geom, d_images, nproj, store, mx, 1, d_filtered, d_scales, st);
 }
 
 ctg_status ctg_backproject(ctg_context* ctx, const void* d_filtered, ctg_store store, const float* d_scales,

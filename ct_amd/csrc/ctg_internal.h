@@ -76,15 +76,6 @@ __device__ inline int opaque_uniform(int v) {
     return v;
 }
 
-// Raises the running maximum *m (bits of a non-negative float, which order like unsigned
-// integers) to v.  Atomics to one address run one after another (about 10 ns each here: the
-// one per wave of every row of an image took longer than the row's filter), so a value
-// that is already covered only reads: what it reads may be old, but then only lower.
-__device__ inline void raise_max(unsigned* m, float v) {
-    const unsigned b = __float_as_uint(v);
-    if (__hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < b) atomicMax(m, b);
-}
-
 // Grow-only device buffer owned by a context.
 struct DevBuf {
     void* ptr = nullptr;
@@ -153,6 +144,9 @@ ctg_status launch_maxabs(const float* d_images, size_t per_image, int nproj, uns
 
 ctg_status ensure_filter_tables(ctg_context* ctx, int W, int filter);
 
+// The row filter keeps every image's running maximum in a cache line of its own (128 bytes).
+constexpr int kMaxStride = 32;
+
 // ---- preprocess.hip
 ctg_status launch_preprocess_rows(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel,
                                   int nproj, float base, ctg_log_form form, ctg_filter filter,
@@ -163,8 +157,9 @@ ctg_status launch_filter_rows_only(ctg_context* ctx, const float* d_in, float* d
 ctg_status launch_preprocess_rows_f64(ctg_context* ctx, const void* d_raw, ctg_pixel_type pixel,
                                       int nproj, float base, ctg_filter filter, double* d_out,
                                       hipStream_t st);
+// d_maxabs: the images' max |x|, mstride counters apart (not read for FP32 entries).
 ctg_status launch_layout(const ctg_geometry& g, const float* d_rows, int nproj, ctg_store store,
-                         const unsigned* d_maxabs, void* d_out, float* d_scales, hipStream_t st);
+                         const unsigned* d_maxabs, int mstride, void* d_out, float* d_scales, hipStream_t st);
 
 // ---- backproject.hip
 struct BpLaunch {

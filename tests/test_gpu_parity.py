@@ -1423,3 +1423,32 @@ def test_layout_covers_every_tile_of_every_image(gpu, W, H, P):
     ctx.layout_projections(img, P, "f32", entries, scales)
     torch.cuda.synchronize()
     assert torch.equal(entries, want) and (scales == 1.0).all()
+
+
+@pytest.mark.parametrize("W,H,P", [(256, 192, 360), (64, 64, 2000), (512, 512, 200)])
+def test_image_maxima_cost_no_more_than_the_entries(gpu, W, H, P):
+    """Many small images to FP16: the images' maxima come beside the row filter, and the entries
+    are half the size of FP32 ones, so the call takes less time than with FP32 entries.  A factor of
+    2 covers the noise of either time (each the least of eight)."""
+    import torch
+    import ct_amd
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, H, 5.0 * W, 0.0, 4, 4, 4))
+    ctx.set_projections(np.zeros(P), None)
+    raw = torch.randint(3000, 32000, (P, H, W), dtype=torch.int16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def ms(store):
+        entries = torch.empty(ctx.filtered_bytes(store, P), dtype=torch.uint8, device="cuda")
+        scales = torch.empty(P, device="cuda")
+        times = []
+        for _ in range(9):
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record()
+            ctx.preprocess(raw, "u16", P, 1.0, "cpu", "hann", store, entries, scales, stream)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times[1:])
+
+    assert ms("f16") < 2.0 * ms("f32")
