@@ -21,6 +21,7 @@ namespace {
 struct FpArgs {
     int W, H, nx, ny, nzs, z0, nproj;
     int zstride;  // slices per voxel column of the volume buffer (nzs of them from z0 are projected)
+    int cblock;   // pixel columns per unit of fp_rows_kernel's numbering
     float xpre, ypre, zpre, upre, vpre;
     float r2, fcd, uoff, ulo, uhi, vlo, vhi;
 };
@@ -768,22 +769,29 @@ __device__ inline float lane_value(int x, int lane) { return __int_as_float(__bu
 // The workgroups that an XCD runs together (dispatch is round-robin over 8 XCDs) should read
 // the same voxels: a voxel column is read once per projection, by the column it falls on, and
 // for neighbouring projections by neighbouring columns.  So the work is cut into units of
-// kPBlock projections x kCBlock columns, dealt to the XCDs in turn (columns vary slowest, so
+// kPBlock projections x cblock columns, dealt to the XCDs in turn (columns vary slowest, so
 // that short rays at the edges spread over the XCDs), and inside a unit the projections vary
-// fastest.  Units of the rounded-up grid beyond it exit.
-constexpr int kPBlock = 4, kCBlock = 64;
-__host__ __device__ inline unsigned fp_units(int W, int nproj) {
-    return (unsigned)((W + kCBlock - 1) / kCBlock) * (unsigned)((nproj + kPBlock - 1) / kPBlock);
+// fastest.  Units of the rounded-up grid beyond it exit, and the last workgroups of a unit that
+// reaches past the last projection or column (not every fourth: an XCD deals workgroups to its
+// shader engines in turn, and one projection of 384^3 took 182 us so, with work on one engine).
+//
+// Columns per unit: 64, halved down to 8 while there are fewer than 64 units, that is eight for
+// each XCD: 40 projections of 50 columns are 10 units of 64, two of them for two of the XCDs.
+constexpr int kPBlock = 4, kCBlock = 64, kMinCBlock = 8;
+__host__ __device__ inline unsigned fp_units(int W, int nproj, int cblock) {
+    return (unsigned)((W + cblock - 1) / cblock) * (unsigned)((nproj + kPBlock - 1) / kPBlock);
 }
 __device__ inline bool fp_item(const FpArgs& a, int& c, int& p) {
-    constexpr unsigned per = kPBlock * kCBlock;
+    const unsigned per = (unsigned)(kPBlock * a.cblock);
     const unsigned xcd = blockIdx.x & 7u, k = blockIdx.x >> 3;
     const unsigned unit = (k / per) * 8u + xcd, r = k % per;
     const unsigned npb = (unsigned)((a.nproj + kPBlock - 1) / kPBlock);
     const unsigned cb = unit / npb, pb = unit - cb * npb;
-    c = (int)(cb * kCBlock + r / kPBlock);
-    p = (int)(pb * kPBlock + r % kPBlock);
-    return c < a.W && p < a.nproj;
+    const unsigned np = (unsigned)min(kPBlock, a.nproj - (int)pb * kPBlock);  // projections of this unit
+    const unsigned cl = r / np;
+    c = (int)(cb * a.cblock + cl);
+    p = (int)(pb * kPBlock + (r - cl * np));
+    return cl < (unsigned)a.cblock && c < a.W;
 }
 
 template <int G>
@@ -1444,7 +1452,9 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
         CTG_TRY(work.reserve(pixels * sizeof(float2)));
         float2* ps = work.as<float2>();
         bool entries = false;
-        const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj) + 7) / 8) * 8 * kPBlock * kCBlock;
+        a.cblock = kCBlock;
+        while (a.cblock > kMinCBlock && fp_units(a.W, nproj, a.cblock) < 64) a.cblock /= 2;
+        const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj, a.cblock) + 7) / 8) * 8 * kPBlock * a.cblock;
         if (blocks > 0x7fffffffull) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
         const dim3 rgrid((unsigned)blocks);
         // Volumes of at most two chunks of slices (one window) and short rays go to the entry

@@ -1452,3 +1452,30 @@ def test_image_maxima_cost_no_more_than_the_entries(gpu, W, H, P):
         return min(times[1:])
 
     assert ms("f16") < 2.0 * ms("f32")
+
+
+@pytest.mark.parametrize("P", [1, 2, 3, 5, 9])
+@pytest.mark.parametrize("W", [16, 170, 530])
+def test_forward_projector_unit_shapes_match_gather_form(gpu, monkeypatch, P, W):
+    """The numbering of the row runs' workgroups by units of up to four projections and 8 to 64
+    columns, with units past the last projection or column: every column of every projection once,
+    as in the gather form (2e-6, as above)."""
+    import torch
+    import ct_amd
+    n, nz = W - 4, 140
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, 40, 4.0 * W, 0.75, n, n, nz))
+    ctx.set_projections(np.linspace(5.0, 330.0, P), np.linspace(-2.0, 3.0, P))
+    x = torch.randn((n, n, nz), generator=torch.Generator(device="cuda").manual_seed(P), device="cuda")
+
+    def project():
+        y = torch.full((P, 40, W), float("nan"), device="cuda")
+        ctx.forward_project(x, 0, nz, 0, P, y)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    got = project()
+    monkeypatch.setenv("CTG_FP_GATHER", "1")
+    want = project()
+    assert (np.abs(want).max(axis=(1, 2)) > 0.0).all()
+    assert rel_rmse(got, want) < 2e-6
