@@ -406,8 +406,16 @@ struct FpWin {
 // faster one where columns are short (see the launch): 59 against 64 us at 96^2 x 72 from 48
 // projections of 103 x 83, 296 against 311 at 128^3 from 200, but 217 against 207 at 200^2 x
 // 128 from 60 and 428 against 302 at 160^3 from 100, where a third window is begun.
-constexpr int kEntryMaxSpan = 256;  // entry rows per copy
+constexpr int kEntryMaxSpan = 320;  // entry rows per copy (three workgroups per CU)
 constexpr int kEntryMaxSide = 160;  // voxels
+// Windows whose runs would be shorter than this many candidates take the entry form too, two
+// chunks at a time: a run end then costs as much as it saves.  200^2 x 200 (a window of 256
+// slices) from 250 projections and a source 1.2, 1.4 detector widths away, runs of 1.6, 1.9: rows
+// 2.04, 1.93 ms, entries 1.77, 1.73; 150^2 x 223, 2 widths, 2.0: 0.83, 0.88; 200^2 x 256, 1.6
+// widths, 2.5: 1.06, 1.24; 125^2 x 223, 2.5 widths, 2.2: 0.64, 0.66.
+// Heights that spread over many rows take that away, as every copy holds the rows of all of them
+// (109^2 x 223, 2.5 widths, 1.9: 0.48 and 0.48 ms, with heights of -22 to 22 0.52 and 0.58).
+constexpr double kMinRun = 1.95, kMinRunHeights = 16.0;
 
 __device__ inline int flr_i32(float x) {
     int r;
@@ -415,7 +423,7 @@ __device__ inline int flr_i32(float x) {
     return r;
 }
 
-template <int G>
+template <int G, bool CHECK>
 __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win, const float4* __restrict__ pp,
                                                              const float* __restrict__ vol,
                                                              float2* __restrict__ ps) {
@@ -433,8 +441,6 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int span = win.span, stride = win.stride;
-    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) entry_lds[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-
     const float4 g = pp[p];
     const float sn = g.x, cs = g.y, h = g.z;
     const float Sx = a.fcd * cs + a.uoff * sn, Sy = a.fcd * sn - a.uoff * cs;
@@ -486,6 +492,13 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
     const float* colbase = vol + (zrb - a.z0);
     const int zc = win.wz0 - zrb;  // the window's first slice relative to the run base
     const unsigned lane4 = (unsigned)lane * (unsigned)sizeof(float);
+
+    // An infinite voxel makes NaN of the pixels' differences of entry sums, and of pixels that it
+    // has no weight in.  CHECK: a column with sums that are not finite is computed again, tap by
+    // tap (small volumes do without: the check and its code take 5 to 14 % of a small launch).
+    int by_tap = 0;
+again:
+    for (int i = tid; i < 2 * kGWaves * stride; i += kGThreads) entry_lds[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     __syncthreads();
 
     int ncand = 0;
@@ -632,17 +645,42 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
                     *e[k] = v[k];
                 }
             };
-            Slot sa, sb, sc;
-            bool ha = next(sa), hb = next(sb), hc = next(sc);
-            while (ha) {
-                process(sa);
-                ha = next(sa);
-                if (!hb) break;
-                process(sb);
-                hb = next(sb);
-                if (!hc) break;
-                process(sc);
-                hc = next(sc);
+            if (CHECK && opaque_uniform(by_tap)) {
+                for (int ci = wv; ci < ncand; ci += kGWaves) {
+                    const int4 r = slots[ci];
+                    const int lo = r.w & ((1 << kFpZBits) - 1), hi1 = (r.w >> kFpZBits) & ((1 << kFpZBits) - 1);
+                    const float U = __int_as_float(r.y), ws = __int_as_float(r.z), wo = U * U - ws;
+                    for (int k = 0; k < G; ++k) {
+                        const int z = zc + 64 * k + lane;
+                        const float vI = det_row_index(lane_k, U, fmaf(-zh[k], U, a.vpre)), v0 = floorf(vI);
+                        const bool on = z >= lo && z < hi1;
+                        const float x = on ? colbase[(size_t)r.x * a.zstride + z] : 0.0f;
+                        float4* const e = reinterpret_cast<float4*>(acc_bytes + ((int)v0 * 16 + lane_base));
+                        for (int j = 0; j < 2; ++j) {
+                            const float wr = j ? vI - v0 : 1.0f - (vI - v0);
+                            float4 o = e[j];
+                            o.x += wo * wr * x;
+                            o.y += ws * wr * x;
+                            if (on) e[j] = o;
+                            // the next row of one lane may be the row of another
+                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                            __builtin_amdgcn_wave_barrier();
+                        }
+                    }
+                }
+            } else {
+                Slot sa, sb, sc;
+                bool ha = next(sa), hb = next(sb), hc = next(sc);
+                while (ha) {
+                    process(sa);
+                    ha = next(sa);
+                    if (!hb) break;
+                    process(sb);
+                    hb = next(sb);
+                    if (!hc) break;
+                    process(sc);
+                    hc = next(sc);
+                }
             }
             ncand = 0;
             __syncthreads();  // every wave is done with the slots
@@ -651,7 +689,7 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
     // sum the eight copies per entry row (waves in order, even before odd) and turn the
     // entry gradients into pixel partials: own column (q00 at row v, q01 at v + 1) and
     // the next column (q10 at v, q11 at v + 1); pixel row rbase + r takes entry rows r
-    // and r - 1
+    // and r - 1 (tap by tap: its own row's sums)
     float2* col = ps + ((size_t)p * a.W + c) * a.H;
     auto entry = [&](int r) {
         float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -664,12 +702,27 @@ __global__ __launch_bounds__(kGThreads) void fp_entry_kernel(FpArgs a, FpWin win
         }
         return sum;
     };
+    if constexpr (CHECK) {
+        bool bad = false;
+        for (int r = tid; r < span; r += kGThreads) {
+            const float4 e = entry(r);
+            bad |= !((fabsf(e.x) + fabsf(e.y)) + (fabsf(e.z) + fabsf(e.w)) <= 3.402823466e38f);
+        }
+        if (__builtin_amdgcn_readfirstlane(__syncthreads_or(bad)) && !by_tap) {
+            by_tap = 1;
+            goto again;
+        }
+    }
     const int row0 = win.first ? 0 : max(win.rbase, 0), row1 = win.first ? a.H - 1 : min(win.rbase + span, a.H - 1);
     for (int row = row0 + tid; row <= row1; row += kGThreads) {
         const int r = row - win.rbase;
         const float4 e0 = entry(r), e1 = entry(r - 1);  // entries at rows v = row and v = row - 1
-        const float own = ((e0.x - e0.y) - e0.z + e0.w) + (e1.z - e1.w);
-        const float side = (e0.y - e0.w) + e1.w;
+        float own = ((e0.x - e0.y) - e0.z + e0.w) + (e1.z - e1.w);
+        float side = (e0.y - e0.w) + e1.w;
+        if (CHECK && by_tap) {
+            own = e0.x;
+            side = e0.y;
+        }
         float2 o = win.first ? make_float2(0.0f, 0.0f) : col[row];
         o.x += own;
         o.y += side;
@@ -788,7 +841,7 @@ __device__ inline bool fp_item(const FpArgs& a, int& c, int& p) {
     const unsigned npb = (unsigned)((a.nproj + kPBlock - 1) / kPBlock);
     const unsigned cb = unit / npb, pb = unit - cb * npb;
     const unsigned np = (unsigned)min(kPBlock, a.nproj - (int)pb * kPBlock);  // projections of this unit
-    const unsigned cl = r / np;
+    const unsigned cl = np == kPBlock ? r / kPBlock : r / np;
     c = (int)(cb * a.cblock + cl);
     p = (int)(pb * kPBlock + (r - cl * np));
     return cl < (unsigned)a.cblock && c < a.W;
@@ -1420,6 +1473,12 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
     double hmin = 0.0, hmax = 0.0;
     const double R = g.radius, F = g.fcd;
     const double Umin = F / (F + R) * (1.0 - 1e-5), Umax = F / (F - R) * (1.0 + 1e-5);
+    // Candidates per run of a window's outermost slice: neighbours along a ray are a voxel apart in
+    // depth, so their magnifications differ by about 1 / FCD, and a run spans 0.98 rows.
+    auto run_of = [&](int w0, int chunks) {
+        const double y = w0 - g.z_pre + 0.5 * (hmin + hmax);
+        return 0.98 * F / std::max(std::fabs(y), std::fabs(y + 64 * chunks - 1));
+    };
     const bool entry_ok = h_params != nullptr && R < 0.5 * F && !std::getenv("CTG_FP_GATHER");
     if (entry_ok) {
         hmin = hmax = h_params[0].z;
@@ -1445,44 +1504,65 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
                 }
             if (fits) G = cand;
         }
+        // Windows of a single chunk with short runs, where the rows of one column span too much for
+        // more, have neither form's advantage: 656^2 x 1015 from a source 1.3 detector widths away
+        // takes 15.2 ms so, 11.6 in the gather form; 48^2 x 2000 from 2.5 widths 0.30 and 0.26.
+        if (G == 1 && deep > 1 && std::min(run_of(zrb, 1), run_of(z0 + nz - 64, 1)) < kMinRun) G = 0;
     }
     if (G > 0) {
         // the first window writes the column sums and fp_finish_kernel the images, so neither is
         // cleared first
         CTG_TRY(work.reserve(pixels * sizeof(float2)));
         float2* ps = work.as<float2>();
-        bool entries = false;
         a.cblock = kCBlock;
         while (a.cblock > kMinCBlock && fp_units(a.W, nproj, a.cblock) < 64) a.cblock /= 2;
         const unsigned long long blocks = (unsigned long long)((fp_units(a.W, nproj, a.cblock) + 7) / 8) * 8 * kPBlock * a.cblock;
         if (blocks > 0x7fffffffull) return fail(CTG_ERROR_UNSUPPORTED, "forward projection grid too large");
         const dim3 rgrid((unsigned)blocks);
+        auto window = [&](int w0, int chunks) {
+            FpWin win{};
+            win.wz0 = w0;
+            window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * chunks, win.rbase, win.span);
+            return win;
+        };
+        // windows whose rows all lie off the detector are left out
+        auto off = [&](const FpWin& win) { return win.rbase >= a.H || win.rbase + win.span <= 0; };
+        int first = 1;  // the first window to run writes the column sums
         // Volumes of at most two chunks of slices (one window) and short rays go to the entry
         // form: its time per update is larger, but it spends less per column (figures there).
-        if (z0 + nz - (z0 & ~(kRowAnchor - 1)) <= 128 && std::max(g.nx, g.ny) <= kEntryMaxSide && G <= 2) {
-            FpWin win{};
-            win.wz0 = z0 & ~(kRowAnchor - 1);
-            window_rows(g, hmin, hmax, Umin, Umax, win.wz0, 64 * G, win.rbase, win.span);
-            entries = win.wz0 + 64 * G >= z0 + nz && win.span <= kEntryMaxSpan;
-            win.stride = (win.span + 15) & ~15;
-            win.first = 1;
-            const size_t lds = sizeof(float4) * 2 * kGWaves * (size_t)win.stride;
-            if (entries) {
-                if (G == 2) hipLaunchKernelGGL(fp_entry_kernel<2>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-                else hipLaunchKernelGGL(fp_entry_kernel<1>, grid, dim3(kGThreads), lds, st, a, win, d_params, d_volume, ps);
-                CTG_HIP(hipGetLastError());
-            }
-        }
+        const bool small = z0 + nz - (z0 & ~(kRowAnchor - 1)) <= 128 && std::max(g.nx, g.ny) <= kEntryMaxSide;
         // the candidate records hold z relative to the launch's run base in kFpZBits bits
-        for (int s = 0; s < nz && !entries; s += kFpMaxSlab) {
+        for (int s = 0; s < nz; s += kFpMaxSlab) {
             a.z0 = z0 + s;
             a.nzs = std::min(kFpMaxSlab, nz - s);
-            for (int w0 = a.z0 & ~(kRowAnchor - 1); w0 < a.z0 + a.nzs; w0 += 64 * G) {
-                FpWin win{};
-                win.wz0 = w0;
-                window_rows(g, hmin, hmax, Umin, Umax, w0, 64 * G, win.rbase, win.span);
+            const int zend = a.z0 + a.nzs;
+            for (int w0 = a.z0 & ~(kRowAnchor - 1); w0 < zend; w0 += 64 * G) {
+                FpWin win = window(w0, G);
+                if (off(win)) continue;
+                bool entries = small || (hmax - hmin <= kMinRunHeights && run_of(w0, G) < kMinRun);
+                for (int e0 = w0; e0 < std::min(w0 + 64 * G, zend) && entries; e0 += 128)
+                    entries = window(e0, std::min(2, (zend - e0 + 63) / 64)).span <= kEntryMaxSpan;
+                for (int e0 = w0; e0 < std::min(w0 + 64 * G, zend) && entries; e0 += 128) {
+                    const int chunks = std::min({2, (zend - e0 + 63) / 64, G - (e0 - w0) / 64});
+                    FpWin part = window(e0, chunks);
+                    if (off(part)) continue;
+                    part.stride = (part.span + 15) & ~15;
+                    part.first = first;
+                    const size_t lds = sizeof(float4) * 2 * kGWaves * (size_t)part.stride;
+#define CTG_ENTRY(G, CHECK) \
+    hipLaunchKernelGGL((fp_entry_kernel<G, CHECK>), grid, dim3(kGThreads), lds, st, a, part, d_params, d_volume + s, ps)
+                    if (small && chunks == 2) CTG_ENTRY(2, false);
+                    else if (small) CTG_ENTRY(1, false);
+                    else if (chunks == 2) CTG_ENTRY(2, true);
+                    else CTG_ENTRY(1, true);
+#undef CTG_ENTRY
+                    CTG_HIP(hipGetLastError());
+                    first = 0;
+                }
+                if (entries) continue;
                 win.stride = (win.span + 1) & ~1;
-                win.first = s == 0 && w0 <= z0;
+                win.first = first;
+                first = 0;
                 const size_t lds = sizeof(float2) * 2 * kGWaves * (size_t)win.stride;
                 if (G == 4) hipLaunchKernelGGL(fp_rows_kernel<4>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
                 else if (G == 3) hipLaunchKernelGGL(fp_rows_kernel<3>, rgrid, dim3(kGThreads), lds, st, a, win, d_params, d_volume + s, ps);
@@ -1491,6 +1571,7 @@ ctg_status launch_forward_project(const ctg_geometry& g, const float4* d_params,
                 CTG_HIP(hipGetLastError());
             }
         }
+        if (first) return accumulate ? CTG_OK : fill_u32(d_proj, 0u, pixels, st);  // no voxel is seen
         dim3 fg((unsigned)((a.W + 31) / 32), (unsigned)((a.H + 31) / 32), (unsigned)nproj);
         hipLaunchKernelGGL(fp_finish_kernel, fg, dim3(256), 0, st, ps, a.W, a.H, accumulate, d_proj);
         CTG_HIP(hipGetLastError());

@@ -1479,3 +1479,51 @@ def test_forward_projector_unit_shapes_match_gather_form(gpu, monkeypatch, P, W)
     want = project()
     assert (np.abs(want).max(axis=(1, 2)) > 0.0).all()
     assert rel_rmse(got, want) < 2e-6
+
+
+@pytest.mark.parametrize("n,nz,z0,W,H,k,h", [(172, 200, 0, 180, 190, 1.2, 0.0), (172, 390, 21, 180, 120, 1.3, 2.0),
+                                             (60, 700, 5, 64, 300, 1.4, 0.0), (90, 330, 32, 100, 60, 3.0, 0.0),
+                                             (172, 260, 0, 180, 100, 1.3, 30.0), (40, 900, 3, 44, 300, 1.6, 0.0)])
+def test_forward_projector_wide_cones_match_gather_form(gpu, monkeypatch, n, nz, z0, W, H, k, h):
+    """Windows of slices with short runs (wide cones, tall volumes) go to the entry form, two
+    chunks or one at a time, beside others in row runs; windows off the detector are left
+    out; single chunks with short runs take the gather form.  The gather form's images (2e-6, as
+    above), also where the first windows are the ones left out, and added to other images."""
+    import torch
+    import ct_amd
+    P = 5
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(W, H, k * W, 1.25, n, n, z0 + nz))
+    ctx.set_projections(np.array([0.0, 44.0, 91.0, 137.0, 290.0]), np.linspace(-h, h, P))
+    x = torch.randn((n, n, nz), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+
+    def project(accumulate=False):
+        y = torch.full((P, H, W), 3.0 if accumulate else float("nan"), device="cuda")
+        ctx.forward_project(x, z0, nz, 0, P, y, accumulate=accumulate)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    got, added = project(), project(True)
+    np.testing.assert_array_equal(added, got + np.float32(3.0))
+    monkeypatch.setenv("CTG_FP_GATHER", "1")
+    want = project()
+    assert np.abs(want).max() > 0.0
+    assert rel_rmse(got, want) < 2e-6
+
+
+def test_forward_projector_of_a_slab_off_the_detector(gpu):
+    """A slab that no row of the detector sees projects to zeros, or adds nothing."""
+    import torch
+    import ct_amd
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(ct_amd.geometry_grid(40, 30, 160.0, 0.0, 36, 36, 900))
+    ctx.set_projections([0.0, 77.0], None)
+    x = torch.ones((36, 36, 100), device="cuda")
+    y = torch.full((2, 30, 40), float("nan"), device="cuda")
+    ctx.forward_project(x, 800, 100, 0, 2, y)
+    torch.cuda.synchronize()
+    assert (y == 0.0).all()
+    y.fill_(2.0)
+    ctx.forward_project(x, 800, 100, 0, 2, y, accumulate=True)
+    torch.cuda.synchronize()
+    assert (y == 2.0).all()
