@@ -79,7 +79,8 @@ struct BpArgs {
     // numbering of the tiles (tile_of)
     int strip_h, nstrips, blk;  // tile rows per strip, tile columns per block
     unsigned nwork, nidle;     // tiles of one layer inside / outside the strips' ranges
-    unsigned per, chunk, extra;  // 8 nzb chunks, the first `extra` of chunk + 1 tiles, the others of chunk; the largest
+    unsigned chunk, extra;     // rounds of 8 chunks, the first `extra` chunks of chunk + 1 tiles, the others of chunk
+    unsigned long_rounds, work_wgs;  // rounds of eight chunks with longer ones among them; working tiles' workgroups of an XCD
     unsigned before[kMaxStrips + 1];  // working tiles of the strips before each
     int first[kMaxStrips];            // first working tile column of each strip
 };
@@ -88,12 +89,15 @@ struct BpArgs {
 // slices) is cut into strips of strip_h tile rows, each with the range of tile columns inside
 // the reconstruction cylinder; a strip is numbered in blocks of blk columns, so that
 // consecutive numbers are neighbours along every ray direction.  The working tiles of all
-// layers, in that order, are cut into chunks of equal size (to one tile), eight per layer, that
-// go to the XCDs in turn (dispatch is round-robin over 8 XCDs).  So an XCD works on a
+// layers, in that order, are cut into chunks of equal size (to one tile), eight per layer
+// (number_chunks), that go to the XCDs in turn (dispatch is round-robin over 8 XCDs).  So an XCD works on a
 // contiguous region, whose footprints its own L2 holds, and yet has an equal share of every
 // layer and, since the turn shifts by three per layer, of every part of the layers: outer
 // layers and tiles leave the detector window and are cheaper.  The tiles outside the
-// cylinder only store; they come last.
+// cylinder only store; they come last.  No workgroup in between has nothing to do: an XCD deals
+// its workgroups to its shader engines in turn, and where most chunks held a tile less than the
+// longest, every chunk's last workgroup was such a one (198^2 x 81 from 289 projections, 661
+// columns: 698 us, 620 so).
 //
 // One contiguous range of all tiles per XCD (outer layers all on two of them) took 2.21 ms for
 // a 256^3 scan of 360 projections of 256 x 192 and 12.6 ms for 512^3 of 512 x 512, this
@@ -102,14 +106,16 @@ struct BpArgs {
 // take 171 and 140 ms there, and blocks numbered column by column 132 with FP16.
 __device__ inline bool tile_of(const BpArgs& a, int& zbi, int& tx, int& ty) {
     const unsigned xcd = blockIdx.x & 7u, k = blockIdx.x >> 3;
-    const bool work = k < (unsigned)a.nzb * a.per;
+    const bool work = k < a.work_wgs;
     unsigned n;
     if (work) {
-        const unsigned m = k / a.per, w = k - m * a.per, i = m * 8u + ((xcd + 3u * m) & 7u);
-        if (w >= a.chunk + (i < a.extra ? 1u : 0u)) return false;
+        const unsigned big = a.long_rounds * (a.chunk + 1u), size = k < big ? a.chunk + 1u : a.chunk;
+        const unsigned kr = k < big ? k : k - big, mr = kr / size, w = kr - mr * size;
+        const unsigned m = k < big ? mr : a.long_rounds + mr, i = m * 8u + ((xcd + 3u * m) & 7u);
+        if (w >= a.chunk + (i < a.extra ? 1u : 0u)) return false;  // (in the last long round only)
         n = i * a.chunk + min(i, a.extra) + w;
     } else {
-        n = (k - (unsigned)a.nzb * a.per) * 8u + xcd;
+        n = (k - a.work_wgs) * 8u + xcd;
         if (n >= a.nidle * (unsigned)a.nzb) return false;
     }
     const unsigned layer = work ? a.nwork : a.nidle;
@@ -825,12 +831,17 @@ void number_tiles(const ctg_geometry& g, BpArgs& a) {
     a.nidle = (unsigned)(a.ntx * a.nty) - a.nwork;
 }
 
-// Its chunks.
+// Its chunks: eight per layer, but of at least 16 tiles where a layer holds at most 20, so that
+// neighbours still share an L2 (FP32 and FP16, chunks of at least 1 and 16 tiles: 48^2 x 2000 from
+// 40 projections, 9 tiles per layer, 359 and 321, 301 and 278 us; 32^2 x 1000 from 100, 4 tiles,
+// 491 and 424, 420 and 362; 160^3 from 200, 100 tiles, no difference).
 void number_chunks(BpArgs& a) {
-    const unsigned total = a.nwork * (unsigned)a.nzb;
-    a.chunk = total / (8u * (unsigned)a.nzb);
-    a.extra = total - a.chunk * 8u * (unsigned)a.nzb;
-    a.per = a.chunk + (a.extra ? 1 : 0);
+    const unsigned total = a.nwork * (unsigned)a.nzb, least = a.nwork <= 20 ? 16 : 1;
+    const unsigned rounds = std::max(1u, std::min((unsigned)a.nzb, total / (8u * least)));
+    a.chunk = total / (8u * rounds);
+    a.extra = total - a.chunk * 8u * rounds;
+    a.long_rounds = (a.extra + 7u) / 8u;
+    a.work_wgs = rounds * a.chunk + a.long_rounds;
 }
 
 // Launches of `step` projections that go on from each other's sums.  One set of tiles and buffers
@@ -886,7 +897,7 @@ ctg_status launch_zpl(const BpLaunch& L, BpArgs a, int step, hipStream_t st) {
     const size_t lds = (size_t)2 * cap * ebytes;
     if ((long long)a.ntx * a.nty * a.nzb > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
     number_chunks(a);
-    const long long grid = 8ll * ((long long)a.nzb * a.per + ((long long)a.nidle * a.nzb + 7) / 8);
+    const long long grid = 8ll * ((long long)a.work_wgs + ((long long)a.nidle * a.nzb + 7) / 8);
     if (grid > 0x7fffffffll) return fail(CTG_ERROR_UNSUPPORTED, "backprojection grid too large");
     const size_t img_bytes = (size_t)g.det_width * g.det_height * ebytes;
     for (int p = 0; p < std::max(L.nproj, 1); p += step) {

@@ -1527,3 +1527,11 @@ def test_forward_projector_of_a_slab_off_the_detector(gpu):
     ctx.forward_project(x, 800, 100, 0, 2, y, accumulate=True)
     torch.cuda.synchronize()
     assert (y == 2.0).all()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(48, 48, 700), (20, 20, 90), (100, 100, 400), (16, 130, 33), (70, 70, 31)])
+def test_backprojection_numbering_covers_every_tile(gpu, nx, ny, nz):
+    """Chunks of tiles longer and shorter by one, several layers to a chunk, and one round for a
+    whole small volume: images of ones give every voxel of the cylinder that the detector sees
+    the sum of U^2 (1e-5, as in the other test of the tiles), from a volume of NaN."""
+    test_backprojection_covers_every_tile(gpu, nx, ny, nz, 2 * max(nx, ny))
