@@ -209,11 +209,13 @@ __device__ inline int cvt_flr(float x) {
 // box: x = first entry column, y = first row, w = rows, z = ncols | flags.
 // bits 28-29: 0 the block cannot hit the detector, 1 staged in LDS, 2 global reads;
 // bit 27: the unmasked path may be used; bit 26: it may be used without any test, because
-// the whole tile and run lie inside the detector window.
+// the whole tile and run lie inside the detector window; bit 25: the box covers the whole run
+// where the slab holds a part of it.
 __device__ inline int box_kind(int4 b) { return ((unsigned)b.z >> 28) & 3; }
 __device__ inline bool box_fast(int4 b) { return (b.z >> 27) & 1; }
 __device__ inline bool box_inside(int4 b) { return (b.z >> 26) & 1; }
-__device__ inline int box_nc(int4 b) { return b.z & 0x03ffffff; }
+__device__ inline bool box_full(int4 b) { return (b.z >> 25) & 1; }
+__device__ inline int box_nc(int4 b) { return b.z & 0x01ffffff; }
 __device__ inline int box_nr(int4 b) { return b.w & 0xffff; }
 __device__ inline int box_pitch(int4 b) { return (unsigned)b.w >> 16; }
 
@@ -260,10 +262,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
     static_assert(ZPL == kRowAnchor || ZPL == kRowAnchor / 2, "a run lies inside one row anchor block");
     const int zrun = a.z0 - a.zshift + zb;
     const float zw0 = (float)zrun - a.zpre;
-    // The slices a step has to cover: the whole run, unless the slab holds so few of it that the
-    // masked form (by groups of four, about 1.5 times the time per slice) is cheaper on those:
-    // 72 slices in runs of 32 at 96^2 x 48 projections took 99 us with a whole last run of 8
-    // slices, 88 so.
+    // The slices a step has to cover: the whole run, unless the slab holds at most two thirds of it
+    // and the run leaves the detector's rows: masked (by groups of four, 1.5 to 2.3 times the time
+    // per slice) those slices alone are then cheaper.  72 slices in runs of 32 at 96^2 x 48
+    // projections took 99 us with a whole last run of 8 slices, 88 so; 221^2 x 21 from 111
+    // projections, inside the rows, 155 us whole and 232 masked.
     const int valid = min(zlast, ZPL) - max(zfirst, 0);
     const bool whole = valid * 3 > ZPL * 2;
     const int kfirst = whole ? 0 : max(zfirst, 0), klast = whole ? ZPL - 1 : min(zlast, ZPL) - 1;
@@ -304,6 +307,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             // changes of uIdx and vIdx along x (the lanes of a 16-lane row), summed over
             // the tile's two y edges and the run's two z ends
             float du = 0.0f, dv = 0.0f;
+            float runlo = INFINITY, runhi = -INFINITY;  // rows of the whole run
             bool bad = false;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -320,6 +324,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
                 const float vb = fmaf(-(zwl + g.z), U, a.vpre);
                 umin = fminf(umin, ui); umax = fmaxf(umax, ui);
                 vmin = fminf(vmin, fminf(va, vb)); vmax = fmaxf(vmax, fmaxf(va, vb));
+                if (!whole) {
+                    const float fa = fmaf(-(zw0 + g.z), U, a.vpre), fb = fmaf(-(zw0 + (float)(ZPL - 1) + g.z), U, a.vpre);
+                    runlo = fminf(runlo, fminf(fa, fb)); runhi = fmaxf(runhi, fmaxf(fa, fb));
+                }
                 du += (c & 1) ? ui : -ui;
                 dv += (c & 1) ? va + vb : -(va + vb);
             }
@@ -332,12 +340,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             // A voxel reads the one entry at (floor(uIdx), floor(vIdx)).  uIdx and vIdx are
             // projective in the voxel's position, so over the tile and run they lie between
             // the corners' values; kBoxMargin covers the rounding of either expression.
-            const int us0 = (int)floorf(umin - kBoxMargin), vs0 = (int)floorf(vmin - kBoxMargin);
+            const int us0 = (int)floorf(umin - kBoxMargin);
             const int us = max(us0, 0);
             const int ue = min((int)floorf(umax + kBoxMargin), a.W - 1);
-            const int vs = max(vs0, 0) & (a.dma16 ? ~1 : ~0);
+            const int nc = ue - us + 1;
+            const int vmask = a.dma16 ? ~1 : ~0;
+            // every slice of the run on the detector's rows: the unmasked path for all of them,
+            // if their box fits the LDS
+            auto rows_in = [&](float lo, float hi) {
+                return lo - kBoxMargin >= fmaxf(a.vpre - a.vhi, 0.0f) && hi + kBoxMargin <= fminf(a.vpre - a.vlo, (float)(a.H - 1));
+            };
+            bool full = false;
+            if (!whole && rows_in(runlo, runhi)) {
+                const int n = (int)floorf(runhi + kBoxMargin) - ((int)floorf(runlo - kBoxMargin) & vmask) + 2;
+                full = nc * (n + ((a.pitch_alt - n) & (a.pitch_mod - 1))) <= a.cap;
+            }
+            if (full) {
+                vmin = runlo;
+                vmax = runhi;
+            }
+            const int vs0 = (int)floorf(vmin - kBoxMargin);
+            const int vs = max(vs0, 0) & vmask;
             const int ve = min((int)floorf(vmax + kBoxMargin), a.H - 1);
-            const int nc = ue - us + 1, nr = ve - vs + 1;
+            const int nr = ve - vs + 1;
             if (nc <= 0 || nr <= 0) { b.z = 0; return b; }
             // LDS column pitch: the rows the DMA writes (an even count when 16-byte lanes
             // carry two 8-byte entries) rounded up to pitch_rem mod pitch_mod (a power of
@@ -362,11 +387,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             const int fast = vs0 >= 0 ? 1 : 0;
             // no voxel of the tile and run can fail a window test (by more than either
             // expression's rounding), and no entry is clipped away
-            const bool in = whole && fast && us0 >= 0 && umin - kBoxMargin >= a.ulo + a.upre &&
-                            umax + kBoxMargin <= fminf(a.uhi + a.upre, (float)(a.W - 1)) &&
-                            vmin - kBoxMargin >= a.vpre - a.vhi &&
-                            vmax + kBoxMargin <= fminf(a.vpre - a.vlo, (float)(a.H - 1));
-            b.z = nc | ((in ? 1 : 0) << 26) | (fast << 27) | ((nc * pitch <= a.cap ? 1 : 2) << 28);
+            const bool in = (whole || full) && fast && us0 >= 0 && umin - kBoxMargin >= a.ulo + a.upre &&
+                            umax + kBoxMargin <= fminf(a.uhi + a.upre, (float)(a.W - 1)) && rows_in(vmin, vmax);
+            b.z = nc | ((full ? 1 : 0) << 25) | ((in ? 1 : 0) << 26) | (fast << 27) | ((nc * pitch <= a.cap ? 1 : 2) << 28);
             return b;
         };
 
@@ -433,7 +456,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(E::kMi
             int mode = kind == 1 ? 1 : 3;
             if (kind == 1 && !box_inside(bx)) {
                 const bool lane_full = !cv || ((zw0 + g.z) * U >= a.vlo && (zwl + g.z) * U <= a.vhi);
-                if (!(whole && box_fast(bx) && __all(lane_full))) mode = 2;
+                if (!((whole || box_full(bx)) && box_fast(bx) && __all(lane_full))) mode = 2;
                 else if (!cv) idle();
             }
             // The three forms follow one another, each under its own opaque condition: as

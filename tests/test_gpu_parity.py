@@ -1535,3 +1535,37 @@ def test_backprojection_numbering_covers_every_tile(gpu, nx, ny, nz):
     whole small volume: images of ones give every voxel of the cylinder that the detector sees
     the sum of U^2 (1e-5, as in the other test of the tiles), from a volume of NaN."""
     test_backprojection_covers_every_tile(gpu, nx, ny, nz, 2 * max(nx, ny))
+
+
+@pytest.mark.parametrize("store", ["f32", "f16"])
+@pytest.mark.parametrize("nz,z0,fcd", [(5, 0, 4.0), (21, 0, 4.0), (21, 3, 1.1), (40, 0, 1.1), (72, 0, 1.5), (9, 2, 6.0)])
+def test_partial_runs_inside_the_window_match_the_global_form(gpu, monkeypatch, store, nz, z0, fcd):
+    """A partly filled run steps over all its slices where they lie on the detector's rows, which
+    is tall here, and over the slab's alone where the longer box does not fit the LDS (wide
+    cones): bit for bit the form that reads global memory voxel by voxel."""
+    import torch
+    import ct_amd
+    W, H, P, n = 100, 300, 7, 100
+    g = ct_amd.geometry_grid(W, H, fcd * W, 2.0, n, n, z0 + nz)
+    ctx = ct_amd.Context(0)
+    ctx.set_geometry(g)
+    ctx.set_projections(np.linspace(0.0, 320.0, P), np.linspace(-120.0, 120.0, P))
+    img = torch.randn((P, H, W), generator=torch.Generator(device="cuda").manual_seed(nz), device="cuda")
+    entries = torch.empty(ctx.filtered_bytes(store, P), dtype=torch.uint8, device="cuda")
+    scales = torch.empty(P, dtype=torch.float32, device="cuda")
+    ctx.layout_projections(img, P, store, entries, scales)
+
+    def volume():
+        v = torch.full((n, n, nz), float("nan"), device="cuda")
+        ctx.backproject(entries, store, scales, 0, P, v, z0, nz, False)
+        torch.cuda.synchronize()
+        return v.cpu().numpy()
+
+    for zpl in ("16", "32"):
+        monkeypatch.setenv("CTG_BP_ZPL", zpl)
+        got = volume()
+        monkeypatch.setenv("CTG_BP_PITCH", "65536,0")
+        ref = volume()
+        monkeypatch.delenv("CTG_BP_PITCH")
+        assert np.isfinite(ref).all() and np.any(ref != 0.0)
+        np.testing.assert_array_equal(got, ref)
