@@ -32,18 +32,17 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E, 8 TB/s
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "backproject_traffic_1024cubed_720proj.json")
 BYTES_PER_UPDATE = 8.0     # one FP32 voxel load + one store per (voxel, projection)
-# VALU issue peak at 4 cycles per wave64 instruction per SIMD: 256 CUs x 64 lanes x
-# 2.4 GHz, in 1e12 lane-instructions/s.  ct_amd/isa_rates measures 4.2-4.4 cycles for
-# v_fract_f32, v_cvt_flr_i32_f32, v_lshl_add_u32 and v_fma_mix_f32 but 2.8 for v_fma_f32,
-# so for an FMA-heavy mix this is a lower bound of the issue rate.
-VALU_PEAK_T = 256 * 64 * 2.4e9 / 1e12
+# VALU issue of one voxel-update, in wave64 instructions and in cycles of a SIMD at the rates
+# that ct_amd/isa_rates measures: the FMA of the detector row, its floor and fraction, the LDS
+# address, three FMAs of the bilinear form and one into the accumulator.  v_fma_f32 takes 2.8
+# cycles, v_cvt_flr_i32_f32, v_fract_f32, v_lshl_add_u32 and v_fma_mix_f32 (two of the FMAs of
+# 8-byte entries) 4.2 to 4.4.  256 CUs x 4 SIMDs x 64 lanes at 2.4 GHz.
+VALU_PER_UPDATE = 8.0
+VALU_CYCLES = {"f32": 26.6, "f16": 29.9}
+VALU_PEAK_T = {k: VALU_PER_UPDATE * 256 * 4 * 64 * 2.4e9 / c / 1e12 for k, c in VALU_CYCLES.items()}
 # MI355X's published FP32 vector peak (TFLOP/s) and the flops of one voxel-update
 FP32_PEAK_TFLOPS = 157.3
 FLOPS_PER_UPDATE = 8.0
-# lane-instructions per voxel-update of the register-accumulating formulation: one FMA
-# for the detector row, floor and fraction of it, three FMAs for the bilinear form and
-# one FMA into the accumulator (the LDS address is not counted)
-VALU_PER_UPDATE = 7.0
 # LDS read bandwidth: 256 bytes per clock per CU (a ds_read_b128 serves 16 lanes per
 # 4-cycle pass: ct_amd/isa_rates measures at most 6.6 cycles per conflict-free wave
 # read and 16.9 for a 4-way conflict), 256 CUs at 2.4 GHz, in TB/s
@@ -478,11 +477,14 @@ def main():
             f"360x192x256 in {cpu['scan256_seconds']:.2f} s")
 
     t32, bp32 = res["f32"]
-    # The FP32 backprojection keeps its voxels in registers, so its binder is the VALU
-    # issue rate, not HBM: achieved = VALU_PER_UPDATE lane-instructions per voxel-update
-    # (the formulation's count, see the constant) / kernel time, against the non-packed
-    # FP32 issue peak of 256 CUs x 64 lanes x 2.4 GHz.
-    achieved = VALU_PER_UPDATE * updates / bp32 / 1e12
+    # The backprojection keeps its voxels in registers, so its binders are on chip: VALU issue and
+    # the LDS reads.  They count the updates of voxels inside the reconstruction cylinder, which
+    # are the ones that run; value counts the grid's, as the metric is defined.
+    import numpy as np
+    x2 = (np.arange(g.nx) - g.x_pre) ** 2
+    y2 = (np.arange(g.ny) - g.y_pre) ** 2
+    inside = updates * float(np.mean(x2[:, None] + y2[None, :] < g.radius ** 2))
+    achieved = VALU_PER_UPDATE * inside / bp32 / 1e12
     traffic = None
     if os.path.exists(TRAFFIC_FILE) and (args.det, args.nproj, args.grid) == (1024, 720, 1024):
         # HBM bytes per launch measured with rocprofv3 FETCH_SIZE/WRITE_SIZE, calibrated
@@ -510,23 +512,23 @@ def main():
         "ms_per_recon_f32": t32 * 1e3,
         "bp_ms_f32": bp32 * 1e3,
         "bp_gups_f32": updates / bp32 / 1e9,
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": VALU_PEAK_T, "unit": "T lane-instr/s",
-                     "frac": achieved / VALU_PEAK_T, "traffic": traffic, "compulsory_bytes": compulsory,
+        "roofline": {"bound": "valu", "achieved": achieved, "peak": VALU_PEAK_T["f32"], "unit": "T lane-instr/s",
+                     "frac": achieved / VALU_PEAK_T["f32"], "traffic": traffic, "compulsory_bytes": compulsory,
                      "traffic_over_compulsory": traffic / compulsory if traffic else None,
-                     "valu_per_update": VALU_PER_UPDATE},
+                     "valu_per_update": VALU_PER_UPDATE, "updates_in_cylinder": inside},
         # against the published FP32 vector peak: the update's arithmetic is the three
         # FMAs of the bilinear form and the accumulating FMA, 8 flops
-        "roofline_fp32_peak": {"bound": "fp32", "achieved": FLOPS_PER_UPDATE * updates / bp32 / 1e12,
+        "roofline_fp32_peak": {"bound": "fp32", "achieved": FLOPS_PER_UPDATE * inside / bp32 / 1e12,
                                "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                               "frac": FLOPS_PER_UPDATE * updates / bp32 / 1e12 / FP32_PEAK_TFLOPS,
+                               "frac": FLOPS_PER_UPDATE * inside / bp32 / 1e12 / FP32_PEAK_TFLOPS,
                                "flops_per_update": FLOPS_PER_UPDATE},
         # the other on-chip ceiling: one 16-byte FP32 entry read from LDS per update,
         # against 256 B per clock per CU (256 CUs at 2.4 GHz), and against the measured
         # rate of conflict-free 16-byte LDS reads
-        "roofline_lds": {"bound": "lds", "achieved": 16.0 * updates / bp32 / 1e12, "peak": LDS_PEAK_TBS,
-                         "unit": "TB/s", "frac": 16.0 * updates / bp32 / 1e12 / LDS_PEAK_TBS, "bytes_per_update": 16,
+        "roofline_lds": {"bound": "lds", "achieved": 16.0 * inside / bp32 / 1e12, "peak": LDS_PEAK_TBS,
+                         "unit": "TB/s", "frac": 16.0 * inside / bp32 / 1e12 / LDS_PEAK_TBS, "bytes_per_update": 16,
                          "peak_measured_ds_read_b128": LDS_READ_MEASURED_TBS,
-                         "frac_of_measured": 16.0 * updates / bp32 / 1e12 / LDS_READ_MEASURED_TBS},
+                         "frac_of_measured": 16.0 * inside / bp32 / 1e12 / LDS_READ_MEASURED_TBS},
         # the 8-byte read-modify-write model of the metric's definition (the reference
         # kernel's per-update voxel load and store, Ct/cuda_ct.cu:193-199): 1000 GUPS
         # at 8 TB/s, against which a 60 % HBM-roofline target reads 600 GUPS
@@ -538,14 +540,13 @@ def main():
         t16, bp16 = res["f16"]
         out.update({"ms_per_recon_f16": t16 * 1e3, "bp_ms_f16": bp16 * 1e3, "bp_gups_f16": updates / bp16 / 1e9,
                     "f16_over_f32_bp": bp32 / bp16, "f16_over_f32_step": t32 / t16,
-                    # the FP16-entry kernel is VALU-bound with the same 7 lane-instructions per
-                    # update (interpolation in FP32): at 100 % of the issue rate it would run at
-                    # VALU_PEAK_T / 7 updates/s, which caps its ratio to this FP32 run
-                    "roofline_f16": {"bound": "valu", "achieved": VALU_PER_UPDATE * updates / bp16 / 1e12,
-                                     "peak": VALU_PEAK_T, "unit": "T lane-instr/s",
-                                     "frac": VALU_PER_UPDATE * updates / bp16 / 1e12 / VALU_PEAK_T,
+                    # the FP16-entry kernel is VALU-bound: at its issue rate it would make
+                    # 1 / 29.9 updates per cycle, which caps its ratio to this FP32 run
+                    "roofline_f16": {"bound": "valu", "achieved": VALU_PER_UPDATE * inside / bp16 / 1e12,
+                                     "peak": VALU_PEAK_T["f16"], "unit": "T lane-instr/s",
+                                     "frac": VALU_PER_UPDATE * inside / bp16 / 1e12 / VALU_PEAK_T["f16"],
                                      "valu_per_update": VALU_PER_UPDATE,
-                                     "f16_over_f32_bp_ceiling": VALU_PEAK_T * 1e12 / VALU_PER_UPDATE / (updates / bp32)}})
+                                     "f16_over_f32_bp_ceiling": VALU_PEAK_T["f16"] * 1e12 / VALU_PER_UPDATE / (inside / bp32)}})
     if e2e is not None:
         out["ms_e2e_from_pinned_host_f32"] = e2e[0] * 1e3
         out["ms_reconstruct_host_to_host_f32"] = h2h * 1e3
