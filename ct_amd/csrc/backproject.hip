@@ -34,13 +34,14 @@
 //    receives contiguous ranges of tiles, in 4x4 blocks of tiles, and shares detector
 //    footprints in its own L2, with an equal part of every layer (tile_of).
 //
-// What bounds it (1024^3 x 720 x 1024^2, MI355X): with FP32 entries the traffic of boxes that
-// miss L2 (658 GB per backprojection, 4.1 TB/s; 137 ms instead of 162 when every line hits),
-// then the LDS (a ds_read_b128 takes 4.8 cycles per wave and CU, a staging DMA instruction
-// 17 whatever its lane mask); with 8-byte entries VALU issue (116 of 133 ms remain without
-// any staging).  Accumulators updated in place, three forms per step and tests left out where
-// a box lies inside the window took FP32 from 177 to 163 ms, FP16 from 147 to 133 ms, and a
-// 256^3 x 360 scan from 2.67 to 2.2 ms.
+// What bounds it (1024^3 x 720 x 1024^2, MI355X, 160 ms FP32 and 130 ms FP16): with FP32 entries
+// the traffic of boxes that miss L2 (658 GB per backprojection, 4.1 TB/s, 39 % L2 hits; an earlier
+// form of 162 ms took 137 with every line a hit), then the LDS (a ds_read_b128 takes 4.8 cycles
+// per wave and CU, a staging DMA instruction 17 whatever its lane mask); with 8-byte entries VALU
+// issue (116 of 133 ms remained without any staging).  Accumulators updated in place, three forms
+// per step and tests left out where a box lies inside the window took FP32 from 177 to 163 ms and
+// FP16 from 147 to 133, launches of about 240 projections the rest; with the numbering of the tiles
+// a 256^3 x 360 scan went from 2.67 to 1.55 ms.
 #include "ctg_internal.h"
 
 #include <hip/hip_fp16.h>
